@@ -166,7 +166,12 @@ int droplet_tile_side(int n);
 int droplet_tile_count(int n);
 hipError_t launch_droplet_order(int n, const DropletParams& p, uint32_t iteration, uint32_t* tiles,
                                 uint32_t* order, hipStream_t s);
-// Per-workgroup sums of one droplet launch (256 droplets per workgroup).
+// Per-workgroup sums of one droplet launch; a partials launch of `count`
+// droplets (at most 256 times HG_DROPLET_PARTIALS_MAX) has
+// droplet_partial_blocks(count) workgroups, never more than
+// HG_DROPLET_PARTIALS_MAX.
+#define HG_DROPLET_PARTIALS_MAX (1u << 14)
+uint32_t droplet_partial_blocks(uint32_t count);
 struct DropletPartial {
     double exported;
     unsigned long long steps;

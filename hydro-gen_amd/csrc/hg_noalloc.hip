@@ -21,8 +21,8 @@
 
 namespace {
 
-constexpr uint32_t kScratchBlocks = 1u << 14;   // droplets per iteration <= 256 * 2^14 = 2^22
-static_assert(256ull * kScratchBlocks == HG_DROPLETS_NOALLOC_MAX, "scratch holds one partial per workgroup");
+constexpr uint32_t kScratchBlocks = HG_DROPLET_PARTIALS_MAX;   // droplets per iteration <= 256 * 2^14 = 2^22
+static_assert(256ull * kScratchBlocks == HG_DROPLETS_NOALLOC_MAX, "scratch holds one partial per workgroup (droplet_partial_blocks)");
 
 __device__ __align__(256) hgk::DropletPartial scratch[kScratchBlocks];
 
@@ -83,7 +83,7 @@ extern "C" int hg_droplets_noalloc(float* rock, float* dirt, uint32_t n, const h
     p.min_slope = s->min_slope; p.init_water = s->init_water; p.init_speed = s->init_speed;
     p.seed_lo = uint32_t(s->seed); p.seed_hi = uint32_t(s->seed >> 32);
     const hgk::Brush brush = hgk::make_brush(s->brush_radius);
-    const uint32_t nblocks = (s->count + 255) / 256;
+    const uint32_t nblocks = hgk::droplet_partial_blocks(s->count);
     const bool totals = exported_mass || droplet_steps;
     if (iterations == 0 && totals) {
         const hipError_t e = hgk::launch_droplet_totals(partials, 0, exported_mass, droplet_steps, false, st);
