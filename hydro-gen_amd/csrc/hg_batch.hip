@@ -41,7 +41,7 @@ struct hg_batch {
     hg_rain_settings rs{};
     int rain_mode = HG_RAIN_OFF;
     uint64_t seed = 0;
-    int hydro_variant = 0, thermal_variant = 1;
+    int hydro_variant = 0, thermal_variant = 0;   // by size until tuned or set
     size_t total_floats = 0;            // size of `block`
     bool persistent = false;            // false: one workgroup per work-list entry
     bool xcd_order = true;              // interleave the work-list for the 8 XCDs
@@ -382,6 +382,8 @@ int hg_batch_create(int device, int count, const uint32_t* sizes, hg_batch** out
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
         return cleanup("hipStreamCreate failed", HG_ERR_HIP);
     b->total_floats = total;
+    b->hydro_variant = hgk::default_hydro_variant(total / (2 * HG_NUM_STATE_PLANES));
+    b->thermal_variant = hgk::default_thermal_variant(total / (2 * HG_NUM_STATE_PLANES));
     if (hipMalloc(&b->block, total * sizeof(float)) != hipSuccess)
         return cleanup("hipMalloc of the batch state failed", HG_ERR_OOM);
     if (hipMalloc(&b->dev_terr, sizeof(BatchTerrain) * count) != hipSuccess ||

@@ -356,6 +356,18 @@ __device__ __forceinline__ void tile_of(int b, int nb, int gx, int xcd, int& bx,
     bx = t - by * gx;
 }
 
+// The order a launch's tiles are walked in for the caller's mode.  Column
+// strips (2) need tile columns in multiples of 8.  Other shapes get
+// contiguous runs (1) as long as two rows of tiles, at `bytes` read per cell,
+// stay in 3 MB of an XCD's 4 MB L2, and row-major order beyond that.  Hydro, us
+// per launch, runs against row-major: 640^2 9.7 / 12.7, 1088^2 20.2 / 29.5,
+// 1408^2 28.7 / 45.5, 2240^2 86.9 / 99.4; 3000^2 173.3 / 170.6.
+int tile_order(int mode, int nx, int tx, int ty, int bytes) {
+    if (mode != 2) return mode;
+    if (((nx + tx - 1) / tx) % 8 == 0) return 2;
+    return size_t(2) * size_t(nx) * size_t(ty) * size_t(bytes) <= (size_t(3) << 20) ? 1 : 0;
+}
+
 template <int TX, int TY, int HA, int NT, bool EXTRA, bool NTS>
 __global__ __launch_bounds__(NT) void k_fused_hydro(HydroIO io, int nx, int ny, uint32_t step,
                                                     uint32_t terrain, int rain, int xcd, KParams k) {
@@ -606,7 +618,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     X(4,  64, 16, 3, 256)    \
     X(5, 128,  8, 2, 256)    \
     X(6,  64, 16, 2, 512)    \
-    X(7, 128, 16, 2, 1024)
+    X(7, 128, 16, 2, 1024)   \
+    X(8,  64,  8, 2, 512)
 //                        TX   TY   NT
 #define HG_THERMAL_VARIANTS(X) \
     X(0,  64, 16, 256)         \
@@ -617,9 +630,37 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     X(5,  32, 32, 256)         \
     X(6, 128, 16, 512)         \
     X(7,  64, 64, 1024)        \
-    X(8, 128, 32, 1024)
+    X(8, 128, 32, 1024)        \
+    X(9,  64, 16, 512)         \
+    X(10, 64,  8, 1024)
 
 }  // namespace
+
+// The variants a map gets that was not tuned, by its number of 64 x 16 tiles
+// (cells / 1024).  Few tiles leave CUs idle and each cell of a tile is on the
+// critical path, so small maps get small tiles with more threads per cell;
+// large ones get the tiles with less halo.  us per launch, alone / with three
+// maps at once (hydro; thermal figures are of the whole step):
+//          hydro 64x8/512  64x16/256  64x16/512  128x16/512
+//   256^2     6.8/ 3.1     10.8/ 4.8
+//   512^2     9.5/ 4.7     14.9/ 6.8      - / 4.8
+//  1024^2                  22.4/15.5   18.3/13.7    - /14.6
+//  2048^2                  72.6/61.8   69.7/62.9  70.4/62.7
+//  4096^2                 265.7/253.0 265.2/258.1 261.8/249.6
+//        thermal 64x8/1024 64x16/512  64x32/256  64x32/512
+//   256^2    15.5/ 6.3       - / 6.6  28.7/10.1
+//   512^2    20.2/ -         - / 8.8  31.8/11.3
+//   768^2                  33.8/16.3  41.2/17.8    - /17.0
+//  1024^2                  36.3/ -    41.4/23.4  36.7/22.0
+//  2048^2                            126.3/99.9 118.0/97.8
+int default_hydro_variant(size_t cells) {
+    const size_t tiles = cells / 1024;
+    return tiles < 512 ? 8 : tiles < 4096 ? 6 : 2;
+}
+int default_thermal_variant(size_t cells) {
+    const size_t tiles = cells / 1024;
+    return tiles < 128 ? 10 : tiles < 1024 ? 9 : 2;
+}
 
 int hydro_variant_count() {
 #define X(i, tx, ty, ha, nt) +1
@@ -654,10 +695,11 @@ bool thermal_variant_info(int v, int* tx, int* ty, int* halo, int* nt) {
 }
 
 hipError_t launch_fused_hydro(int variant, const HydroIO& io, int nx, int ny, uint32_t step,
-                              uint32_t terrain, bool rain, int xcd, const KParams& k, hipStream_t s) {
+                              uint32_t terrain, bool rain, int xcd_mode, const KParams& k, hipStream_t s) {
     switch (variant) {
 #define X(i, TX_, TY_, HA_, NT_)                                                              \
     case i: {                                                                                 \
+        const int xcd = tile_order(xcd_mode, nx, TX_, TY_, 36);                               \
         const unsigned grid = unsigned((nx + TX_ - 1) / TX_) * unsigned((ny + TY_ - 1) / TY_); \
         const bool ex = io.vx || io.tb1;                                                      \
         const int r = rain ? 1 : 0;                                                           \
@@ -759,10 +801,11 @@ int batch_thermal_blocks_per_cu(int variant) {
 }
 
 hipError_t launch_fused_thermal(int variant, const ThermIO& io, int nx, int ny, bool thermal,
-                                bool smooth, int xcd, const KParams& k, hipStream_t s) {
+                                bool smooth, int xcd_mode, const KParams& k, hipStream_t s) {
     switch (variant) {
 #define X(i, TX_, TY_, NT_)                                                                  \
     case i: {                                                                                \
+        const int xcd = tile_order(xcd_mode, nx, TX_, TY_, 8);                               \
         const unsigned grid = unsigned((nx + TX_ - 1) / TX_) * unsigned((ny + TY_ - 1) / TY_); \
         const int th = thermal ? 1 : 0, sm = smooth ? 1 : 0;                                 \
         if (io.tr5 && k.store_nt)                                                            \

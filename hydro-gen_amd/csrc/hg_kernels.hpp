@@ -107,6 +107,9 @@ __device__ inline void eroded_sediment_global(const HydroIO& io, int qx, int qy,
                  rd(qx, qy - 1), k);
 }
 
+// variants of a map (or batch) of `cells` cells that was not tuned
+int default_hydro_variant(size_t cells);
+int default_thermal_variant(size_t cells);
 int hydro_variant_count();
 int thermal_variant_count();
 bool hydro_variant_info(int v, int* tx, int* ty, int* halo, int* nt);

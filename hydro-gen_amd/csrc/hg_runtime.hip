@@ -33,8 +33,6 @@ struct TunedTiles {
     int hydro, thermal, sweep;
 };
 std::map<std::pair<int, std::string>, TunedTiles> g_tune_cache;
-constexpr int DEFAULT_HYDRO_VARIANT = 0;
-constexpr int DEFAULT_THERMAL_VARIANT = 1;
 constexpr int DEFAULT_SWEEP_VARIANT = -1;
 
 }  // namespace
@@ -342,8 +340,8 @@ int hg_create(int device, uint32_t n, uint32_t particle_count, hg_ctx** out) {
     c->ds.init_water = 1.0f; c->ds.init_speed = 1.0f; c->ds.seed = 0;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->arch = prop.gcnArchName;
-    c->hydro_variant = DEFAULT_HYDRO_VARIANT;
-    c->thermal_variant = DEFAULT_THERMAL_VARIANT;
+    c->hydro_variant = hgk::default_hydro_variant(pn);
+    c->thermal_variant = hgk::default_thermal_variant(pn);
     c->sweep_variant = DEFAULT_SWEEP_VARIANT;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
