@@ -20,6 +20,8 @@
 // tile plus an HA-cell halo; a back-trace whose bilinear taps fall outside it
 // recomputes the eroded sediment of those taps from the step's input planes
 // (still intact: every pass is ping-pong), which is exact.
+#include <algorithm>
+
 #include "hg_kernels.hpp"
 
 namespace hgk {
@@ -41,6 +43,16 @@ __device__ __forceinline__ void st_out(float* p, float v) {
         __builtin_nontemporal_store(v, p);
     else
         *p = v;
+}
+
+template <bool NTS>
+__device__ __forceinline__ void st_out2(float* p, float a, float b) {
+    typedef float v2 __attribute__((ext_vector_type(2)));
+    const v2 v = {a, b};
+    if constexpr (NTS)
+        __builtin_nontemporal_store(v, reinterpret_cast<v2*>(p));
+    else
+        *reinterpret_cast<v2*>(p) = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -542,6 +554,305 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 }
 
 // ---------------------------------------------------------------------------
+// thermal kernel, marching form
+//
+// A wave owns a strip of 128 columns, two per lane, of which it writes the
+// inner 116, and marches down its rows: each new row advances layer 0, layer 1
+// and smoothing, each two to three rows behind the one before it.
+// Vertical neighbours stay in registers and horizontal ones come from the
+// adjacent lane (DPP wave shifts): no LDS, no barriers.
+//
+// Why: the tile form is bound by VALU issue (485 instructions per cell), and
+// there every pair of neighbours is looked at four times, by both cells, once
+// for the outflow scale and once for the transport.  Here a pair (an edge from
+// cell p to cell q) is looked at once: its difference D = p - q gives
+//   P = D > thr ? D : 0     what p sends towards q, over g_p
+//   N = D < -thr ? D : 0    (-) what q sends towards p, over g_q
+// both cells' sums over marked directions take P or -N, and when both g are
+// known the transfer is T = P g_p + N g_q: one of the products is the tile
+// form's G * D, the other is a zero.  p adds -T, q adds T, in the same
+// order of directions as thermal_g and thermal_term, so the results are the
+// same bit for bit (for finite heights: beside a cell whose g is not a number,
+// the tile form's unmarked transfer is 0 and this one is not).
+//
+// About 260 VALU instructions per cell, times 1.10 for the columns and 1.12
+// (at 49 rows) for the rows that are not its own, issued at one per 3.5 cycles
+// per SIMD, near the rate of their mix (2.7 with two operands, 4.2 with three
+// or a lane shift).  137 registers: three waves per SIMD; held to 128 for four
+// it spills and slows down (150).  4096^2: 165 -> 126 us per launch, a step
+// 430 -> 389 us, with three maps at once 402 -> 354; 2048^2 with three maps at
+// once 104 -> 91 us per step.
+// ---------------------------------------------------------------------------
+constexpr int MARCH_TX = 116;          // columns a wave writes
+constexpr int MARCH_BATCH_TY = 192;    // rows of a batch's work-list entry, 48 per wave
+constexpr int MARCH_HX = 6;            // halo columns on each side (5 needed, even for the pairs)
+
+// Value of the next (right) and the previous (left) lane.
+__device__ __forceinline__ float lane_right(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xf, 0xf, true));   // wave_shl:1
+}
+__device__ __forceinline__ float lane_left(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xf, 0xf, true));   // wave_shr:1
+}
+
+// A row of the strip: the lane's two cells and the right lane's first cell.
+// Layer 0 looks at rock alone, layer 1 at rock + dirt.
+template <int LAYER>
+struct MarchRow {
+    float r[2], d[2], r_right, d_right;
+};
+template <int LAYER>
+__device__ __forceinline__ float march_diff(float ra, float da, float rb, float db) {
+    return LAYER == 0 ? ra - rb : (ra - rb) + (da - db);
+}
+struct MarchEdge {
+    float D[2], P[2], N[2];
+    __device__ __forceinline__ void mark(float thr) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            P[c] = D[c] > thr ? D[c] : 0.0f;
+            N[c] = D[c] < -thr ? D[c] : 0.0f;
+        }
+    }
+};
+// What a layer carries from row to row.  a: the newest row; z: the row below it.
+template <int LAYER>
+struct MarchLayer {
+    MarchRow<LAYER> a, z;
+    MarchEdge h;                        // edges along row a: (x, x+1)
+    float h_D_left, h_N_left;           // the left lane's second edge
+    MarchEdge v, e, f;                  // edges z-a: (x,z)-(x,a), (x,z)-(x+1,a), (x+1,z)-(x,a); D unused
+    float e_N_left;
+    float mc[2], md[2];                 // largest difference of row a's cells towards row z
+    float gz[2], gz_right;              // outflow scale of row z
+    float th[2], th_left;               // transfers along row z
+    float tv[2], te[2], te_left, tf[2]; // transfers between row z and the row below it
+};
+
+// Takes the next row b; returns in out[] the layer's new heights of row z
+// (a.* are then b, z.* a).  in_a, in_z: whether this lane's cells of those rows
+// are on the grid.
+template <int LAYER>
+__device__ __forceinline__ void march_advance(MarchLayer<LAYER>& s, const MarchRow<LAYER>& b, bool in_a, bool in_z,
+                                              const KParams& k, float (&out)[2]) {
+    const float ta = k.tan_alpha[LAYER], td = k.thr_diag[LAYER];
+    const MarchRow<LAYER>& a = s.a;
+    auto diff = [](float ra, float da, float rb, float db) { return march_diff<LAYER>(ra, da, rb, db); };
+    MarchEdge v, e, f;
+    v.D[0] = diff(a.r[0], a.d[0], b.r[0], b.d[0]);
+    v.D[1] = diff(a.r[1], a.d[1], b.r[1], b.d[1]);
+    e.D[0] = diff(a.r[0], a.d[0], b.r[1], b.d[1]);
+    e.D[1] = diff(a.r[1], a.d[1], b.r_right, b.d_right);
+    f.D[0] = diff(a.r[1], a.d[1], b.r[0], b.d[0]);
+    f.D[1] = diff(a.r_right, a.d_right, b.r[1], b.d[1]);
+    v.mark(ta);
+    e.mark(td);
+    f.mark(td);
+    const float e_D_left = lane_left(e.D[1]), e_N_left = lane_left(e.N[1]);
+    const float f_D_left = lane_left(f.D[1]), f_P_left = lane_left(f.P[1]);
+    // outflow scale of row a (thermal_g)
+    float g[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const float DL = c ? s.h.D[0] : s.h_D_left, NL = c ? s.h.N[0] : s.h_N_left;
+        const float DLT = c ? f.D[0] : f_D_left, PLT = c ? f.P[0] : f_P_left;
+        const float NLB = c ? s.e.N[0] : s.e_N_left;
+        float bk = s.h.P[c] - NL;
+        bk = bk + v.P[c];
+        bk = bk - s.v.N[c];
+        bk = bk + PLT;
+        bk = bk + e.P[c];
+        bk = bk - NLB;
+        bk = bk - s.f.N[c];
+        const float mc = fmaxf(fmaxf(-DL, s.h.D[c]), fmaxf(v.D[c], s.mc[c]));
+        const float md = fmaxf(fmaxf(DLT, e.D[c]), s.md[c]);
+        const float H = fminf(LAYER == 0 ? a.r[c] : a.d[c], fmaxf(fmaxf(mc, md), 0.0f));
+        const float rmax = fmaxf(mc, md * 0.70710678118654752f);
+        float sharp = fmaxf(1.0f + atanf(rmax) - k.Kalpha[LAYER], 1.0f);
+        sharp = sharp * (sharp * sharp);
+        const float S = (k.dt * k.Kspeed[LAYER] * 0.5f) * sharp * H;
+        g[c] = (bk > 0.0f && in_a) ? S * rcp(bk) : 0.0f;
+    }
+    const float g_right = lane_right(g[0]);
+    // transfers along row a and between rows z and a
+    auto send = [](float P, float gp, float N, float gq) { return fmaf(N, gq, P * gp); };
+    float th[2], tv[2], te[2], tf[2];
+    th[0] = send(s.h.P[0], g[0], s.h.N[0], g[1]);
+    th[1] = send(s.h.P[1], g[1], s.h.N[1], g_right);
+    tv[0] = send(s.v.P[0], s.gz[0], s.v.N[0], g[0]);
+    tv[1] = send(s.v.P[1], s.gz[1], s.v.N[1], g[1]);
+    te[0] = send(s.e.P[0], s.gz[0], s.e.N[0], g[1]);
+    te[1] = send(s.e.P[1], s.gz[1], s.e.N[1], g_right);
+    tf[0] = send(s.f.P[0], s.gz[1], s.f.N[0], g[0]);
+    tf[1] = send(s.f.P[1], s.gz_right, s.f.N[1], g[1]);
+    const float th_left = lane_left(th[1]), te_left = lane_left(te[1]), tf_left = lane_left(tf[1]);
+    // new heights of row z: L, R, T, B, LT, RT, LB, RB
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        float acc = (c ? s.th[0] : s.th_left) - s.th[c];
+        acc = acc - tv[c];
+        acc = acc + s.tv[c];
+        acc = acc - (c ? tf[0] : tf_left);
+        acc = acc - te[c];
+        acc = acc + (c ? s.te[0] : s.te_left);
+        acc = acc + s.tf[c];
+        const float h = LAYER == 0 ? s.z.r[c] : s.z.d[c];
+        out[c] = in_z ? h + acc : h;
+    }
+    // the next row
+    s.h.D[0] = diff(b.r[0], b.d[0], b.r[1], b.d[1]);
+    s.h.D[1] = diff(b.r[1], b.d[1], b.r_right, b.d_right);
+    s.h.mark(ta);
+    s.h_D_left = lane_left(s.h.D[1]);
+    s.h_N_left = lane_left(s.h.N[1]);
+    s.mc[0] = -v.D[0];
+    s.mc[1] = -v.D[1];
+    s.md[0] = fmaxf(-e_D_left, -f.D[0]);
+    s.md[1] = fmaxf(-e.D[0], -f.D[1]);
+    s.v = v;
+    s.e = e;
+    s.f = f;
+    s.e_N_left = e_N_left;
+    s.z = a;
+    s.a = b;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        s.gz[c] = g[c];
+        s.th[c] = th[c];
+        s.tv[c] = tv[c];
+        s.te[c] = te[c];
+        s.tf[c] = tf[c];
+    }
+    s.gz_right = g_right;
+    s.th_left = th_left;
+    s.te_left = te_left;
+}
+
+// Rows per wave.  A wave also runs 4 to 10 rows of every stage above and below
+// its own, and a workgroup (4 waves, one below the other) occupies a third of
+// a CU: the most rows that still fill the 256 CUs three times over are the
+// fastest, 49 at 4096^2 (us per launch: 16 rows 139, 37 rows 133, 49 rows 126,
+// 56 rows 139, 64 rows 156).  Above 96 rows a second round costs less than the
+// last one's idle CUs.
+inline int march_rows(int nx, int ny) {
+    const int strips = (nx + MARCH_TX - 1) / MARCH_TX;
+    for (int rounds = 1;; ++rounds) {
+        const int segs = std::max(1, rounds * 3 * 256 / strips);
+        const int rows = (ny + 4 * segs - 1) / (4 * segs);
+        if (rows <= 96) return std::max(rows, 8);
+    }
+}
+
+// Rows [ys, ye) of the strip whose first written column is xs.
+template <bool EXTRA, bool NTS>
+__device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny, int xs, int ys, int ye, int do_thermal,
+                                              int do_smooth, const KParams& k) {
+    const int lane = int(threadIdx.x) & 63;
+    const int x = xs - MARCH_HX + 2 * lane;                  // the lane's first column; even, like nx
+    const bool inx = x >= 0 && x < nx;
+    const bool mine = inx && lane >= MARCH_HX / 2 && lane < 64 - MARCH_HX / 2;
+    const int xc = min(max(x, 0), nx - 2);
+    auto iny = [&](int y) { return y >= 0 && y < ny; };
+    auto load = [&](const float* p, int y) {
+        return *reinterpret_cast<const float2*>(p + at(xc, min(max(y, 0), ny - 1), nx));
+    };
+    float r1[3][2], d1[3][2];                                // rows yo-1, yo, yo+1 after both layers
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) r1[j][c] = d1[j][c] = 0.0f;
+    auto push = [&](float ra, float rb, float da, float db) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            r1[0][c] = r1[1][c];
+            r1[1][c] = r1[2][c];
+            d1[0][c] = d1[1][c];
+            d1[1][c] = d1[2][c];
+        }
+        r1[2][0] = ra;
+        r1[2][1] = rb;
+        d1[2][0] = da;
+        d1[2][1] = db;
+    };
+    // smoothing of row yo, write it
+    auto emit = [&](int yo) {
+        const float r0 = r1[1][0], rr1 = r1[1][1], d0 = d1[1][0], dd1 = d1[1][1];
+        float r[2] = {r0, rr1}, d[2] = {d0, dd1};
+        const float rl = lane_left(rr1), rr = lane_right(r0), dl = lane_left(dd1), dr = lane_right(d0);
+        const bool rows = do_smooth && yo > 0 && yo < ny - 1;
+        if (rows && x > 0)
+            smooth_cell(r[0], d[0], rl, dl, rr1, dd1, r1[2][0], d1[2][0], r1[0][0], d1[0][0], k.smooth_m);
+        if (rows && x + 1 < nx - 1)
+            smooth_cell(r[1], d[1], r0, d0, rr, dr, r1[2][1], d1[2][1], r1[0][1], d1[0][1], k.smooth_m);
+        if (mine) {
+            const size_t g = at(x, yo, nx);
+            if (EXTRA && io.tr5) {
+                st_out2<NTS>(&io.tr5[g], r0, rr1);
+                st_out2<NTS>(&io.td6[g], d0, dd1);
+            }
+            st_out2<NTS>(&io.ro[g], r[0], r[1]);
+            st_out2<NTS>(&io.dout[g], d[0], d[1]);
+        }
+    };
+    if (!do_thermal) {                                       // smoothing alone
+        for (int y = ys - 1; y <= ye; ++y) {
+            const float2 r = load(io.r, y), d = load(io.d, y);
+            push(r.x, r.y, d.x, d.y);
+            if (y > ys) emit(y - 1);
+        }
+        return;
+    }
+    MarchLayer<0> l0{};
+    MarchLayer<1> l1{};
+    float2 nr = load(io.r, ys - TH), nd = make_float2(0.0f, 0.0f);
+    // y: the row layer 0 takes; layer 1 takes y - 2, smoothing gives y - 5
+    auto row = [&](int y, bool upper) {
+        const bool in = inx && iny(y);
+        MarchRow<0> b;
+        b.r[0] = in ? nr.x : HG_OOB_HEIGHT;
+        b.r[1] = in ? nr.y : HG_OOB_HEIGHT;
+        b.d[0] = b.d[1] = b.d_right = 0.0f;
+        const float2 dd = nd;
+        nr = load(io.r, y + 1);
+        if (upper) nd = load(io.d, y - 1);
+        b.r_right = lane_right(b.r[0]);
+        float rz[2];
+        march_advance<0>(l0, b, inx && iny(y - 1), inx && iny(y - 2), k, rz);
+        if (!upper) return;
+        const bool in2 = inx && iny(y - 2);
+        MarchRow<1> q;
+        q.r[0] = rz[0];
+        q.r[1] = rz[1];
+        q.d[0] = in2 ? dd.x : HG_OOB_HEIGHT;
+        q.d[1] = in2 ? dd.y : HG_OOB_HEIGHT;
+        q.r_right = lane_right(q.r[0]);
+        q.d_right = lane_right(q.d[0]);
+        const float rock[2] = {l1.z.r[0], l1.z.r[1]};        // rock of row y - 4
+        float dz[2];
+        march_advance<1>(l1, q, inx && iny(y - 3), inx && iny(y - 4), k, dz);
+        push(rock[0], rock[1], dz[0], dz[1]);
+        if (y - 5 >= ys && y - 5 < ye) emit(y - 5);
+    };
+    for (int y = ys - TH; y < ys - 1; ++y) row(y, false);
+    nd = load(io.d, ys - 3);
+    for (int y = ys - 1; y <= ye + 4; y += 2) {              // two at a time: the carried rows swap roles
+        row(y, true);
+        row(y + 1, true);
+    }
+}
+
+template <bool EXTRA, bool NTS>
+__global__ __launch_bounds__(256) void k_march_thermal(ThermIO io, int nx, int ny, int rows, int do_thermal,
+                                                       int do_smooth, int xcd, KParams k) {
+    const int gx = (nx + MARCH_TX - 1) / MARCH_TX;
+    int bx, by;
+    tile_of(blockIdx.x, gridDim.x, gx, xcd, bx, by);
+    const int ys = (by * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6)) * rows;
+    if (ys >= ny) return;
+    thermal_march<EXTRA, NTS>(io, nx, ny, bx * MARCH_TX, ys, min(ys + rows, ny), do_thermal, do_smooth, k);
+}
+
+// ---------------------------------------------------------------------------
 // Batched persistent kernels: one launch per pass covers the tiles of every
 // terrain of a batch.  Workgroup b processes work-list entries b, b+G, ...
 // (G = grid size); an entry packs (terrain << 24) | (tile_y << 12) | tile_x.
@@ -581,6 +892,31 @@ __global__ __launch_bounds__(NT) void k_batch_hydro(const BatchTerrain* __restri
         const int n = T.n;
         hydro_tile<TX, TY, HA, NT, false, NTS>(lds, io, n, n, bx, by, step, uint32_t(ti), rain, k);
         __syncthreads();
+    }
+}
+
+// The marching form over a work-list of MARCH_TX x MARCH_BATCH_TY entries.
+template <bool NTS>
+__global__ __launch_bounds__(256) void k_batch_march(const BatchTerrain* __restrict__ terr,
+                                                     const uint32_t* __restrict__ tiles, int ntiles, uint32_t cur,
+                                                     int do_thermal, int do_smooth) {
+    for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+        const uint32_t e = tiles[t];
+        if (e == 0xffffffffu) continue;
+        const int ti = int(e >> 24), by = int((e >> 12) & 0xfffu), bx = int(e & 0xfffu);
+        const BatchTerrain& T = terr[ti];
+        ThermIO io;
+        const int cr = cur & 1, cd = (cur >> 1) & 1;
+        io.r = T.plane[HG_P_ROCK][cr];
+        io.ro = T.plane[HG_P_ROCK][cr ^ 1];
+        io.d = T.plane[HG_P_DIRT][cd];
+        io.dout = T.plane[HG_P_DIRT][cd ^ 1];
+        const KParams k = T.k;
+        const int n = T.n;
+        const int ys = by * MARCH_BATCH_TY + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) * (MARCH_BATCH_TY / 4);
+        if (ys < n)
+            thermal_march<false, NTS>(io, n, n, bx * MARCH_TX, ys, min(ys + MARCH_BATCH_TY / 4, n), do_thermal, do_smooth,
+                                      k);
     }
 }
 
@@ -633,6 +969,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     X(8, 128, 32, 1024)        \
     X(9,  64, 16, 512)         \
     X(10, 64,  8, 1024)
+// the marching form follows them (in HG_THERMAL_VARIANTS' numbering)
+constexpr int MARCH_VARIANT = 11;
 
 }  // namespace
 
@@ -659,7 +997,7 @@ int default_hydro_variant(size_t cells) {
 }
 int default_thermal_variant(size_t cells) {
     const size_t tiles = cells / 1024;
-    return tiles < 128 ? 10 : tiles < 1024 ? 9 : 2;
+    return tiles < 128 ? 10 : tiles < 1024 ? 9 : tiles < 4096 ? 2 : MARCH_VARIANT;
 }
 
 int hydro_variant_count() {
@@ -670,7 +1008,7 @@ int hydro_variant_count() {
 
 int thermal_variant_count() {
 #define X(i, tx, ty, nt) +1
-    return 0 HG_THERMAL_VARIANTS(X);
+    return 1 HG_THERMAL_VARIANTS(X);
 #undef X
 }
 
@@ -686,6 +1024,7 @@ bool hydro_variant_info(int v, int* tx, int* ty, int* halo, int* nt) {
 
 bool thermal_variant_info(int v, int* tx, int* ty, int* halo, int* nt) {
     switch (v) {
+        case MARCH_VARIANT: *tx = MARCH_TX; *ty = MARCH_BATCH_TY; *halo = TH; *nt = 256; return true;
 #define X(i, TX_, TY_, NT_) \
     case i: *tx = TX_; *ty = TY_; *halo = TH; *nt = NT_; return true;
         HG_THERMAL_VARIANTS(X)
@@ -742,6 +1081,14 @@ hipError_t launch_batch_hydro(int variant, const BatchTerrain* terr, const uint3
 
 hipError_t launch_batch_thermal(int variant, const BatchTerrain* terr, const uint32_t* tiles, int ntiles,
                                 int grid, uint32_t cur, bool thermal, bool smooth, bool nts, hipStream_t s) {
+    if (variant == MARCH_VARIANT) {
+        const int th = thermal ? 1 : 0, sm = smooth ? 1 : 0;
+        if (nts)
+            k_batch_march<true><<<grid, 256, 0, s>>>(terr, tiles, ntiles, cur, th, sm);
+        else
+            k_batch_march<false><<<grid, 256, 0, s>>>(terr, tiles, ntiles, cur, th, sm);
+        return hipGetLastError();
+    }
     switch (variant) {
 #define X(i, TX_, TY_, NT_)                                                                   \
     case i:                                                                                   \
@@ -787,6 +1134,7 @@ int batch_hydro_blocks_per_cu(int variant) {
 int batch_thermal_blocks_per_cu(int variant) {
     int nb = 0;
     switch (variant) {
+        case MARCH_VARIANT: return 3;
 #define X(i, TX_, TY_, NT_)                                                                   \
     case i:                                                                                   \
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_batch_thermal<TX_, TY_, NT_, true>, \
@@ -802,6 +1150,20 @@ int batch_thermal_blocks_per_cu(int variant) {
 
 hipError_t launch_fused_thermal(int variant, const ThermIO& io, int nx, int ny, bool thermal,
                                 bool smooth, int xcd_mode, const KParams& k, hipStream_t s) {
+    if (variant == MARCH_VARIANT) {
+        const int rows = march_rows(nx, ny);
+        const unsigned grid = unsigned((nx + MARCH_TX - 1) / MARCH_TX) * unsigned((ny + 4 * rows - 1) / (4 * rows));
+        const int th = thermal ? 1 : 0, sm = smooth ? 1 : 0, xcd = tile_order(xcd_mode, nx, MARCH_TX, 4 * rows, 8);
+        if (io.tr5 && k.store_nt)
+            k_march_thermal<true, true><<<grid, 256, 0, s>>>(io, nx, ny, rows, th, sm, xcd, k);
+        else if (io.tr5)
+            k_march_thermal<true, false><<<grid, 256, 0, s>>>(io, nx, ny, rows, th, sm, xcd, k);
+        else if (k.store_nt)
+            k_march_thermal<false, true><<<grid, 256, 0, s>>>(io, nx, ny, rows, th, sm, xcd, k);
+        else
+            k_march_thermal<false, false><<<grid, 256, 0, s>>>(io, nx, ny, rows, th, sm, xcd, k);
+        return hipGetLastError();
+    }
     switch (variant) {
 #define X(i, TX_, TY_, NT_)                                                                  \
     case i: {                                                                                \
