@@ -42,6 +42,7 @@ struct hg_batch {
     int rain_mode = HG_RAIN_OFF;
     uint64_t seed = 0;
     int hydro_variant = 0, thermal_variant = 0;   // by size until tuned or set
+    int rows_t = 0;                     // rows of a thermal work-list entry
     size_t total_floats = 0;            // size of `block`
     bool persistent = false;            // false: one workgroup per work-list entry
     bool xcd_order = true;              // interleave the work-list for the 8 XCDs
@@ -162,6 +163,7 @@ int build_tiles(hg_batch* b) {
     hgk::hydro_variant_info(b->hydro_variant, &tx, &ty, &h, &nt);
     std::vector<uint32_t> lh = work_list(b, tx, ty);
     hgk::thermal_variant_info(b->thermal_variant, &tx, &ty, &h, &nt);
+    ty = b->rows_t = hgk::batch_thermal_rows(b->thermal_variant, b->n.data(), b->count);
     std::vector<uint32_t> lt = work_list(b, tx, ty);
     if (b->dev_tiles_h) (void)hipFree(b->dev_tiles_h);
     if (b->dev_tiles_t) (void)hipFree(b->dev_tiles_t);
@@ -183,7 +185,7 @@ int build_tiles(hg_batch* b) {
         hgk::hydro_variant_info(b->hydro_variant, &tx, &ty, &h, &nt);
         std::vector<uint32_t> nh = natural_list(b, tx, ty, &b->first_h, &b->count_h);
         hgk::thermal_variant_info(b->thermal_variant, &tx, &ty, &h, &nt);
-        std::vector<uint32_t> ntl = natural_list(b, tx, ty, &b->first_t, &b->count_t);
+        std::vector<uint32_t> ntl = natural_list(b, tx, b->rows_t, &b->first_t, &b->count_t);
         if (b->dev_nat_h) (void)hipFree(b->dev_nat_h);
         if (b->dev_nat_t) (void)hipFree(b->dev_nat_t);
         b->dev_nat_h = b->dev_nat_t = nullptr;
@@ -240,11 +242,11 @@ int enqueue_steps(hg_batch* b, uint32_t nsteps, uint32_t flags, bool per_terrain
         if (thermal || smooth) {
             if (per_terrain) {
                 for (int t = 0; t < b->count; ++t)
-                    BH(b, hgk::launch_batch_thermal(b->thermal_variant, b->dev_terr, b->dev_nat_t + b->first_t[t],
+                    BH(b, hgk::launch_batch_thermal(b->thermal_variant, b->rows_t, b->dev_terr, b->dev_nat_t + b->first_t[t],
                                                     b->count_t[t], b->count_t[t], b->cur, thermal, smooth, nts,
                                                     b->stream));
             } else {
-                BH(b, hgk::launch_batch_thermal(b->thermal_variant, b->dev_terr, b->dev_tiles_t, b->ntiles_t,
+                BH(b, hgk::launch_batch_thermal(b->thermal_variant, b->rows_t, b->dev_terr, b->dev_tiles_t, b->ntiles_t,
                                                 b->grid_t, b->cur, thermal, smooth, nts, b->stream));
             }
             b->cur ^= (1u << HG_P_ROCK) | (1u << HG_P_DIRT);

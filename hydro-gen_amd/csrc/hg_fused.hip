@@ -584,7 +584,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // once 104 -> 91 us per step.
 // ---------------------------------------------------------------------------
 constexpr int MARCH_TX = 116;          // columns a wave writes
-constexpr int MARCH_BATCH_TY = 192;    // rows of a batch's work-list entry, 48 per wave
 constexpr int MARCH_HX = 6;            // halo columns on each side (5 needed, even for the pairs)
 
 // Value of the next (right) and the previous (left) lane.
@@ -895,11 +894,11 @@ __global__ __launch_bounds__(NT) void k_batch_hydro(const BatchTerrain* __restri
     }
 }
 
-// The marching form over a work-list of MARCH_TX x MARCH_BATCH_TY entries.
+// The marching form over a work-list of MARCH_TX x (4 rows) entries.
 template <bool NTS>
 __global__ __launch_bounds__(256) void k_batch_march(const BatchTerrain* __restrict__ terr,
                                                      const uint32_t* __restrict__ tiles, int ntiles, uint32_t cur,
-                                                     int do_thermal, int do_smooth) {
+                                                     int rows, int do_thermal, int do_smooth) {
     for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const uint32_t e = tiles[t];
         if (e == 0xffffffffu) continue;
@@ -913,10 +912,8 @@ __global__ __launch_bounds__(256) void k_batch_march(const BatchTerrain* __restr
         io.dout = T.plane[HG_P_DIRT][cd ^ 1];
         const KParams k = T.k;
         const int n = T.n;
-        const int ys = by * MARCH_BATCH_TY + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) * (MARCH_BATCH_TY / 4);
-        if (ys < n)
-            thermal_march<false, NTS>(io, n, n, bx * MARCH_TX, ys, min(ys + MARCH_BATCH_TY / 4, n), do_thermal, do_smooth,
-                                      k);
+        const int ys = (by * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6)) * rows;
+        if (ys < n) thermal_march<false, NTS>(io, n, n, bx * MARCH_TX, ys, min(ys + rows, n), do_thermal, do_smooth, k);
     }
 }
 
@@ -1000,6 +997,26 @@ int default_thermal_variant(size_t cells) {
     return tiles < 128 ? 10 : tiles < 1024 ? 9 : tiles < 4096 ? 2 : MARCH_VARIANT;
 }
 
+// Rows of a thermal work-list entry for a batch of these sides.  The marching
+// form has no fixed tile: a workgroup's rows cost about rows / 4 + 6 (see
+// march_rows), times the rounds the entries take at 3 workgroups per CU.
+int batch_thermal_rows(int variant, const int* sides, int count) {
+    int tx = 0, ty = 0, h = 0, nt = 0;
+    if (!thermal_variant_info(variant, &tx, &ty, &h, &nt) || variant != MARCH_VARIANT) return ty;
+    long best_cost = 0;
+    for (int rows = 8; rows <= 96; ++rows) {
+        long entries = 0;
+        for (int t = 0; t < count; ++t)
+            entries += long((sides[t] + tx - 1) / tx) * ((sides[t] + 4 * rows - 1) / (4 * rows));
+        const long cost = (entries + 3 * 256 - 1) / (3 * 256) * (rows + 6);
+        if (rows == 8 || cost <= best_cost) {
+            best_cost = cost;
+            ty = 4 * rows;
+        }
+    }
+    return ty;
+}
+
 int hydro_variant_count() {
 #define X(i, tx, ty, ha, nt) +1
     return 0 HG_HYDRO_VARIANTS(X);
@@ -1024,7 +1041,7 @@ bool hydro_variant_info(int v, int* tx, int* ty, int* halo, int* nt) {
 
 bool thermal_variant_info(int v, int* tx, int* ty, int* halo, int* nt) {
     switch (v) {
-        case MARCH_VARIANT: *tx = MARCH_TX; *ty = MARCH_BATCH_TY; *halo = TH; *nt = 256; return true;
+        case MARCH_VARIANT: *tx = MARCH_TX; *ty = 4 * 48; *halo = TH; *nt = 256; return true;   // rows by size
 #define X(i, TX_, TY_, NT_) \
     case i: *tx = TX_; *ty = TY_; *halo = TH; *nt = NT_; return true;
         HG_THERMAL_VARIANTS(X)
@@ -1079,14 +1096,15 @@ hipError_t launch_batch_hydro(int variant, const BatchTerrain* terr, const uint3
     return hipGetLastError();
 }
 
-hipError_t launch_batch_thermal(int variant, const BatchTerrain* terr, const uint32_t* tiles, int ntiles,
-                                int grid, uint32_t cur, bool thermal, bool smooth, bool nts, hipStream_t s) {
+hipError_t launch_batch_thermal(int variant, int tile_rows, const BatchTerrain* terr, const uint32_t* tiles,
+                                int ntiles, int grid, uint32_t cur, bool thermal, bool smooth, bool nts,
+                                hipStream_t s) {
     if (variant == MARCH_VARIANT) {
         const int th = thermal ? 1 : 0, sm = smooth ? 1 : 0;
         if (nts)
-            k_batch_march<true><<<grid, 256, 0, s>>>(terr, tiles, ntiles, cur, th, sm);
+            k_batch_march<true><<<grid, 256, 0, s>>>(terr, tiles, ntiles, cur, tile_rows / 4, th, sm);
         else
-            k_batch_march<false><<<grid, 256, 0, s>>>(terr, tiles, ntiles, cur, th, sm);
+            k_batch_march<false><<<grid, 256, 0, s>>>(terr, tiles, ntiles, cur, tile_rows / 4, th, sm);
         return hipGetLastError();
     }
     switch (variant) {

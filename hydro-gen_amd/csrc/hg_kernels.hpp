@@ -137,8 +137,11 @@ hipError_t launch_batch_hydro(int variant, const BatchTerrain* terr, const uint3
                               bool rain, bool nts, hipStream_t s);
 // *step_ptr += n (a kernel, so it can sit in a captured graph)
 hipError_t launch_step_advance(uint32_t* step_ptr, uint32_t n, hipStream_t s);
-hipError_t launch_batch_thermal(int variant, const BatchTerrain* terr, const uint32_t* tiles, int ntiles,
-                                int grid, uint32_t cur, bool thermal, bool smooth, bool nts, hipStream_t s);
+// tile_rows: the rows of a work-list entry, batch_thermal_rows()
+int batch_thermal_rows(int variant, const int* sides, int count);
+hipError_t launch_batch_thermal(int variant, int tile_rows, const BatchTerrain* terr, const uint32_t* tiles,
+                                int ntiles, int grid, uint32_t cur, bool thermal, bool smooth, bool nts,
+                                hipStream_t s);
 int batch_hydro_blocks_per_cu(int variant);
 int batch_thermal_blocks_per_cu(int variant);
 
