@@ -1492,6 +1492,22 @@ extern "C" int hg_adjoint_rollout(hg_ctx* c, uint32_t nsteps, uint32_t k_ckpt, u
     HG_HIP(c, hipMemsetAsync(w.gpart, 0, nblk * 4 * sizeof(double), c->stream));
     const uint64_t step0 = c->step;
 
+    // ---- adjoint of the final state: dL/dH on rock and dirt.  Before the
+    // forward, so that the host waits for this copy with little queued and then
+    // stays ahead of the GPU through forward and reverse.
+    float* lam[HG_NUM_PLANES];
+    {
+        std::vector<float*> z;
+        for (int p = 0; p < HG_NUM_PLANES; ++p) z.push_back(lam[p] = take(w.pool));
+        const int rz = zero_planes(c, z, pn);
+        if (rz != HG_OK) return rz;
+    }
+    {
+        const int rc = write_floats(c, dL_dH_final, lam[HG_P_ROCK], pn);
+        if (rc != HG_OK) return rc;
+    }
+    HG_HIP(c, hipMemcpyAsync(lam[HG_P_DIRT], lam[HG_P_ROCK], pn * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
+
     // ---- forward with checkpoints every k_ckpt steps.  Segment `seg` is
     // reversed from plane set (nck - 1 - seg) % 2.  The last two segments (the
     // only one, if there is one) run through the taped kernels straight into
@@ -1536,17 +1552,6 @@ extern "C" int hg_adjoint_rollout(hg_ctx* c, uint32_t nsteps, uint32_t k_ckpt, u
         if (rc != HG_OK) return rc;
     }
     const uint64_t step_end = c->step;
-
-    // ---- adjoint of the final state: dL/dH on rock and dirt
-    float* lam[HG_NUM_PLANES];
-    {
-        std::vector<float*> z;
-        for (int p = 0; p < HG_NUM_PLANES; ++p) z.push_back(lam[p] = take(w.pool));
-        const int rz = zero_planes(c, z, pn);
-        if (rz != HG_OK) return rz;
-    }
-    HG_HIP(c, hipMemcpyAsync(lam[HG_P_ROCK], dL_dH_final, pn * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    HG_HIP(c, hipMemcpyAsync(lam[HG_P_DIRT], lam[HG_P_ROCK], pn * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
 
     // reverse units in forward order (they run from the last): a thermal
     // layer (outflow then transport) is one unit, named by its transport
@@ -1759,7 +1764,7 @@ extern "C" int hg_adjoint_rollout(hg_ctx* c, uint32_t nsteps, uint32_t k_ckpt, u
     }
     c->step = step_end;
     {
-        const int rc = read_pinned(c, lam[HG_P_ROCK], dL_dH0, pn);
+        const int rc = read_floats(c, lam[HG_P_ROCK], dL_dH0, pn);
         if (rc != HG_OK) return rc;
     }
     std::vector<double> part(nblk * 4);

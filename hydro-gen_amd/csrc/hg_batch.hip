@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "hg_hostcopy.hpp"
 #include "hg_kernels.hpp"
 
 using hgk::BatchTerrain;
@@ -31,6 +32,7 @@ struct hg_batch {
     std::vector<int> n;
     std::vector<size_t> offset;         // float offset of terrain t's plane block
     void* block = nullptr;              // 2 buffers x 9 planes per terrain
+    HostCopy copy;                      // to and from the caller's memory
     void* scratch = nullptr;            // per-pass baseline: velocity + thermal planes (largest terrain)
     std::vector<hg_erosion_settings> es;
     std::vector<BatchTerrain> terr;     // host copy of the descriptors
@@ -661,8 +663,7 @@ int hg_batch_read_plane(hg_batch* b, int terrain, int plane, float* dst, size_t 
         return bfail(b, HG_ERR_INVALID, "hg_batch_read_plane: bad argument");
     Guard g(b->device);
     const float* src = plane_ptr(b, terrain, plane, int((b->cur >> plane) & 1));
-    BH(b, hipMemcpyAsync(dst, src, n_floats * sizeof(float), hipMemcpyDeviceToHost, b->stream));
-    BH(b, hipStreamSynchronize(b->stream));
+    BH(b, b->copy.to_host(src, dst, n_floats * sizeof(float), b->stream));
     return HG_OK;
 }
 
@@ -673,8 +674,7 @@ int hg_batch_write_plane(hg_batch* b, int terrain, int plane, const float* src, 
         return bfail(b, HG_ERR_INVALID, "hg_batch_write_plane: bad argument");
     Guard g(b->device);
     float* dst = plane_ptr(b, terrain, plane, int((b->cur >> plane) & 1));
-    BH(b, hipMemcpyAsync(dst, src, n_floats * sizeof(float), hipMemcpyHostToDevice, b->stream));
-    BH(b, hipStreamSynchronize(b->stream));
+    BH(b, b->copy.to_device(src, dst, n_floats * sizeof(float), b->stream));
     return HG_OK;
 }
 

@@ -9,6 +9,7 @@
 #include <utility>
 #include <vector>
 
+#include "hg_hostcopy.hpp"
 #include "hg_kernels.hpp"
 
 using hgk::KParams;
@@ -71,11 +72,7 @@ struct hg_ctx {
     std::vector<KernelStat> stats;
     std::vector<PendingTiming> pending;
     std::vector<hipEvent_t> event_pool;
-    // pinned staging for device-to-host reads (two chunks, allocated on the
-    // first read): copies into pageable memory straight from the device ran
-    // at ~5 GB/s
-    void* pin[2] = {};
-    hipEvent_t pin_ev[2] = {};
+    HostCopy copy;                   // to and from the caller's memory
     float* rgba_dev = nullptr;       // 4 n^2 floats for hg_read's texels (allocated on first use)
 };
 
@@ -89,9 +86,10 @@ int stat_index(hg_ctx* c, const char* name);
 hipEvent_t take_event(hg_ctx* c);
 int run_pass(hg_ctx* c, int pass);
 int fused_step(hg_ctx* c, bool rain, bool thermal, bool smooth, bool keep_velocity);
-// n_floats from device `src` to host `dst` through the context's pinned chunks
-// (ordered after the work on the context's stream; returns when dst is filled)
-int read_pinned(hg_ctx* c, const float* src, float* dst, size_t n_floats);
+// n_floats from device `src` to host `dst` (ordered after the work on the
+// context's stream; returns when dst is filled), and from host to device
+int read_floats(hg_ctx* c, const float* src, float* dst, size_t n_floats);
+int write_floats(hg_ctx* c, const float* src, float* dst, size_t n_floats);
 
 // Launch helper: brackets the launch with events when timing is on.
 template <class F>

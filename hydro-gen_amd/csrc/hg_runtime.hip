@@ -238,43 +238,12 @@ bool finite_settings(const hg_erosion_settings* s) {
     return true;
 }
 
-// Device-to-host copy through the context's two pinned chunks: the copy of
-// chunk i+1 runs while chunk i is copied out to `dst`.
-constexpr size_t kPinChunk = size_t(16) << 20;
-int read_pinned(hg_ctx* c, const float* src, float* dst, size_t n_floats) {
-    for (int b = 0; b < 2; ++b) {            // each piece stored only once it exists
-        if (!c->pin[b]) {
-            void* p = nullptr;
-            HG_HIP(c, hipHostMalloc(&p, kPinChunk, hipHostMallocDefault));
-            c->pin[b] = p;
-        }
-        if (!c->pin_ev[b]) {
-            hipEvent_t e = nullptr;
-            HG_HIP(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-            c->pin_ev[b] = e;
-        }
-    }
-    const size_t bytes = n_floats * sizeof(float);
-    const char* s = reinterpret_cast<const char*>(src);
-    char* d = reinterpret_cast<char*>(dst);
-    auto issue = [&](size_t off, int b) -> int {
-        const size_t len = std::min(kPinChunk, bytes - off);
-        HG_HIP(c, hipMemcpyAsync(c->pin[b], s + off, len, hipMemcpyDeviceToHost, c->stream));
-        HG_HIP(c, hipEventRecord(c->pin_ev[b], c->stream));
-        return HG_OK;
-    };
-    if (bytes == 0) return HG_OK;
-    int rc = issue(0, 0);
-    if (rc != HG_OK) return rc;
-    for (size_t off = 0, k = 0; off < bytes; off += kPinChunk, ++k) {
-        const int b = int(k & 1);
-        if (off + kPinChunk < bytes) {           // the other chunk was copied out last round
-            rc = issue(off + kPinChunk, 1 - b);
-            if (rc != HG_OK) return rc;
-        }
-        HG_HIP(c, hipEventSynchronize(c->pin_ev[b]));
-        std::memcpy(d + off, c->pin[b], std::min(kPinChunk, bytes - off));
-    }
+int read_floats(hg_ctx* c, const float* src, float* dst, size_t n_floats) {
+    HG_HIP(c, c->copy.to_host(src, dst, n_floats * sizeof(float), c->stream));
+    return HG_OK;
+}
+int write_floats(hg_ctx* c, const float* src, float* dst, size_t n_floats) {
+    HG_HIP(c, c->copy.to_device(src, dst, n_floats * sizeof(float), c->stream));
     return HG_OK;
 }
 
@@ -373,10 +342,6 @@ int hg_destroy(hg_ctx* c) {
     if (c->adj_block) (void)hipFree(c->adj_block);
     if (c->rgba_dev) (void)hipFree(c->rgba_dev);
     if (c->drop_order) (void)hipFree(c->drop_order);
-    for (int b = 0; b < 2; ++b) {
-        if (c->pin[b]) (void)hipHostFree(c->pin[b]);
-        if (c->pin_ev[b]) (void)hipEventDestroy(c->pin_ev[b]);
-    }
     (void)hipStreamDestroy(c->stream);
     delete c;
     return HG_OK;
@@ -683,8 +648,7 @@ int hg_ref_particles_read(hg_ctx* c, hg_ref_particle* out, uint32_t count) {
     if (!c || !out) return HG_ERR_INVALID;
     if (count != c->refp_count) return fail(c, HG_ERR_INVALID, "hg_ref_particles_read: count differs from hg_ref_particles_init");
     DeviceGuard guard(c->device);
-    HG_HIP(c, hipMemcpyAsync(out, c->refp, size_t(count) * sizeof(hg_ref_particle), hipMemcpyDeviceToHost, c->stream));
-    HG_HIP(c, hipStreamSynchronize(c->stream));
+    HG_HIP(c, c->copy.to_host(c->refp, out, size_t(count) * sizeof(hg_ref_particle), c->stream));
     return HG_OK;
 }
 
@@ -692,8 +656,7 @@ int hg_ref_particles_write(hg_ctx* c, const hg_ref_particle* in, uint32_t count)
     if (!c || !in) return HG_ERR_INVALID;
     if (count != c->refp_count) return fail(c, HG_ERR_INVALID, "hg_ref_particles_write: count differs from hg_ref_particles_init");
     DeviceGuard guard(c->device);
-    HG_HIP(c, hipMemcpyAsync(c->refp, in, size_t(count) * sizeof(hg_ref_particle), hipMemcpyHostToDevice, c->stream));
-    HG_HIP(c, hipStreamSynchronize(c->stream));
+    HG_HIP(c, c->copy.to_device(in, c->refp, size_t(count) * sizeof(hg_ref_particle), c->stream));
     return HG_OK;
 }
 
@@ -795,7 +758,7 @@ int hg_read_plane(hg_ctx* c, int plane, float* dst, size_t n_floats) {
     if (plane < 0 || plane >= HG_NUM_PLANES) return fail(c, HG_ERR_INVALID, "hg_read_plane: bad plane");
     if (!dst || n_floats != plane_n(c)) return fail(c, HG_ERR_INVALID, "hg_read_plane: bad buffer size");
     DeviceGuard guard(c->device);
-    return read_pinned(c, c->cur[plane], dst, n_floats);
+    return read_floats(c, c->cur[plane], dst, n_floats);
 }
 
 int hg_write_plane(hg_ctx* c, int plane, const float* src, size_t n_floats) {
@@ -803,9 +766,7 @@ int hg_write_plane(hg_ctx* c, int plane, const float* src, size_t n_floats) {
     if (plane < 0 || plane >= HG_NUM_PLANES) return fail(c, HG_ERR_INVALID, "hg_write_plane: bad plane");
     if (!src || n_floats != plane_n(c)) return fail(c, HG_ERR_INVALID, "hg_write_plane: bad buffer size");
     DeviceGuard guard(c->device);
-    HG_HIP(c, hipMemcpyAsync(c->cur[plane], src, n_floats * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    HG_HIP(c, hipStreamSynchronize(c->stream));
-    return HG_OK;
+    return write_floats(c, src, c->cur[plane], n_floats);
 }
 
 int hg_read(hg_ctx* c, int channel, float* rgba, size_t n_floats) {
@@ -820,7 +781,7 @@ int hg_read(hg_ctx* c, int channel, float* rgba, size_t n_floats) {
         case HG_CH_SEDIMENT: planes[0] = HG_P_SED_ROCK; planes[1] = HG_P_SED_DIRT; break;
         default: return fail(c, HG_ERR_INVALID, "hg_read: bad channel");
     }
-    // texels assembled on the device, then one copy through the pinned chunks
+    // texels assembled on the device, then one copy to the host
     DeviceGuard guard(c->device);
     if (!c->rgba_dev) {
         void* p = nullptr;
@@ -830,7 +791,7 @@ int hg_read(hg_ctx* c, int channel, float* rgba, size_t n_floats) {
     const float* src[4];
     for (int k = 0; k < 4; ++k) src[k] = planes[k] < 0 ? nullptr : c->cur[planes[k]];
     HG_HIP(c, hgk::launch_interleave_rgba(c->rgba_dev, src, pn, channel == HG_CH_HEIGHT, c->stream));
-    return read_pinned(c, c->rgba_dev, rgba, 4 * pn);
+    return read_floats(c, c->rgba_dev, rgba, 4 * pn);
 }
 
 // ---- heightmap files: NumPy .npy v1.0, little-endian float32, shape (n, n, 4)
@@ -907,7 +868,8 @@ int hg_write(hg_ctx* c, int channel, const float* rgba, size_t n_floats) {
         HG_HIP(c, hipMalloc(&p, 4 * pn * sizeof(float)));
         c->rgba_dev = static_cast<float*>(p);
     }
-    HG_HIP(c, hipMemcpyAsync(c->rgba_dev, rgba, 4 * pn * sizeof(float), hipMemcpyHostToDevice, c->stream));
+    const int rc = write_floats(c, rgba, c->rgba_dev, 4 * pn);
+    if (rc != HG_OK) return rc;
     float* dst[4];
     for (int k = 0; k < 4; ++k) dst[k] = planes[k] < 0 ? nullptr : c->cur[planes[k]];
     HG_HIP(c, hgk::launch_deinterleave_rgba(c->rgba_dev, dst, pn, c->stream));
