@@ -1399,12 +1399,17 @@ int step_into(hg_ctx* c, float* const* in, float* const* out, float* const* tp, 
     io.s0o = out[HG_P_SED_ROCK]; io.s1o = out[HG_P_SED_DIRT];
     io.vx = tp[T_VX]; io.vy = tp[T_VY]; io.vz = tp[T_VZ];
     io.tb1 = tp[T_B1]; io.tb2 = tp[T_B2]; io.ts0 = tp[T_S0]; io.ts1 = tp[T_S1];
-    HG_HIP(c, hgk::launch_fused_hydro(c->hydro_variant, io, c->n, c->n, step, 0u, rain, c->xcd_order, c->kp, st));
-    if (!th) return HG_OK;
     hgk::ThermIO tio;
     tio.r = tp[T_R3]; tio.d = tp[T_D3];
     tio.ro = out[HG_P_ROCK]; tio.dout = out[HG_P_DIRT];
     tio.tr5 = tp[T_R5]; tio.td6 = tp[T_D6];
+    if (th && c->step_variant() >= hgk::step_tile_first()) {
+        HG_HIP(c, hgk::launch_step_tile(c->step_variant() - hgk::step_tile_first(), io, tio, c->n, c->n, step, 0u, rain,
+                                        thermal, smooth, c->xcd_order, c->kp, st));
+        return HG_OK;
+    }
+    HG_HIP(c, hgk::launch_fused_hydro(c->hydro_variant, io, c->n, c->n, step, 0u, rain, c->xcd_order, c->kp, st));
+    if (!th) return HG_OK;
     HG_HIP(c, hgk::launch_fused_thermal(c->thermal_variant, tio, c->n, c->n, thermal, smooth, c->xcd_order, c->kp,
                                         st));
     return HG_OK;

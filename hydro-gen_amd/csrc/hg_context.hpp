@@ -49,7 +49,12 @@ struct hg_ctx {
     unsigned long long* dev_dsteps = nullptr;
     int hydro_variant = 0;           // fused kernel tile variants (see hg_autotune)
     int thermal_variant = 0;
-    int sweep_variant = 0;           // one-kernel step variant; -1: the hydro and thermal kernels
+    int sweep_variant = -1;          // one-kernel step variant; -1: the hydro and thermal kernels
+    // the one-kernel variant of a small map whose steps were neither tuned nor
+    // set (hg_set_sweep); -1: none.  Not while launches are timed, so that
+    // the two kernels are seen apart.
+    int small_map_variant = -1;
+    int step_variant() const { return sweep_variant < 0 && !timing ? small_map_variant : sweep_variant; }
     int xcd_order = 2;               // fused kernels' tile order (hg_set_xcd_order)
     float rain_time = 0.0f;          // HG_RAIN_REFERENCE time seed
     float map_max_height = 256.0f;   // HG_RAIN_REFERENCE mountain scale (src/settings.hpp:30)

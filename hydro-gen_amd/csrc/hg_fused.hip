@@ -142,7 +142,10 @@ struct HydroTile {
 // EXTRA: also write the optional outputs (velocity, adjoint tape) that are
 // not null; without it their pointers are never read, which keeps them out
 // of the scalar registers of the common case.
-template <int TX, int TY, int HA, int NT, bool EXTRA = false, bool NTS = false>
+// STEP (k_step_tile): rock and dirt after erosion are left in LDS on the whole
+// region, as the thermal stages take them (see StepTile), and written to memory
+// only as part of the tape.
+template <int TX, int TY, int HA, int NT, bool EXTRA = false, bool NTS = false, bool STEP = false>
 __device__ __forceinline__ void hydro_tile(float* lds, const HydroIO& io, int nx, int ny, int bx,
                                            int by, uint32_t step, uint32_t terrain, int rain,
                                            const KParams& k) {
@@ -231,6 +234,11 @@ __device__ __forceinline__ void hydro_tile(float* lds, const HydroIO& io, int nx
     // rock, dirt and sediment of the region, at clamped addresses, all
     // issued before the first cell is evaluated
     float gr[IE], gd[IE], g0[IE], g1[IE];
+    float er[STEP ? IE : 1], ed[STEP ? IE : 1];
+    if constexpr (STEP) {
+#pragma unroll
+        for (int it = 0; it < IE; ++it) er[it] = ed[it] = HG_OOB_HEIGHT;
+    }
     walk([&](int it, int ex, int ey) {
         const int gx = min(max(x0 - HA + ex, 0), nx - 1), gy = min(max(y0 - HA + ey, 0), ny - 1);
         const size_t g = at(gx, gy, nx);
@@ -259,10 +267,13 @@ __device__ __forceinline__ void hydro_tile(float* lds, const HydroIO& io, int nx
         erosion_cell(r, d, s0, s1, vx, vy, vz, s_rd[li - 1], s_rd[li + 1], s_rd[li + T::WI],
                      s_rd[li - T::WI], k);
         es0[it] = s0; es1[it] = s1; evx[it] = vx; evy[it] = vy;
+        if constexpr (STEP) { er[it] = r; ed[it] = d; }
         const bool tile = ex >= HA && ex < HA + TX && ey >= HA && ey < HA + TY;
         if (tile) {
-            st_out<NTS>(&io.ro[g], r);
-            st_out<NTS>(&io.dout[g], d);
+            if (!STEP || EXTRA) {
+                st_out<NTS>(&io.ro[g], r);
+                st_out<NTS>(&io.dout[g], d);
+            }
             st_out<NTS>(&io.bo[g], d2 * k.evap);     // sediment_transport.glsl:75
             st_out<NTS>(&io.flo[g], f[0]);
             st_out<NTS>(&io.fro[g], f[1]);
@@ -296,6 +307,11 @@ __device__ __forceinline__ void hydro_tile(float* lds, const HydroIO& io, int nx
             const int t = (ey - HA) * TX + (ex - HA);
             s_vx[t] = evx[it];
             s_vy[t] = evy[it];
+        }
+        if constexpr (STEP) {
+            float* s_r = lds + 2 * T::NE + 2 * T::NTILE;
+            s_r[e] = er[it];
+            s_r[T::NE + e] = ed[it];
         }
     });
     __syncthreads();
@@ -414,7 +430,8 @@ struct ThermalTile {
 };
 
 // One output tile (bx, by) of the thermal kernel; `lds` holds 3*N0 floats.
-template <int TX, int TY, int NT, bool EXTRA = false, bool NTS = false>
+// LOADED: its first two arrays already hold rock and dirt.
+template <int TX, int TY, int NT, bool EXTRA = false, bool NTS = false, bool LOADED = false>
 __device__ __forceinline__ void thermal_tile(float* lds, const ThermIO& io, int nx, int ny, int bx,
                                              int by, int do_thermal, int do_smooth, const KParams& k) {
     constexpr int W0 = ThermalTile<TX, TY>::W0, N0 = ThermalTile<TX, TY>::N0;
@@ -438,7 +455,7 @@ __device__ __forceinline__ void thermal_tile(float* lds, const ThermIO& io, int 
 
     // load rock, dirt; out of grid reads HG_OOB_HEIGHT (thermal_erosion.glsl:20-26).
     // Loads use clamped addresses and are all issued before the first LDS write.
-    {
+    if constexpr (!LOADED) {
         constexpr int IL = Region<TX, TY, NT, TH>::ITER;
         float lr[IL], ld[IL];
         region_for<TX, TY, NT, TH>(tid, [&](int it, int lx, int ly) {
@@ -452,8 +469,8 @@ __device__ __forceinline__ void thermal_tile(float* lds, const ThermIO& io, int 
             s_r[ly * W0 + lx] = lr[it];
             s_d[ly * W0 + lx] = ld[it];
         });
+        __syncthreads();
     }
-    __syncthreads();
 
     if (do_thermal) {
         // ---- A: layer-0 outflow scale
@@ -551,6 +568,43 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     int bx, by;
     tile_of(blockIdx.x, gridDim.x, (nx + TX - 1) / TX, xcd, bx, by);
     thermal_tile<TX, TY, NT, EXTRA, NTS>(lds, io, nx, ny, bx, by, do_thermal, do_smooth, k);
+}
+
+// ---------------------------------------------------------------------------
+// The whole step on one tile, for small maps
+//
+// A small map's step is bound by its launches, not by their work: two kernels
+// of about 6 us each with 4 us between them, and 3 us of host time per launch.
+// One launch does both: the hydro stages run on the tile +- 5 cells the thermal
+// stages need (2 cells otherwise), hand rock and dirt over in LDS, and the
+// halo's repeated work is the price (2.1 times the cells of a 32 x 16 tile, 3
+// times those of a 32 x 8 one).  us per step, alone / with three maps at once:
+//         two kernels  32x8/768   32x16/512  64x16/1024
+//    64^2  10.8/ 6.0    6.7/ 3.3   9.7/ 3.6  10.3/ 3.8
+//   256^2  12.9/ 6.4    8.4/ 3.6  11.2/ 4.2  11.0/ 4.3
+//   384^2  17.1/ 8.1   12.7/ 7.0  12.8/ 5.3  11.4/ 6.3
+//   512^2  20.4/10.2   17.1/12.2  15.8/ 7.9  14.5/11.9
+//   640^2  23.7/12.5   24.8/18.8  21.7/12.1  21.7/16.3
+//   768^2  28.2/14.4   31.5/26.8  26.0/17.3  32.0/22.8
+// ---------------------------------------------------------------------------
+template <int TX, int TY>
+struct StepTile {
+    using H = HydroTile<TX, TY, TH, 64>;
+    static constexpr int THERMAL = 2 * H::NE + 2 * H::NTILE;     // rock, dirt, g of the thermal stages
+    static constexpr int NLDS = 6 * H::NLDS > THERMAL + 3 * H::NE ? 6 * H::NLDS : THERMAL + 3 * H::NE;
+    static_assert(H::NE == ThermalTile<TX, TY>::N0, "both stages number the tile +- 5 cells alike");
+};
+
+template <int TX, int TY, int NT, bool EXTRA>
+__global__ __launch_bounds__(NT) void k_step_tile(HydroIO io, ThermIO tio, int nx, int ny, uint32_t step,
+                                                  uint32_t terrain, int rain, int do_thermal, int do_smooth, int xcd,
+                                                  KParams k) {
+    __shared__ float lds[StepTile<TX, TY>::NLDS];
+    int bx, by;
+    tile_of(blockIdx.x, gridDim.x, (nx + TX - 1) / TX, xcd, bx, by);
+    hydro_tile<TX, TY, TH, NT, EXTRA, false, true>(lds, io, nx, ny, bx, by, step, terrain, rain, k);
+    thermal_tile<TX, TY, NT, EXTRA, false, true>(lds + StepTile<TX, TY>::THERMAL, tio, nx, ny, bx, by, do_thermal,
+                                                 do_smooth, k);
 }
 
 // ---------------------------------------------------------------------------
@@ -1070,6 +1124,53 @@ hipError_t launch_fused_hydro(int variant, const HydroIO& io, int nx, int ny, ui
         break;                                                                                \
     }
         HG_HYDRO_VARIANTS(X)
+#undef X
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+//                        TX  TY   NT
+#define HG_STEP_TILES(X)  \
+    X(0, 32,  8, 768)     \
+    X(1, 32, 16, 512)
+
+// The k_step_tile variant of a map of `cells` cells that was not tuned; -1: the
+// two kernels (figures at k_step_tile).
+int default_step_tile(size_t cells) { return cells <= 288 * 288 ? 0 : cells <= 648 * 648 ? 1 : -1; }
+
+int step_tile_count() {
+#define X(i, tx, ty, nt) +1
+    return 0 HG_STEP_TILES(X);
+#undef X
+}
+
+bool step_tile_info(int v, int* tx, int* ty, int* nt) {
+    switch (v) {
+#define X(i, TX_, TY_, NT_) \
+    case i: *tx = TX_; *ty = TY_; *nt = NT_; return true;
+        HG_STEP_TILES(X)
+#undef X
+        default: return false;
+    }
+}
+
+hipError_t launch_step_tile(int variant, const HydroIO& io, const ThermIO& tio, int nx, int ny, uint32_t step,
+                            uint32_t terrain, bool rain, bool thermal, bool smooth, int xcd_mode, const KParams& k,
+                            hipStream_t s) {
+    switch (variant) {
+#define X(i, TX_, TY_, NT_)                                                                       \
+    case i: {                                                                                     \
+        const unsigned grid = unsigned((nx + TX_ - 1) / TX_) * unsigned((ny + TY_ - 1) / TY_);    \
+        const int xcd = tile_order(xcd_mode, nx, TX_, TY_, 36);                                   \
+        const int r = rain ? 1 : 0, th = thermal ? 1 : 0, sm = smooth ? 1 : 0;                    \
+        if (io.tb1)                                                                               \
+            k_step_tile<TX_, TY_, NT_, true><<<grid, NT_, 0, s>>>(io, tio, nx, ny, step, terrain, r, th, sm, xcd, k);  \
+        else                                                                                      \
+            k_step_tile<TX_, TY_, NT_, false><<<grid, NT_, 0, s>>>(io, tio, nx, ny, step, terrain, r, th, sm, xcd, k); \
+        break;                                                                                    \
+    }
+        HG_STEP_TILES(X)
 #undef X
         default: return hipErrorInvalidValue;
     }

@@ -33,7 +33,6 @@ struct TunedTiles {
     int hydro, thermal, sweep;
 };
 std::map<std::pair<int, std::string>, TunedTiles> g_tune_cache;
-constexpr int DEFAULT_SWEEP_VARIANT = -1;
 
 }  // namespace
 
@@ -196,10 +195,11 @@ int fused_step(hg_ctx* c, bool rain, bool thermal, bool smooth, bool keep_veloci
     io.vy = keep_velocity ? c->alt[HG_P_VEL_V] : nullptr;
     io.vz = keep_velocity ? c->alt[HG_P_VEL_DEPTH] : nullptr;
     const uint32_t step = uint32_t(c->step);
-    if (c->sweep_variant >= 0 && !keep_velocity) {
+    const int one_kernel = c->step_variant();
+    if (one_kernel >= 0 && !keep_velocity) {
         // the whole step in one kernel; rock and dirt come out of its last pass
         const int rc = timed_launch(c, "step_sweep", [&] {
-            return hgk::launch_step_sweep(c->sweep_variant, io, c->n, step, 0u, rain, thermal, smooth, c->kp,
+            return hgk::launch_step_sweep(one_kernel, io, c->n, step, 0u, rain, thermal, smooth, c->kp,
                                           c->stream);
         });
         if (rc != HG_OK) return rc;
@@ -311,7 +311,8 @@ int hg_create(int device, uint32_t n, uint32_t particle_count, hg_ctx** out) {
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->arch = prop.gcnArchName;
     c->hydro_variant = hgk::default_hydro_variant(pn);
     c->thermal_variant = hgk::default_thermal_variant(pn);
-    c->sweep_variant = DEFAULT_SWEEP_VARIANT;
+    const int tile = hgk::default_step_tile(pn);
+    c->small_map_variant = tile < 0 ? -1 : hgk::step_tile_first() + tile;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         auto it = g_tune_cache.find({c->n, c->arch});
@@ -319,6 +320,7 @@ int hg_create(int device, uint32_t n, uint32_t particle_count, hg_ctx** out) {
             c->hydro_variant = it->second.hydro;
             c->thermal_variant = it->second.thermal;
             c->sweep_variant = it->second.sweep;
+            c->small_map_variant = -1;
         }
     }
     *out = c;
@@ -957,6 +959,7 @@ int hg_set_sweep(hg_ctx* c, int variant) {
     if (variant < -1 || variant >= hgk::sweep_variant_count())
         return fail(c, HG_ERR_INVALID, "hg_set_sweep: variant is -1 or a HG_KERNEL_SWEEP variant");
     c->sweep_variant = variant;
+    c->small_map_variant = -1;
     return HG_OK;
 }
 
@@ -1025,7 +1028,9 @@ int hg_autotune(hg_ctx* c, uint32_t steps, uint32_t flags, int* hydro_best, int*
     int sweep_pick = -1;
     {
         double best_step = (thermal || smooth) ? best[0] + best[1] : best[0];
-        for (int v = 0; v < hgk::sweep_variant_count() && rc == HG_OK; ++v) {
+        // (the small maps' tiles only where they can win)
+        const int nv = pn <= size_t(1024) * 1024 ? hgk::sweep_variant_count() : hgk::step_tile_first();
+        for (int v = 0; v < nv && rc == HG_OK; ++v) {
             c->sweep_variant = v;
             rc = fused_step(c, rain, thermal, smooth, false);   // warm-up
             if (rc == HG_OK) rc = resolve_timing(c);
@@ -1053,6 +1058,7 @@ int hg_autotune(hg_ctx* c, uint32_t steps, uint32_t flags, int* hydro_best, int*
         c->sweep_variant = s0;
         return rc;
     }
+    c->small_map_variant = -1;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tune_cache[{c->n, c->arch}] = {pick[0], pick[1], sweep_pick};

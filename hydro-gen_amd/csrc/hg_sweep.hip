@@ -681,12 +681,14 @@ __global__ __launch_bounds__(64 * WV_WAVES) __attribute__((amdgpu_waves_per_eu(O
 }  // namespace
 
 // Variants 0 .. (wave variants - 1) are the one-wave-per-strip kernel, the
-// rest the workgroup kernel with LDS rings.
-int sweep_variant_count() {
+// next ones the workgroup kernel with LDS rings, and from step_tile_first() on
+// the tile kernel of small maps (k_step_tile).
+int step_tile_first() {
 #define X(i, ...) +1
     return 0 HG_WAVE_VARIANTS(X) HG_SWEEP_VARIANTS(X);
 #undef X
 }
+int sweep_variant_count() { return step_tile_first() + step_tile_count(); }
 
 namespace {
 constexpr int kWaveVariants = 0
@@ -697,6 +699,11 @@ constexpr int kWaveVariants = 0
 }  // namespace
 
 bool sweep_variant_info(int v, int* strip_w, int* rows, int* threads, int* seg_rows) {
+    if (v >= step_tile_first()) {
+        if (!step_tile_info(v - step_tile_first(), strip_w, seg_rows, threads)) return false;
+        *rows = *seg_rows;
+        return true;
+    }
     if (v < kWaveVariants) {
         switch (v) {
 #define X(i, RS_, OCC_) \
@@ -717,6 +724,14 @@ bool sweep_variant_info(int v, int* strip_w, int* rows, int* threads, int* seg_r
 
 hipError_t launch_step_sweep(int variant, const HydroIO& io, int n, uint32_t step, uint32_t terrain, bool rain,
                              bool thermal, bool smooth, const KParams& k, hipStream_t s) {
+    if (variant >= step_tile_first()) {
+        HydroIO h = io;
+        ThermIO t{};
+        t.ro = io.ro;
+        t.dout = io.dout;
+        h.ro = h.dout = nullptr;
+        return launch_step_tile(variant - step_tile_first(), h, t, n, n, step, terrain, rain, thermal, smooth, 2, k, s);
+    }
     SweepArgs a;
     a.io = io; a.n = n;
     a.step = step; a.terrain = terrain;

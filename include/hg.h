@@ -465,13 +465,16 @@ int hg_get_tiles(const hg_ctx* ctx, int* hydro_variant, int* thermal_variant);
  * L2 (the default).  Returns HG_ERR_INVALID for other modes. */
 int hg_set_xcd_order(hg_ctx* ctx, int mode);
 /* One-kernel steps.  With a HG_KERNEL_SWEEP variant, hg_step_grid runs
- * each fused step as one kernel: each wave (variants 0-4) or workgroup (the
- * rest) sweeps a strip of columns row by row and runs every pass of the step
+ * each fused step as one kernel: each wave (variants 0-4) or workgroup (5-9)
+ * sweeps a strip of columns row by row and runs every pass of the step
  * a few rows behind the one it depends on, so the step reads and writes its
- * 9 state planes once.  -1 (the default, kept by hg_autotune unless a
- * one-kernel variant times faster) runs the hydro kernel and then the
- * thermal kernel.  Both give the per-pass result bit for bit; steps with
- * HG_STEP_KEEP_VELOCITY always use the two kernels. */
+ * 9 state planes once.  The last variants instead work tile by tile, with a
+ * halo of 5 cells, and are for small maps, whose steps are bound by their
+ * launches.  -1 (the default, kept by hg_autotune unless a one-kernel variant
+ * times faster) runs the hydro kernel and then the thermal kernel; until this
+ * call or hg_autotune, a map of up to 648 x 648 cells runs a tile variant
+ * instead while launches are not timed.  All give the per-pass result bit for
+ * bit; steps with HG_STEP_KEEP_VELOCITY always use the two kernels. */
 int hg_set_sweep(hg_ctx* ctx, int variant);
 int hg_get_sweep(const hg_ctx* ctx, int* variant);
 /* Times `steps` fused steps per variant (state and step counter are restored
