@@ -21,6 +21,7 @@
 // recomputes the eroded sediment of those taps from the step's input planes
 // (still intact: every pass is ping-pong), which is exact.
 #include <algorithm>
+#include <type_traits>
 
 #include "hg_kernels.hpp"
 
@@ -133,7 +134,14 @@ struct HydroTile {
     static constexpr int NTILE = TX * TY;
     static constexpr int ITER_T = (NTILE + NT - 1) / NT;
     static constexpr int NLDS = WI * HI;
-    static_assert(2 * NE + 2 * NTILE <= 6 * NLDS, "aliased outputs must fit the input arrays");
+    // Where the list of cells with far taps lies after stage 1 (in the place of
+    // the thermal stages' g in a STEP), and its length's distance from it.
+    template <bool STEP>
+    static constexpr int FAR = 2 * NE + 2 * NTILE + (STEP ? 2 * NE : 0);
+    template <bool STEP>
+    static constexpr int NFAR = STEP ? NE : NTILE;
+    static_assert(NTILE <= NE, "the list fits g's place");
+    static_assert(FAR<false> + NFAR<false> < 6 * NLDS, "aliased outputs must fit the input arrays");
     static_assert(TX % 4 == 0, "tile width must be a multiple of 4");
 };
 
@@ -299,6 +307,7 @@ __device__ __forceinline__ void hydro_tile(float* lds, const HydroIO& io, int nx
     float* s_s1 = lds + T::NE;
     float* s_vx = lds + 2 * T::NE;
     float* s_vy = lds + 2 * T::NE + T::NTILE;
+    if (tid == 0) reinterpret_cast<int*>(lds)[T::template FAR<STEP> + T::template NFAR<STEP>] = 0;
     walk([&](int it, int ex, int ey) {
         const int e = ey * T::WE + ex;
         s_s0[e] = es0[it];
@@ -317,47 +326,74 @@ __device__ __forceinline__ void hydro_tile(float* lds, const HydroIO& io, int nx
     __syncthreads();
 
     // ---- stage 2: back-trace + bilinear gather on the tile -----------------
+    // Cells whose taps leave the halo are listed and done afterwards, four
+    // lanes to a cell, one per tap: done where they are met, each wave with such
+    // a lane recomputed its four taps one after the other.
+    int* s_far = reinterpret_cast<int*>(lds) + T::template FAR<STEP>;
+    int* s_nfar = s_far + T::template NFAR<STEP>;
+    struct Taps {
+        int ix, iy, ix1, iy1;
+        float fx, fy;
+    };
+    auto taps_of = [&](int t) {
+        const int ty = t / TX, tx = t - ty * TX;
+        float bx, by;
+        back_trace(x0 + tx, y0 + ty, s_vx[t], s_vy[t], k.dt, nx, ny, bx, by);
+        Taps p;
+        p.ix = int(bx);
+        p.iy = int(by);
+        p.fx = bx - float(p.ix);
+        p.fy = by - float(p.iy);
+        p.ix1 = min(p.ix + 1, nx - 1);
+        p.iy1 = min(p.iy + 1, ny - 1);
+        return p;
+    };
     for (int t = tid; t < T::NTILE; t += NT) {
         const int ty = t / TX, tx = t - ty * TX;
         const int gx = x0 + tx, gy = y0 + ty;
         if (gx >= nx || gy >= ny) continue;
-        float bx, by;
-        back_trace(gx, gy, s_vx[t], s_vy[t], k.dt, nx, ny, bx, by);
-        const int ix = int(bx), iy = int(by);
-        const float fx = bx - float(ix), fy = by - float(iy);
-        const int ix1 = min(ix + 1, nx - 1), iy1 = min(iy + 1, ny - 1);
+        const Taps p = taps_of(t);
         // region-local coordinates of the taps
-        const int ex0 = ix - (x0 - HA), ey0 = iy - (y0 - HA);
-        const int ex1 = ix1 - (x0 - HA), ey1 = iy1 - (y0 - HA);
-        float o0, o1;
+        const int ex0 = p.ix - (x0 - HA), ey0 = p.iy - (y0 - HA);
+        const int ex1 = p.ix1 - (x0 - HA), ey1 = p.iy1 - (y0 - HA);
         if (ex0 >= 0 && ey0 >= 0 && ex1 < T::WE && ey1 < T::HE) {
             const int e00 = ey0 * T::WE + ex0, e10 = ey0 * T::WE + ex1;
             const int e01 = ey1 * T::WE + ex0, e11 = ey1 * T::WE + ex1;
-            o0 = lerp1(lerp1(s_s0[e00], s_s0[e10], fx), lerp1(s_s0[e01], s_s0[e11], fx), fy);
-            o1 = lerp1(lerp1(s_s1[e00], s_s1[e10], fx), lerp1(s_s1[e01], s_s1[e11], fx), fy);
+            const size_t g = at(gx, gy, nx);
+            st_out<NTS>(&io.s0o[g], lerp1(lerp1(s_s0[e00], s_s0[e10], p.fx), lerp1(s_s0[e01], s_s0[e11], p.fx), p.fy));
+            st_out<NTS>(&io.s1o[g], lerp1(lerp1(s_s1[e00], s_s1[e10], p.fx), lerp1(s_s1[e01], s_s1[e11], p.fx), p.fy));
         } else {
-            // taps outside the halo (rare): one copy of the recompute, looped
-            // over the taps (00, 10, 01, 11) with the same lerp order
-            float p0 = 0.0f, p1 = 0.0f, t0 = 0.0f, t1 = 0.0f, b0 = 0.0f, b1 = 0.0f;
-#pragma unroll 1
-            for (int tap = 0; tap < 4; ++tap) {
-                const int qx = (tap & 1) ? ix1 : ix, qy = (tap & 2) ? iy1 : iy;
-                float v0, v1;
-                eroded_sediment_global(io, qx, qy, nx, ny, step, terrain, rain != 0, k, v0, v1);
-                if ((tap & 1) == 0) {
-                    p0 = v0; p1 = v1;
-                } else if (tap == 1) {
-                    t0 = lerp1(p0, v0, fx); t1 = lerp1(p1, v1, fx);
-                } else {
-                    b0 = lerp1(p0, v0, fx); b1 = lerp1(p1, v1, fx);
-                }
-            }
-            o0 = lerp1(t0, b0, fy);
-            o1 = lerp1(t1, b1, fy);
+            s_far[atomicAdd(s_nfar, 1)] = t;
         }
-        const size_t g = at(gx, gy, nx);
-        st_out<NTS>(&io.s0o[g], o0);
-        st_out<NTS>(&io.s1o[g], o1);
+    }
+    __syncthreads();
+    const int nfar = 4 * __builtin_amdgcn_readfirstlane(*s_nfar);
+    if (nfar > 0) {
+        for (int j = tid; j < nfar; j += NT) {
+            const int t = s_far[j >> 2];
+            const Taps p = taps_of(t);
+            float v0, v1;
+            eroded_sediment_global(io, (j & 1) ? p.ix1 : p.ix, (j & 2) ? p.iy1 : p.iy, nx, ny, step, terrain,
+                                   rain != 0, k, v0, v1);
+            // taps 00, 10, 01, 11 of lanes 0 .. 3 of the group
+            auto tap = [](float v, auto c) {
+                return __int_as_float(
+                    __builtin_amdgcn_mov_dpp(__float_as_int(v), decltype(c)::value * 0x55, 0xf, 0xf, true));
+            };
+            auto mix = [&](float v) {
+                const float v00 = tap(v, std::integral_constant<int, 0>{}), v10 = tap(v, std::integral_constant<int, 1>{});
+                const float v01 = tap(v, std::integral_constant<int, 2>{}), v11 = tap(v, std::integral_constant<int, 3>{});
+                return lerp1(lerp1(v00, v10, p.fx), lerp1(v01, v11, p.fx), p.fy);
+            };
+            const float o0 = mix(v0), o1 = mix(v1);
+            if ((j & 3) == 0) {
+                const int ty = t / TX, tx = t - ty * TX;
+                const size_t g = at(x0 + tx, y0 + ty, nx);
+                st_out<NTS>(&io.s0o[g], o0);
+                st_out<NTS>(&io.s1o[g], o1);
+            }
+        }
+        if constexpr (STEP) __syncthreads();     // the list's place is the thermal stages' scale g
     }
 }
 
@@ -591,7 +627,8 @@ template <int TX, int TY>
 struct StepTile {
     using H = HydroTile<TX, TY, TH, 64>;
     static constexpr int THERMAL = 2 * H::NE + 2 * H::NTILE;     // rock, dirt, g of the thermal stages
-    static constexpr int NLDS = 6 * H::NLDS > THERMAL + 3 * H::NE ? 6 * H::NLDS : THERMAL + 3 * H::NE;
+    static constexpr int NLDS = 6 * H::NLDS;
+    static_assert(THERMAL + 3 * H::NE < NLDS, "the thermal stages and the far list's length fit the input arrays");
     static_assert(H::NE == ThermalTile<TX, TY>::N0, "both stages number the tile +- 5 cells alike");
 };
 
