@@ -1,6 +1,6 @@
 // hg_particle.hip — droplet (particle) erosion.
 //
-// A group of 8 lanes per droplet; the droplets of an iteration run concurrently
+// A group of 16 lanes per droplet; the droplets of an iteration run concurrently
 // and change the height planes with float atomic adds (global_atomic_add_f32),
 // so a droplet sees the others' changes in whatever order the memory system
 // applies them.  Height reads are relaxed atomic loads.  Erosion takes from a
@@ -24,7 +24,13 @@ namespace hgk {
 
 namespace {
 
-__device__ __forceinline__ void atomic_addf(float* p, float v) { unsafeAtomicAdd(p, v); }
+// The height planes are global memory, which the compiler no longer sees once a
+// pointer has been through an array or a select.
+using global_float = __attribute__((address_space(1))) float;
+__device__ __forceinline__ float fetch_addf(float* p, float v) {
+    return __builtin_amdgcn_global_atomic_fadd_f32((global_float*)p, v);
+}
+__device__ __forceinline__ void atomic_addf(float* p, float v) { (void)fetch_addf(p, v); }
 
 // Height reads are relaxed device-scope atomic loads: they are served by L2,
 // where the atomic adds land, and never by a stale line of the non-coherent
@@ -43,80 +49,105 @@ __device__ __forceinline__ int cell_of(float p, int n) { return min(int(p), n - 
 // All lanes of a group hold the same droplet (the same registers, bit for
 // bit, so they branch alike); what differs is which cell a lane touches: one
 // of the 8 heights of a 2x2 stencil (4 corners x 2 layers), one of the 4
-// corners of a deposit, one cell in kGroup of the erosion brush.  A brush row
-// or a stencil row is then one request of neighbouring lanes instead of one
-// per cell, and a brush costs one round trip per layer instead of one per cell.
+// corners of a deposit, one layer of one of 8 cells of a row of the erosion
+// brush.  What neighbouring lanes touch in one cache line is one request.
 //
-// With a thread per droplet a step was a chain of up to 2 x 25 dependent
-// returning atomics (radius 3), each a request of its own.  2048^2 with 2^20
-// droplets of 64 steps: 61.2 -> 23.6 ms per iteration; 512^2 with 20000 of 30
-// steps: 1.20 -> 0.41 ms.  What bounds it now: the atomics, 474 million
-// requests per iteration at 2048^2, all of which the L2s pass on to memory
-// (TCC_EA0_ATOMIC = TCC_ATOMIC), 20 per ns.  Running the droplets of one part
-// of the map together (sorted by 0.5 to 4 MB regions, with or without each XCD
-// keeping to its own) halves the lines fetched and is slower, 31 to 73 ms:
-// requests to the same lines then wait for each other.
-constexpr int kGroup = 8;
-constexpr int kBrushSlots = 32;                  // brush cells in flight together
-constexpr int kPerLane = kBrushSlots / kGroup;
-constexpr int kGotPitch = kBrushSlots + 4;       // 16-byte rows; the 8 groups of a wave start in different banks
-static_assert(kGroup == 8, "the lane exchanges of stencil_heights are written for 8 lanes");
+// Requests are what bounds it: the L2s pass every atomic on to memory, which
+// takes about 20 a ns (TCC_EA0_ATOMIC = TCC_ATOMIC = 474 million per iteration
+// of 2^20 droplets at 2048^2 when 8 lanes ran a droplet on the two planes).
+// So hg_step_particle runs on a map that holds rock and dirt of a cell next to
+// each other (HeightMap, PAIRED): a brush row is one request for both layers,
+// a stencil row too.  ms per iteration, 2^20 droplets of 64 steps at 2048^2 /
+// 20000 of 30 steps at 512^2 (with the thermal pass):
+//   a thread per droplet                            61.2 / 1.21
+//   8 lanes, planes                                 23.7 / 0.37
+//   16 lanes, paired                                20.5 / 0.25
+// (hg_droplets_noalloc has no room for pairs: 16 lanes, planes, 26.8.)  367
+// million atomic requests are left, a 40-byte row being 1.5 requests of 64
+// bytes on average, and the arithmetic, at 4 droplets per wave, half the time.
+// More in flight does not help: half the waves per CU run as fast, sending a
+// step's dirt and rock atomics and the next step's loads together, or loading
+// the brush beside the stencil, is slower (29 and 30 ms with planes).  Nor does
+// running the droplets of one part of the map together (sorted by 0.5 to 4 MB
+// regions, with or without each XCD keeping to its own): that halves the lines
+// fetched, but the requests to a line then wait for each other, 31 to 73 ms.
+constexpr int kGroup = 16;
+constexpr int kRowCells = kGroup / 2;            // cells of a brush row in flight together
+constexpr int kRows = 5;                         // brush rows in flight together (all of radius 3)
+constexpr int kGotPitch = kRows * kRowCells + 4; // 16-byte rows; the groups of a wave start in different banks
+constexpr int kSlots = 11 * 16;                  // brush rows padded to whole row chunks: radius 6 has 11 rows of 2
+static_assert(kGroup == 16, "the lane exchanges are written for the 16 lanes of a DPP row");
 
-template <int CTRL, int BANKS>
-__device__ __forceinline__ float dpp(float old, float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xf, BANKS, false));
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float other_layer(float v) { return dpp<0xb1>(v); }   // quad_perm 1, 0, 3, 2
+
+// The heights.  Planes: rock in a, dirt in b, row by row.  PAIRED: rows of
+// (rock, dirt) pairs, those below `half` in a and the others in b, so that two
+// separate planes of n x n floats hold them.
+template <bool PAIRED>
+struct HeightMap {
+    float *a, *b;
+    int n, half;
+    __device__ __forceinline__ float* at(int layer, int x, int y) const {
+        // 32-bit cell numbers: n <= 32768
+        if constexpr (PAIRED) {
+            const bool up = y >= half;
+            const uint32_t i = uint32_t(up ? y - half : y) * uint32_t(2 * n) + uint32_t(2 * x + layer);
+            return (up ? b : a) + size_t(i);
+        } else {
+            return (layer ? b : a) + size_t(uint32_t(y) * uint32_t(n) + uint32_t(x));
+        }
+    }
+};
+
+// Heights (rock + dirt) at the corners (0,0), (1,0), (0,1), (1,1) of cell (x,
+// y): lane g of the group loads layer g & 1 of corner (g >> 1) & 1 of row
+// (g >> 2) & 1, adds the other layer's value from the lane beside it, and every
+// lane takes the four sums, two from its own quad, two from the next.
+template <class Map>
+__device__ __forceinline__ void stencil_heights(const Map& m, int x, int y, int g, float& h00, float& h10, float& h01,
+                                                float& h11) {
+    const bool top = (g & 4) != 0;
+    const float v = ld(m.at(g & 1, x + ((g >> 1) & 1), y + (top ? 1 : 0)));
+    const float h = v + other_layer(v);
+    const float h0 = dpp<0x00>(h), h1 = dpp<0xaa>(h);            // quad_perm broadcasts of lanes 0 and 2
+    const float o0 = dpp<0x124>(h0), o1 = dpp<0x124>(h1);        // row_ror:4
+    h00 = top ? o0 : h0;
+    h10 = top ? o1 : h1;
+    h01 = top ? h0 : o0;
+    h11 = top ? h1 : o1;
 }
 
-// Heights (rock + dirt) at the corners (0,0), (1,0), (0,1), (1,1) of cell c:
-// lane g of the group loads corner g & 3 of layer g >> 2, adds the other
-// layer's value from the lane 4 away and every lane takes the four sums.
-__device__ __forceinline__ void stencil_heights(const float* R, const float* D, size_t c, int n, int g, float& h00,
-                                                float& h10, float& h01, float& h11) {
-    const float* layer = (g & 4) ? D : R;
-    const float v = ld(layer + (c + size_t(g & 1) + ((g & 2) ? size_t(n) : size_t(0))));
-    float o = dpp<0x104, 0x5>(v, v);             // row_shl:4 into lanes 0-3 and 8-11 of each 16
-    o = dpp<0x114, 0xa>(o, v);                   // row_shr:4 into lanes 4-7 and 12-15
-    const float h = v + o;
-    h00 = dpp<0x00, 0xf>(h, h);                  // quad_perm broadcasts
-    h10 = dpp<0x55, 0xf>(h, h);
-    h01 = dpp<0xaa, 0xf>(h, h);
-    h11 = dpp<0xff, 0xf>(h, h);
-}
-
-// Bilinear deposit of `amount` into dirt around (px, py): lane g < 4 of the
-// group adds corner g's share.
-__device__ __forceinline__ void deposit(float* D, int n, int g, float px, float py, float amount) {
-    const int x = cell_of(px, n), y = cell_of(py, n);
+// Bilinear deposit of `amount` into dirt around (px, py): the four dirt lanes
+// of a stencil add a corner's share each.
+template <class Map>
+__device__ __forceinline__ void deposit(const Map& m, int g, float px, float py, float amount) {
+    const int x = cell_of(px, m.n), y = cell_of(py, m.n);
     const float u = px - float(x), v = py - float(y);
-    const float share = amount * ((g & 1) ? u : 1.0f - u) * ((g & 2) ? v : 1.0f - v);
-    if (g < 4) atomic_addf(D + (size_t(y) * n + x + size_t(g & 1) + ((g & 2) ? size_t(n) : size_t(0))), share);
+    const bool right = (g & 2) != 0, top = (g & 4) != 0;
+    const float share = amount * (right ? u : 1.0f - u) * (top ? v : 1.0f - v);
+    if (g < 8 && (g & 1)) atomic_addf(m.at(1, x + (right ? 1 : 0), y + (top ? 1 : 0)), share);
 }
 
-// Taking material.  Removes up to want[i] from p[idx[i]] for a lane's cells,
-// never more than a cell holds, and returns in got[i] what was removed.  The
-// amount `seen`, a relaxed load's value, says is there is subtracted with a
+// Taking material.  Up to `want` is removed from a cell, never more than it
+// holds.  What a relaxed load says is there (`seen`) is subtracted with a
 // returning atomic add; if other droplets took from the cell in between, the
 // height it replaced is smaller, and the part that was not there is added
-// back.  Each take is then at most max(0, what the cell held at its atomic
-// add, less the give-backs still outstanding), so the takes of all droplets
-// from one cell never exceed what it held and it never ends below 0 in exact
-// arithmetic; in FP32 the subtraction and the give-back round, which can
-// leave a residue of a few ulp of the amounts involved below 0.  All of a
-// lane's atomics are issued before the first result is looked at.
-__device__ __forceinline__ void take(float* p, const size_t (&idx)[kPerLane], const float (&seen)[kPerLane],
-                                     const float (&want)[kPerLane], float (&got)[kPerLane]) {
-    float est[kPerLane], old[kPerLane];
-#pragma unroll
-    for (int i = 0; i < kPerLane; ++i) {
-        est[i] = fminf(fmaxf(seen[i], 0.0f), want[i]);
-        old[i] = 0.0f;
-        if (est[i] > 0.0f) old[i] = atomicAdd(p + idx[i], -est[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < kPerLane; ++i) {
-        got[i] = est[i] > 0.0f ? fminf(fmaxf(old[i], 0.0f), est[i]) : 0.0f;
-        if (got[i] < est[i]) atomic_addf(p + idx[i], est[i] - got[i]);
-    }
+// back (taken).  Each take is then at most max(0, what the cell held at its
+// atomic add, less the give-backs still outstanding), so the takes of all
+// droplets from one cell never exceed what it held and it never ends below 0
+// in exact arithmetic; in FP32 the subtraction and the give-back round, which
+// can leave a residue of a few ulp of the amounts involved below 0.
+__device__ __forceinline__ float estimate(float seen, float want) { return fminf(fmaxf(seen, 0.0f), want); }
+__device__ __forceinline__ float taken(float* p, float old, float est) {
+    // min(max(old, 0), est), spelt with two uses of `old`: with one, the compiler
+    // moves the max behind the atomic, where it waits for the result
+    const float got = est > 0.0f ? (!(old >= est) ? fmaxf(old, 0.0f) : est) : 0.0f;
+    if (got < est) atomic_addf(p, est - got);
+    return got;
 }
 
 // Start position of droplet `id` in an iteration: uniform over [0, n-1)^2.
@@ -144,29 +175,33 @@ constexpr uint32_t kChunk = 64 / kGroup;         // droplets of a wave
 // that number.  1 without an order; with one, neighbouring chunks of the order
 // lie side by side on the map and are kept apart in time: run next to each
 // other, their requests queue for the same lines (2048^2, 2^20 droplets sorted
-// by tile: 48.8 ms per iteration, spread 19.2 ms).
+// by tile, 8 lanes, planes: 48.8 ms per iteration, spread 19.2 ms).
 //
 // PARTIALS = false: the workgroup's exported mass and droplet steps are added
 // atomically to *exported_out and *steps_out.  PARTIALS = true: they are
 // written to partials[blockIdx.x], for k_droplet_totals to sum in a fixed
 // order.
-template <bool PARTIALS>
-__global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R, float* __restrict__ D, int n,
-                                                           DropletParams p, Brush brush, uint32_t iteration,
+template <bool PARTIALS, bool PAIRED>
+__global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map, DropletParams p, Brush brush, uint32_t iteration,
                                                            uint32_t rounds, uint32_t spread,
                                                            const uint32_t* __restrict__ order,
                                                            double* exported_out, unsigned long long* steps_out,
                                                            DropletPartial* partials) {
     __shared__ double s_exp[kDropletsPerBlock];
     __shared__ unsigned s_steps[kDropletsPerBlock];
-    __shared__ float s_w[HG_BRUSH_MAX];
-    __shared__ int s_dxy[HG_BRUSH_MAX];                            // dx in the low half, dy in the high half
+    __shared__ float s_w[kSlots];        // the brush's weights, its rows padded to whole chunks of kRowCells
     __shared__ __align__(16) float s_got[kDropletsPerBlock][kGotPitch];   // what a group's brush cells gave
     const int g = int(threadIdx.x) & (kGroup - 1), group = int(threadIdx.x) / kGroup;
-    if (threadIdx.x < HG_BRUSH_MAX) {
+    const int n = map.n;
+    const int reach = brush.r - 1, width = 2 * reach + 1;         // cells closer than r: rows and columns -reach .. reach
+    const int twice = width > kRowCells ? 1 : 0;                  // a row is one chunk, or two (radius 5 and 6)
+    const int row_slots = kRowCells << twice, chunks_of_rows = width << twice;
+    static_assert(2 * kRowCells >= 11, "radius 6: rows of 11 cells");
+    for (int t = int(threadIdx.x); t < kSlots; t += kDropThreads) s_w[t] = 0.0f;
+    __syncthreads();
+    if (int(threadIdx.x) < brush.count) {
         const int t = int(threadIdx.x);
-        s_w[t] = brush.w[t];
-        s_dxy[t] = (int(brush.dx[t]) & 0xffff) | (int(brush.dy[t]) << 16);
+        s_w[(brush.dy[t] + reach) * row_slots + brush.dx[t] + reach] = brush.w[t];
     }
     __syncthreads();
     double exported = 0.0;
@@ -179,7 +214,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
         if (w >= chunks) break;
         const uint32_t slot = uint32_t(uint64_t(w) * spread % chunks) * kChunk + uint32_t(group) % kChunk;
         if (slot >= p.count) continue;
-        if (end_sed != 0.0f) deposit(D, n, g, end_px, end_py, end_sed);   // the round before
+        if (end_sed != 0.0f) deposit(map, g, end_px, end_py, end_sed);   // the round before
         const uint32_t id = order ? order[slot] : slot;
         const float span = float(n - 1);
         float px, py;
@@ -191,7 +226,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
             const int cx = cell_of(px, n), cy = cell_of(py, n);
             const float u = px - float(cx), v = py - float(cy);
             float h00, h10, h01, h11;
-            stencil_heights(R, D, size_t(cy) * n + cx, n, g, h00, h10, h01, h11);
+            stencil_heights(map, cx, cy, g, h00, h10, h01, h11);
             const float gx = (h10 - h00) * (1.0f - v) + (h11 - h01) * v;
             const float gy = (h01 - h00) * (1.0f - u) + (h11 - h10) * u;
             const float h = h00 * (1.0f - u) * (1.0f - v) + h10 * u * (1.0f - v) + h01 * (1.0f - u) * v +
@@ -203,13 +238,14 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
             // and sqrtf lower to the IEEE sequences; HIP's __fsqrt_rn lowers to
             // the native 3-ulp sqrt.
             const float len = sqrtf(dx * dx + dy * dy);
-            if (len > 0.0f) {
-                dx = dx / len;
-                dy = dy / len;
+            if (len > 0.0f) {                     // one division: even lanes divide dx, odd lanes dy
+                const float q = ((g & 1) ? dy : dx) / len, beside = other_layer(q);
+                dx = (g & 1) ? beside : q;
+                dy = (g & 1) ? q : beside;
             }
             const float ox = px, oy = py;
             if (dx == 0.0f && dy == 0.0f) {       // not moving: drop the load here
-                deposit(D, n, g, px, py, sed);
+                deposit(map, g, px, py, sed);
                 sed = 0.0f;
                 alive = false;
                 break;
@@ -225,7 +261,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
             const int nx2 = cell_of(px, n), ny2 = cell_of(py, n);
             const float u2 = px - float(nx2), v2 = py - float(ny2);
             float k00, k10, k01, k11;
-            stencil_heights(R, D, size_t(ny2) * n + nx2, n, g, k00, k10, k01, k11);
+            stencil_heights(map, nx2, ny2, g, k00, k10, k01, k11);
             const float hn = k00 * (1.0f - u2) * (1.0f - v2) + k10 * u2 * (1.0f - v2) + k01 * (1.0f - u2) * v2 +
                              k11 * u2 * v2;
             const float dh = hn - h;
@@ -233,7 +269,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
             if (sed > cap || dh > 0.0f) {
                 const float amount = dh > 0.0f ? fminf(dh, sed) : (sed - cap) * p.deposition;
                 sed -= amount;
-                deposit(D, n, g, ox, oy, amount);
+                deposit(map, g, ox, oy, amount);
             } else {
                 const float amount = fminf((cap - sed) * p.erosion, -dh);
                 const bool interior = cx >= brush.r && cy >= brush.r && cx < n - brush.r && cy < n - brush.r;
@@ -246,43 +282,66 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
                     }
                 }
                 const float scale = interior ? amount : amount / wsum;
-                for (int base = 0; base < brush.count; base += kBrushSlots) {
-                    size_t idx[kPerLane];
-                    float want[kPerLane], seen_d[kPerLane], seen_r[kPerLane], td[kPerLane], tr[kPerLane];
+                for (int base = 0; base < chunks_of_rows; base += kRows) {
+                    // lane g: layer g & 1 of cell g >> 1 of each row chunk.  The
+                    // dirt goes first, the rock gives the rest, both sent
+                    // together as if all the dirt seen will be got.
+                    float *at[kRows], want[kRows], seen[kRows], est[kRows], dirt[kRows], old[kRows];
 #pragma unroll
-                    for (int i = 0; i < kPerLane; ++i) {
-                        const int t = base + i * kGroup + g;
-                        idx[i] = 0;
-                        want[i] = seen_d[i] = seen_r[i] = 0.0f;
-                        if (t < brush.count) {
-                            const int dxy = s_dxy[t];
-                            const int x = cx + int(int16_t(dxy & 0xffff)), y = cy + (dxy >> 16);
-                            if (interior || (x >= 0 && y >= 0 && x < n && y < n)) {
-                                idx[i] = size_t(y) * n + x;
-                                want[i] = scale * s_w[t];
-                                seen_d[i] = ld(D + idx[i]);
-                                seen_r[i] = ld(R + idx[i]);
+                    for (int i = 0; i < kRows; ++i) {
+                        at[i] = map.a;
+                        want[i] = seen[i] = 0.0f;
+                        if (base + i < chunks_of_rows) {
+                            const int row = (base + i) >> twice, column = ((base + i) & twice) * kRowCells;
+                            const int x = cx - reach + column + (g >> 1), y = cy - reach + row;
+                            const float w = s_w[(base + i) * kRowCells + (g >> 1)];
+                            if (w > 0.0f && (interior || (x >= 0 && y >= 0 && x < n && y < n))) {
+                                at[i] = map.at(g & 1, x, y);
+                                want[i] = scale * w;
+                                seen[i] = ld(at[i]);
                             }
                         }
                     }
-                    take(D, idx, seen_d, want, td);
 #pragma unroll
-                    for (int i = 0; i < kPerLane; ++i) want[i] = want[i] - td[i];
-                    take(R, idx, seen_r, want, tr);
-                    // sed += td + tr, cell by cell in the brush's order (cells
-                    // that gave nothing add 0): the group passes its cells'
-                    // amounts round through LDS.  One wave reads and writes a
-                    // group's row, and a wave's LDS accesses keep their order.
+                    for (int i = 0; i < kRows; ++i) {
+                        const float beside = other_layer(seen[i]);
+                        dirt[i] = estimate((g & 1) ? seen[i] : beside, want[i]);
+                        est[i] = (g & 1) ? dirt[i] : estimate(seen[i], want[i] - dirt[i]);
+                    }
 #pragma unroll
-                    for (int i = 0; i < kPerLane; ++i) s_got[group][i * kGroup + g] = td[i] + tr[i];
+                    for (int i = 0; i < kRows; ++i) {
+                        // any value where nothing is taken (taken() does not look
+                        // at it): a 0 would have to be merged with the atomic's
+                        // result, which waits for it before the next is sent
+                        old[i] = __builtin_nondeterministic_value(old[i]);
+                        if (est[i] > 0.0f) old[i] = fetch_addf(at[i], -est[i]);
+                    }
+                    // sed += dirt + rock, cell by cell in the brush's order
+                    // (slots that gave nothing add 0): the group passes its
+                    // cells' amounts round through LDS.  One wave reads and
+                    // writes a group's row, and a wave's LDS accesses keep their
+                    // order.
+#pragma unroll
+                    for (int i = 0; i < kRows; ++i) {
+                        const float mine = taken(at[i], old[i], est[i]);
+                        const float beside = other_layer(mine);
+                        if ((g & 1) == 0) {
+                            float rock = mine;
+                            if (beside < dirt[i]) {      // another droplet had the dirt: the rest from the rock after all
+                                const float more = estimate(ld(at[i]), dirt[i] - beside);
+                                if (more > 0.0f) rock += taken(at[i], fetch_addf(at[i], -more), more);
+                            }
+                            s_got[group][i * kRowCells + (g >> 1)] = beside + rock;
+                        }
+                    }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    const int m = (min(kBrushSlots, brush.count - base) + 3) / 4;
+                    const int m = min(kRows, chunks_of_rows - base) * (kRowCells / 4);
                     for (int q = 0; q < m; ++q) {
-                        const float4 a = *reinterpret_cast<const float4*>(&s_got[group][4 * q]);
-                        sed += a.x;
-                        sed += a.y;
-                        sed += a.z;
-                        sed += a.w;
+                        const float4 v4 = *reinterpret_cast<const float4*>(&s_got[group][4 * q]);
+                        sed += v4.x;
+                        sed += v4.y;
+                        sed += v4.z;
+                        sed += v4.w;
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 }
@@ -295,7 +354,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
         end_sed = alive ? sed : 0.0f;
     }
     __syncthreads();
-    if (end_sed != 0.0f) deposit(D, n, g, end_px, end_py, end_sed);
+    if (end_sed != 0.0f) deposit(map, g, end_px, end_py, end_sed);
     if (g == 0) {
         s_exp[group] = exported;
         s_steps[group] = steps;
@@ -317,6 +376,30 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(float* __restrict__ R
             atomicAdd(steps_out, (unsigned long long)s_steps[0]);
         }
     }
+}
+
+// Rock and dirt planes to rows of pairs and back: n * n cells, the first half
+// of the rows in `low`, the other in `high`, 4 cells per thread, `quads` per
+// half (n is a multiple of 8).
+__global__ __launch_bounds__(256) void k_pair_heights(const float* __restrict__ rock, const float* __restrict__ dirt,
+                                                      float* __restrict__ low, float* __restrict__ high,
+                                                      size_t quads) {
+    const size_t q = size_t(blockIdx.x) * 256 + threadIdx.x;
+    if (q >= 2 * quads) return;
+    const float4 r = reinterpret_cast<const float4*>(rock)[q], d = reinterpret_cast<const float4*>(dirt)[q];
+    float4* out = reinterpret_cast<float4*>(q < quads ? low : high) + 2 * (q < quads ? q : q - quads);
+    out[0] = make_float4(r.x, d.x, r.y, d.y);
+    out[1] = make_float4(r.z, d.z, r.w, d.w);
+}
+__global__ __launch_bounds__(256) void k_unpair_heights(const float* __restrict__ low, const float* __restrict__ high,
+                                                        float* __restrict__ rock, float* __restrict__ dirt,
+                                                        size_t quads) {
+    const size_t q = size_t(blockIdx.x) * 256 + threadIdx.x;
+    if (q >= 2 * quads) return;
+    const float4* in = reinterpret_cast<const float4*>(q < quads ? low : high) + 2 * (q < quads ? q : q - quads);
+    const float4 a = in[0], b = in[1];
+    reinterpret_cast<float4*>(rock)[q] = make_float4(a.x, a.z, b.x, b.z);
+    reinterpret_cast<float4*>(dirt)[q] = make_float4(a.y, a.w, b.y, b.w);
 }
 
 // ---- droplet ordering (counting sort by start tile) --------------------------
@@ -434,13 +517,27 @@ static uint32_t chunk_spread(uint32_t count) {
     return k;
 }
 
-hipError_t launch_droplets(float* rock, float* dirt, int n, const DropletParams& p, const Brush& brush,
+hipError_t launch_droplets(float* pairs_low, float* pairs_high, int n, const DropletParams& p, const Brush& brush,
                            uint32_t iteration, const uint32_t* order, double* exported,
                            unsigned long long* steps, hipStream_t s) {
     if (p.count == 0) return hipSuccess;
     const uint32_t blocks = (p.count + kDropletsPerBlock - 1) / kDropletsPerBlock;
-    k_droplets<false><<<blocks, kDropThreads, 0, s>>>(rock, dirt, n, p, brush, iteration, 1,
-                                                      order ? chunk_spread(p.count) : 1u, order, exported, steps, nullptr);
+    const HeightMap<true> map{pairs_low, pairs_high, n, n / 2};
+    k_droplets<false, true><<<blocks, kDropThreads, 0, s>>>(map, p, brush, iteration, 1,
+                                                            order ? chunk_spread(p.count) : 1u, order, exported, steps,
+                                                            nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_heights(const float* rock, const float* dirt, float* low, float* high, int n, hipStream_t s) {
+    const size_t quads = size_t(n) * size_t(n) / 8;          // 4 cells each, per half
+    k_pair_heights<<<unsigned((2 * quads + 255) / 256), 256, 0, s>>>(rock, dirt, low, high, quads);
+    return hipGetLastError();
+}
+
+hipError_t launch_unpair_heights(const float* low, const float* high, float* rock, float* dirt, int n, hipStream_t s) {
+    const size_t quads = size_t(n) * size_t(n) / 8;
+    k_unpair_heights<<<unsigned((2 * quads + 255) / 256), 256, 0, s>>>(low, high, rock, dirt, quads);
     return hipGetLastError();
 }
 
@@ -478,8 +575,9 @@ uint32_t droplet_partial_blocks(uint32_t count) {
 hipError_t launch_droplets_partials(float* rock, float* dirt, int n, const DropletParams& p, const Brush& brush,
                                     uint32_t iteration, DropletPartial* partials, hipStream_t s) {
     if (p.count == 0) return hipSuccess;
-    k_droplets<true><<<droplet_partial_blocks(p.count), kDropThreads, 0, s>>>(
-        rock, dirt, n, p, brush, iteration, partial_rounds(p.count), 1u, nullptr, nullptr, nullptr, partials);
+    const HeightMap<false> map{rock, dirt, n, 0};
+    k_droplets<true, false><<<droplet_partial_blocks(p.count), kDropThreads, 0, s>>>(
+        map, p, brush, iteration, partial_rounds(p.count), 1u, nullptr, nullptr, nullptr, partials);
     return hipGetLastError();
 }
 

@@ -578,9 +578,20 @@ int hg_step_particle(hg_ctx* c, uint32_t iterations, uint32_t flags) {
         }
         tiles = c->drop_order + p.count;
     }
+    // The droplets run on (rock, dirt) pairs, kept in the alternate buffers of
+    // the two planes (every pass that reads those writes them first).
+    bool paired = false;
     for (uint32_t it = 0; it < iterations; ++it) {
         const uint32_t iter = c->particle_iter;
         int rc = HG_OK;
+        if (!paired && p.count > 0) {
+            rc = timed_launch(c, "pair_heights", [&] {
+                return hgk::launch_pair_heights(c->cur[HG_P_ROCK], c->cur[HG_P_DIRT], c->alt[HG_P_ROCK],
+                                                c->alt[HG_P_DIRT], c->n, c->stream);
+            });
+            if (rc != HG_OK) return rc;
+            paired = true;
+        }
         if (ordered) {
             rc = timed_launch(c, "droplet_order", [&] {
                 return hgk::launch_droplet_order(c->n, p, iter, tiles, c->drop_order, c->stream);
@@ -588,11 +599,19 @@ int hg_step_particle(hg_ctx* c, uint32_t iterations, uint32_t flags) {
             if (rc != HG_OK) return rc;
         }
         rc = timed_launch(c, "droplets", [&] {
-            return hgk::launch_droplets(c->cur[HG_P_ROCK], c->cur[HG_P_DIRT], c->n, p, brush, iter,
+            return hgk::launch_droplets(c->alt[HG_P_ROCK], c->alt[HG_P_DIRT], c->n, p, brush, iter,
                                         ordered ? c->drop_order : nullptr, c->dev_exported, c->dev_dsteps,
                                         c->stream);
         });
         if (rc != HG_OK) return rc;
+        if (paired && (thermal || smooth || it + 1 == iterations)) {
+            rc = timed_launch(c, "unpair_heights", [&] {
+                return hgk::launch_unpair_heights(c->alt[HG_P_ROCK], c->alt[HG_P_DIRT], c->cur[HG_P_ROCK],
+                                                  c->cur[HG_P_DIRT], c->n, c->stream);
+            });
+            if (rc != HG_OK) return rc;
+            paired = false;
+        }
         if (thermal || smooth) {
             hgk::ThermIO tio;
             tio.r = c->cur[HG_P_ROCK]; tio.d = c->cur[HG_P_DIRT];

@@ -316,16 +316,16 @@ int hg_step_particle(hg_ctx* ctx, uint32_t iterations, uint32_t flags);
 /* Which lanes run which droplet of an iteration (the droplets and their
  * start positions are the same in both modes; only the timing of their
  * atomic updates relative to each other changes):
- *   0  (default) droplets in the order of their numbers, so the 8 droplets
+ *   0  (default) droplets in the order of their numbers, so the 4 droplets
  *      of a wave start at unrelated places;
  *   1  droplets sorted by the tile of their start cell (16 x 16 cells, or
  *      n/128 for n > 2048), so a wave's droplets start close together and
- *      share cache lines: measured 1.07x faster at 2048^2 with 2^20
+ *      share cache lines: measured 1.02x faster at 2048^2 with 2^20
  *      droplets, but neighbouring droplets then run in lockstep and do not
  *      see each other's changes within a step, which moves the statistics
  *      further from the serial model (the spread of heights after 4
- *      iterations of 8192 droplets on 256^2: 3.0 % off the serial oracle,
- *      against 0.2-0.3 % in mode 0).
+ *      iterations of 8192 droplets on 256^2: 2.8 % off the serial oracle,
+ *      against 0.01-1.0 % in mode 0).
  * Mode 1 keeps count + (number of tiles, at most 16384) words of device
  * memory in the context.  No counterpart in the reference. */
 int hg_set_droplet_order(hg_ctx* ctx, int mode);
