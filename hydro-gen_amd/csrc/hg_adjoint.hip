@@ -130,11 +130,17 @@ __device__ void reduce_coef(double* gpart, int slot, double a, double b, double 
 // of a thread's cells before any is evaluated.  Loads use clamped addresses;
 // values off the grid are replaced by the pass's fill after the load.
 // ---------------------------------------------------------------------------
-constexpr int GTX = 64, GTY = 8, GNT = 256;   // 64 x 16 / 512 threads measured slower at 1024^2
+// Tile of 64 x 8 cells, by 256 threads (two cells each and the ring) on large
+// maps and 512 (one cell and the ring) on small ones, where no workgroup waits
+// for a place and a step is the length of one thread's chain: see wide_gather.
+// 64 x 16 with 512 threads is slower at 1024^2; 32 x 8, 32 x 16, 32 x 4 and
+// 16 x 8 with a thread per cell gain nothing over 64 x 8 at 256^2 and above.
+constexpr int GTX = 64, GTY = 8;
 constexpr int GRW = GTX + 2, GRH = GTY + 2, GNR = GRW * GRH;
-constexpr int GIT = (GNR + GNT - 1) / GNT;          // ring/tile cells per thread
 constexpr int SRW = GTX + 4, SRH = GTY + 4, SRN = SRW * SRH;
-constexpr int SIT = (SRN + GNT - 1) / GNT;          // staged cells per thread
+constexpr int per_thread(int cells, int nt) { return (cells + nt - 1) / nt; }
+template <int NT> constexpr int GIT = per_thread(GNR, NT);         // ring/tile cells per thread
+template <int NT> constexpr int SIT = per_thread(SRN, NT);         // staged cells per thread
 
 // Staged-region index of ring cell e.
 __device__ __forceinline__ int sidx(int e) {
@@ -145,13 +151,13 @@ __device__ __forceinline__ int sidx(int e) {
 // fn(it, s, i, in, gx, gy) for the cells of the tile + H region: s its index
 // in a (GTX + 2H) x (GTY + 2H) array, i the (clamped) global index.  Threads
 // past the end redo the last cell.
-template <int H, class F>
+template <int NT, int H, class F>
 __device__ __forceinline__ void region_walk(const TileId& T, int nx, int ny, F&& fn) {
-    constexpr int W = GTX + 2 * H, N = W * (GTY + 2 * H), IT = (N + GNT - 1) / GNT;
+    constexpr int W = GTX + 2 * H, N = W * (GTY + 2 * H), IT = per_thread(N, NT);
     const int x0 = T.x * GTX - H, y0 = T.y * GTY - H;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int s = min(int(threadIdx.x) + it * GNT, N - 1);
+        const int s = min(int(threadIdx.x) + it * NT, N - 1);
         const int sy = s / W, sx = s - sy * W;
         const int gx = x0 + sx, gy = y0 + sy;
         const bool in = gx >= 0 && gy >= 0 && gx < nx && gy < ny;
@@ -162,21 +168,21 @@ __device__ __forceinline__ void region_walk(const TileId& T, int nx, int ny, F&&
 // fn(it, s, i, in) for the cells of the tile + 2-cell region: s its index in
 // the staged (SRW x SRH) arrays, i the (clamped) global index, in whether it is
 // on the grid.
-template <class F>
+template <int NT, class F>
 __device__ __forceinline__ void stage_walk(const TileId& T, int nx, int ny, F&& fn) {
-    static_assert((SRN + GNT - 1) / GNT == SIT, "one iteration per staged cell of a thread");
-    region_walk<2>(T, nx, ny, [&](int it, int s, size_t i, bool in, int, int) { fn(it, s, i, in); });
+    region_walk<NT, 2>(T, nx, ny, [&](int it, int s, size_t i, bool in, int, int) { fn(it, s, i, in); });
 }
 
-// A thread's cells of the tile + ring, numbered j = threadIdx.x + it * GNT:
+// A thread's cells of the tile + ring, numbered j = threadIdx.x + it * NT:
 // the GTX * GTY tile cells first, row by row (whole waves, GTIT iterations),
 // then the ring (bottom row, top row, then the left and right columns).
-constexpr int GTIT = GTX * GTY / GNT;
-static_assert(GTX * GTY % GNT == 0, "the tile fills whole iterations");
-static_assert(GIT == GTIT + 1 && GNR - GTX * GTY <= GNT, "the ring fits one iteration");
+template <int NT> constexpr int GTIT = GTX * GTY / NT;
+template <int NT>
 __device__ __forceinline__ void ring_cell(int it, int& ex, int& ey) {
-    const int j = int(threadIdx.x) + it * GNT;
-    if (it < GTIT) {
+    static_assert(GTX * GTY % NT == 0, "the tile fills whole iterations");
+    static_assert(GIT<NT> == GTIT<NT> + 1 && GNR - GTX * GTY <= NT, "the ring fits one iteration");
+    const int j = int(threadIdx.x) + it * NT;
+    if (it < GTIT<NT>) {
         ey = j / GTX + 1;
         ex = j - (ey - 1) * GTX + 1;
     } else {
@@ -198,32 +204,32 @@ __device__ __forceinline__ void ring_cell(int it, int& ex, int& ey) {
 // with the same (thread, it) as phase 1, so what a cell computes for itself
 // can stay in registers indexed by `it` (it < GTIT); only what it sends to
 // its neighbours goes through LDS.
-template <class Pre, class Cell, class Gather>
+template <int NT, class Pre, class Cell, class Gather>
 __device__ __forceinline__ void tile_gather(const TileId& T, int nx, int ny, Pre&& pre, Cell&& cell,
                                             Gather&& gather) {
     const int x0 = T.x * GTX, y0 = T.y * GTY;
 #pragma unroll
-    for (int it = 0; it < GIT; ++it) {
+    for (int it = 0; it < GIT<NT>; ++it) {
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         const int gx = x0 - 1 + ex, gy = y0 - 1 + ey;
         pre(it, ey * GRW + ex, at(min(max(gx, 0), nx - 1), min(max(gy, 0), ny - 1), nx));
     }
     __syncthreads();   // staged LDS regions are complete
 #pragma unroll
-    for (int it = 0; it < GIT; ++it) {
-        if (it == GTIT && int(threadIdx.x) >= GNR - GTX * GTY) break;   // past the end of the ring
+    for (int it = 0; it < GIT<NT>; ++it) {
+        if (it == GTIT<NT> && int(threadIdx.x) >= GNR - GTX * GTY) break;   // past the end of the ring
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         const int gx = x0 - 1 + ex, gy = y0 - 1 + ey;
         const bool in = gx >= 0 && gy >= 0 && gx < nx && gy < ny;
-        cell(it, ey * GRW + ex, gx, gy, in, it < GTIT);
+        cell(it, ey * GRW + ex, gx, gy, in, it < GTIT<NT>);
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < GTIT; ++it) {
+    for (int it = 0; it < GTIT<NT>; ++it) {
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         const int gx = x0 - 1 + ex, gy = y0 - 1 + ey;
         if (gx < nx && gy < ny) gather(it, ey * GRW + ex, gx, gy);
     }
@@ -233,40 +239,40 @@ __device__ __forceinline__ void tile_gather(const TileId& T, int nx, int ny, Pre
 // e, px, py, in, tile) keeps what a cell sends in registers; after a barrier
 // (every read of the staged regions done) send(it, e) writes it to LDS, and
 // after another the gather runs.
-template <class Pre, class Cell, class Send, class Gather>
+template <int NT, class Pre, class Cell, class Send, class Gather>
 __device__ __forceinline__ void tile_gather_late(const TileId& T, int nx, int ny, Pre&& pre, Cell&& cell,
                                                  Send&& send, Gather&& gather) {
     const int x0 = T.x * GTX, y0 = T.y * GTY;
 #pragma unroll
-    for (int it = 0; it < GIT; ++it) {
+    for (int it = 0; it < GIT<NT>; ++it) {
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         const int gx = x0 - 1 + ex, gy = y0 - 1 + ey;
         pre(it, ey * GRW + ex, at(min(max(gx, 0), nx - 1), min(max(gy, 0), ny - 1), nx));
     }
     __syncthreads();   // staged LDS regions are complete
 #pragma unroll
-    for (int it = 0; it < GIT; ++it) {
-        if (it == GTIT && int(threadIdx.x) >= GNR - GTX * GTY) break;   // past the end of the ring
+    for (int it = 0; it < GIT<NT>; ++it) {
+        if (it == GTIT<NT> && int(threadIdx.x) >= GNR - GTX * GTY) break;   // past the end of the ring
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         const int gx = x0 - 1 + ex, gy = y0 - 1 + ey;
         const bool in = gx >= 0 && gy >= 0 && gx < nx && gy < ny;
-        cell(it, ey * GRW + ex, gx, gy, in, it < GTIT);
+        cell(it, ey * GRW + ex, gx, gy, in, it < GTIT<NT>);
     }
     __syncthreads();   // the staged regions are no longer read
 #pragma unroll
-    for (int it = 0; it < GIT; ++it) {
-        if (it == GTIT && int(threadIdx.x) >= GNR - GTX * GTY) break;
+    for (int it = 0; it < GIT<NT>; ++it) {
+        if (it == GTIT<NT> && int(threadIdx.x) >= GNR - GTX * GTY) break;
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         send(it, ey * GRW + ex);
     }
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < GTIT; ++it) {
+    for (int it = 0; it < GTIT<NT>; ++it) {
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         const int gx = x0 - 1 + ex, gy = y0 - 1 + ey;
         if (gx < nx && gy < ny) gather(it, ey * GRW + ex, gx, gy);
     }
@@ -333,32 +339,33 @@ __device__ __forceinline__ void flux_vjp(float f[4], float b, float w, const flo
 // x: flux inputs (rock, dirt, water after rain, old flux); lo: adjoint of the
 // flux outputs (water, flux, velocity).  Writes li's water and flux (fresh)
 // and adds the total-height adjoint to li's rock and dirt.
-__global__ __launch_bounds__(GNT) void k_adj_flux(Planes x, Planes lo, Planes li, int nx, int ny, KParams k) {
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_flux(Planes x, Planes lo, Planes li, int nx, int ny, KParams k) {
     const TileId T = block_tile();
     // sent to neighbours, per ring/tile cell: inflow adj (4), total-height adj (4);
     // kept per thread: outflow adj (4), own total-height adj, water adj
     __shared__ float s_fin[4][GNR], s_wn[4][GNR];
-    float o_fo[GTIT][4], o_wp[GTIT], o_d1[GTIT];
+    float o_fo[GTIT<NT>][4], o_wp[GTIT<NT>], o_d1[GTIT<NT>];
     __shared__ float t_w[SRN], t_fl[SRN], t_fr[SRN], t_ft[SRN], t_fb[SRN];
     const float* R = x.p[HG_P_ROCK];
     const float* D = x.p[HG_P_DIRT];
     const float* B = x.p[HG_P_WATER];
     {
         // total height (out of grid: HG_OOB_HEIGHT) and old flux (0) of the region
-        float w[SIT], fl[SIT], fr[SIT], ft[SIT], fb[SIT];
-        stage_walk(T, nx, ny, [&](int it, int, size_t i, bool in) {
+        float w[SIT<NT>], fl[SIT<NT>], fr[SIT<NT>], ft[SIT<NT>], fb[SIT<NT>];
+        stage_walk<NT>(T, nx, ny, [&](int it, int, size_t i, bool in) {
             const float t = (R[i] + D[i]) + B[i];
             const float a = x.p[HG_P_FLUX_L][i], b = x.p[HG_P_FLUX_R][i], c = x.p[HG_P_FLUX_T][i],
                         d = x.p[HG_P_FLUX_B][i];
             w[it] = in ? t : HG_OOB_HEIGHT;
             fl[it] = in ? a : 0.0f; fr[it] = in ? b : 0.0f; ft[it] = in ? c : 0.0f; fb[it] = in ? d : 0.0f;
         });
-        stage_walk(T, nx, ny, [&](int it, int s, size_t, bool) {
+        stage_walk<NT>(T, nx, ny, [&](int it, int s, size_t, bool) {
             t_w[s] = w[it]; t_fl[s] = fl[it]; t_fr[s] = fr[it]; t_ft[s] = ft[it]; t_fb[s] = fb[it];
         });
     }
-    float pb[GIT], plf[GIT][4], pld2[GIT], plv[GIT][3];
-    tile_gather(T, nx, ny,
+    float pb[GIT<NT>], plf[GIT<NT>][4], pld2[GIT<NT>], plv[GIT<NT>][3];
+    tile_gather<NT>(T, nx, ny,
         [&](int it, int, size_t i) {
             pb[it] = B[i];
             plf[it][0] = lo.p[HG_P_FLUX_L][i]; plf[it][1] = lo.p[HG_P_FLUX_R][i];
@@ -382,7 +389,7 @@ __global__ __launch_bounds__(GNT) void k_adj_flux(Planes x, Planes lo, Planes li
                 s_fin[j][e] = lfin[j];
                 s_wn[j][e] = lwn[j];
             }
-            if (it < GTIT) {                                  // a tile cell keeps its own part
+            if (it < GTIT<NT>) {                                  // a tile cell keeps its own part
                 for (int j = 0; j < 4; ++j) o_fo[it][j] = lfo[j];
                 o_wp[it] = lwp;
                 o_d1[it] = ld1;
@@ -492,30 +499,33 @@ __device__ __forceinline__ ErosionVjp erosion_vjp(float r_in, float d_in, float 
 }
 
 // Writes li's rock, dirt and sediment (fresh) and adds to li's velocity.
-__global__ __launch_bounds__(GNT) void k_adj_erosion(Planes x, Planes lo, Planes li, int nx, int ny, KParams k,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_erosion(Planes x, Planes lo, Planes li, int nx, int ny, KParams k,
                                                      double* gpart) {
     const TileId T = block_tile();
     // sent to neighbours: the slope adjoints; kept per thread: the cell's own
     // rock, dirt, sediment and velocity adjoints
     __shared__ float s_dx[GNR], s_dz[GNR];
     __shared__ float t_r[SRN], t_d[SRN];
-    float o_r[GTIT], o_d[GTIT], o_s0[GTIT], o_s1[GTIT], o_vx[GTIT], o_vy[GTIT], o_vz[GTIT];
+    constexpr int CT = GTIT<NT>;                          // tile cells per thread
+    float o_r[CT], o_d[CT], o_s0[CT], o_s1[CT], o_vx[CT], o_vy[CT], o_vz[CT];
     const float* R = x.p[HG_P_ROCK];
     const float* D = x.p[HG_P_DIRT];
     {
         // rock and dirt of the region (0 out of the grid)
-        float a[SIT], b[SIT];
-        stage_walk(T, nx, ny, [&](int it, int, size_t i, bool in) {
+        float a[SIT<NT>], b[SIT<NT>];
+        stage_walk<NT>(T, nx, ny, [&](int it, int, size_t i, bool in) {
             const float r = R[i], d = D[i];
             a[it] = in ? r : 0.0f;
             b[it] = in ? d : 0.0f;
         });
-        stage_walk(T, nx, ny, [&](int it, int s, size_t, bool) { t_r[s] = a[it]; t_d[s] = b[it]; });
+        stage_walk<NT>(T, nx, ny, [&](int it, int s, size_t, bool) { t_r[s] = a[it]; t_d[s] = b[it]; });
     }
     auto rd = [&](int sc) -> float { return t_r[sc] + t_d[sc]; };
-    float p0[GIT], p1[GIT], pvx[GIT], pvy[GIT], pvz[GIT], plr[GIT], pld[GIT], pl0[GIT], pl1[GIT];
+    constexpr int C = GIT<NT>;                            // tile and ring cells per thread
+    float p0[C], p1[C], pvx[C], pvy[C], pvz[C], plr[C], pld[C], pl0[C], pl1[C];
     double gKc = 0, gKs = 0, gKd = 0;
-    tile_gather(T, nx, ny,
+    tile_gather<NT>(T, nx, ny,
         [&](int it, int, size_t i) {
             p0[it] = x.p[HG_P_SED_ROCK][i]; p1[it] = x.p[HG_P_SED_DIRT][i];
             pvx[it] = x.p[HG_P_VEL_U][i]; pvy[it] = x.p[HG_P_VEL_V][i]; pvz[it] = x.p[HG_P_VEL_DEPTH][i];
@@ -534,7 +544,7 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion(Planes x, Planes lo, Planes
             }
             s_dx[e] = ev.ldx;
             s_dz[e] = ev.ldz;
-            if (it < GTIT) {                                  // a tile cell keeps its own part
+            if (it < GTIT<NT>) {                                  // a tile cell keeps its own part
                 o_r[it] = ev.lr;
                 o_d[it] = ev.ld;
                 o_s0[it] = ev.ls0;
@@ -555,7 +565,7 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion(Planes x, Planes lo, Planes
             li.p[HG_P_VEL_V][i] += o_vy[it];
             li.p[HG_P_VEL_DEPTH][i] += o_vz[it];
         });
-    reduce_coef<GNT>(gpart, T.slot, gKc, gKs, gKd, 0.0);
+    reduce_coef<NT>(gpart, T.slot, gKc, gKs, gKd, 0.0);
 }
 
 // ---- hydro_erosion and hydro_flux in one launch ----------------------------
@@ -568,7 +578,8 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion(Planes x, Planes lo, Planes
 // and velocity of the step; lo: the adjoints after erosion.  Writes li's rock,
 // dirt, sediment, water and flux (fresh).  The velocity adjoint ends here: it
 // is not written, and the transport VJP of the step before writes it anew.
-__global__ __launch_bounds__(GNT) void k_adj_erosion_flux(Planes x, Planes lo, Planes li, int nx, int ny,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_erosion_flux(Planes x, Planes lo, Planes li, int nx, int ny,
                                                           KParams k, double* gpart) {
     const TileId T = block_tile();
     // One LDS array (26.4 KB), first for the inputs staged on the tile + 2-cell
@@ -589,14 +600,15 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion_flux(Planes x, Planes lo, P
     float* s_dz = u + GNR;
     float (*s_fin)[GNR] = reinterpret_cast<float (*)[GNR]>(u + 2 * GNR);
     float (*s_wn)[GNR] = reinterpret_cast<float (*)[GNR]>(u + 6 * GNR);
-    float o_r[GTIT], o_d[GTIT], o_s0[GTIT], o_s1[GTIT], o_fo[GTIT][4], o_wp[GTIT], o_d1[GTIT];
-    float snd[GIT][10];                          // what each of a thread's cells sends
+    constexpr int CT = GTIT<NT>;                          // tile cells per thread
+    float o_r[CT], o_d[CT], o_s0[CT], o_s1[CT], o_fo[CT][4], o_wp[CT], o_d1[CT];
+    float snd[GIT<NT>][10];                          // what each of a thread's cells sends
     const float* R = x.p[HG_P_ROCK];
     const float* D = x.p[HG_P_DIRT];
     const float* B = x.p[HG_P_WATER];
     {
-        float a[SIT], b[SIT], w[SIT], fl[SIT], fr[SIT], ft[SIT], fb[SIT];
-        stage_walk(T, nx, ny, [&](int it, int, size_t i, bool in) {
+        float a[SIT<NT>], b[SIT<NT>], w[SIT<NT>], fl[SIT<NT>], fr[SIT<NT>], ft[SIT<NT>], fb[SIT<NT>];
+        stage_walk<NT>(T, nx, ny, [&](int it, int, size_t i, bool in) {
             const float r = R[i], d = D[i];
             const float t = (r + d) + B[i];
             const float f0 = x.p[HG_P_FLUX_L][i], f1 = x.p[HG_P_FLUX_R][i], f2 = x.p[HG_P_FLUX_T][i],
@@ -606,16 +618,17 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion_flux(Planes x, Planes lo, P
             w[it] = in ? t : HG_OOB_HEIGHT;
             fl[it] = in ? f0 : 0.0f; fr[it] = in ? f1 : 0.0f; ft[it] = in ? f2 : 0.0f; fb[it] = in ? f3 : 0.0f;
         });
-        stage_walk(T, nx, ny, [&](int it, int s, size_t, bool) {
+        stage_walk<NT>(T, nx, ny, [&](int it, int s, size_t, bool) {
             t_r[s] = a[it]; t_d[s] = b[it]; t_w[s] = w[it];
             t_fl[s] = fl[it]; t_fr[s] = fr[it]; t_ft[s] = ft[it]; t_fb[s] = fb[it];
         });
     }
     auto rd = [&](int sc) -> float { return t_r[sc] + t_d[sc]; };
-    float p0[GIT], p1[GIT], pvx[GIT], pvy[GIT], pvz[GIT], plr[GIT], pld[GIT], pl0[GIT], pl1[GIT];
-    float pb[GIT], plf[GIT][4], pld2[GIT], plv[GIT][3];
+    constexpr int C = GIT<NT>;                            // tile and ring cells per thread
+    float p0[C], p1[C], pvx[C], pvy[C], pvz[C], plr[C], pld[C], pl0[C], pl1[C];
+    float pb[C], plf[C][4], pld2[C], plv[C][3];
     double gKc = 0, gKs = 0, gKd = 0;
-    tile_gather_late(T, nx, ny,
+    tile_gather_late<NT>(T, nx, ny,
         [&](int it, int, size_t i) {
             p0[it] = x.p[HG_P_SED_ROCK][i]; p1[it] = x.p[HG_P_SED_DIRT][i];
             pvx[it] = x.p[HG_P_VEL_U][i]; pvy[it] = x.p[HG_P_VEL_V][i]; pvz[it] = x.p[HG_P_VEL_DEPTH][i];
@@ -653,7 +666,7 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion_flux(Planes x, Planes lo, P
                 snd[it][2 + j] = lfin[j];
                 snd[it][6 + j] = lwn[j];
             }
-            if (it < GTIT) {                                  // a tile cell keeps its own part
+            if (it < GTIT<NT>) {                                  // a tile cell keeps its own part
                 o_r[it] = ev.lr;
                 o_d[it] = ev.ld;
                 o_s0[it] = ev.ls0;
@@ -687,7 +700,7 @@ __global__ __launch_bounds__(GNT) void k_adj_erosion_flux(Planes x, Planes lo, P
             li.p[HG_P_ROCK][i] = lr + lw;
             li.p[HG_P_DIRT][i] = ld + lw;
         });
-    reduce_coef<GNT>(gpart, T.slot, gKc, gKs, gKd, 0.0);
+    reduce_coef<NT>(gpart, T.slot, gKc, gKs, gKd, 0.0);
 }
 
 // ---- sediment_transport --------------------------------------------------
@@ -717,6 +730,7 @@ constexpr int TRANSPORT_LDS = 6 * GNR + (GNR + 3) / 4;
 
 // The transport VJP's near gather on tile T, with `lds` (TRANSPORT_LDS
 // floats) as its LDS.
+template <int NT>
 __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, Planes x, Planes lo, Planes li,
                                                    int nx, int ny, const KParams& k, double* gpart) {
     // per tile/ring cell q: its 4 bilinear weights, its taps as offsets from
@@ -730,16 +744,16 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
     const float* VX = x.p[HG_P_VEL_U];
     const float* VY = x.p[HG_P_VEL_V];
     double gKe = 0;
-    float pvx[GIT], pvy[GIT], pl0[GIT], pl1[GIT];
+    float pvx[GIT<NT>], pvy[GIT<NT>], pl0[GIT<NT>], pl1[GIT<NT>];
     // a tile cell's own water and its adjoint, and the sediment at its own
     // back-trace taps (both layers: s00, s10, s01, s11), loaded before the
     // gather phase needs them
-    float plb[GTIT], pb[GTIT], ps[GTIT][8];
-    tile_gather(T, nx, ny,
+    float plb[GTIT<NT>], pb[GTIT<NT>], ps[GTIT<NT>][8];
+    tile_gather<NT>(T, nx, ny,
         [&](int it, int, size_t i) {
             pvx[it] = VX[i]; pvy[it] = VY[i];
             pl0[it] = lo.p[HG_P_SED_ROCK][i]; pl1[it] = lo.p[HG_P_SED_DIRT][i];
-            if (it < GTIT) {
+            if (it < GTIT<NT>) {
                 plb[it] = lo.p[HG_P_WATER][i];
                 pb[it] = x.p[HG_P_WATER][i];
             }
@@ -754,7 +768,7 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
                            (unsigned(t.iy1 - qy + 1) << 6);
                     w[0] = t.w00; w[1] = t.w10; w[2] = t.w01; w[3] = t.w11;
                 }
-                if (it < GTIT) {
+                if (it < GTIT<NT>) {
                     const size_t j00 = at(t.ix, t.iy, nx), j10 = at(t.ix1, t.iy, nx), j01 = at(t.ix, t.iy1, nx),
                                  j11 = at(t.ix1, t.iy1, nx);
 #pragma unroll
@@ -830,13 +844,14 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
             li.p[HG_P_WATER][i] = lb * k.evap;                   // b' = b (1 - Ke dt)
             gKe += double(lb) * double(pb[it]) * double(-k.dt);
         });
-    reduce_coef<GNT>(gpart, T.slot, 0.0, 0.0, 0.0, gKe);
+    reduce_coef<NT>(gpart, T.slot, 0.0, 0.0, 0.0, gKe);
 }
 
-__global__ __launch_bounds__(GNT) void k_adj_transport(Planes x, Planes lo, Planes li, int nx, int ny, KParams k,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_transport(Planes x, Planes lo, Planes li, int nx, int ny, KParams k,
                                                        double* gpart) {
     __shared__ float lds[TRANSPORT_LDS];
-    adj_transport_tile(block_tile(), lds, x, lo, li, nx, ny, k, gpart);
+    adj_transport_tile<NT>(block_tile(), lds, x, lo, li, nx, ny, k, gpart);
 }
 
 // The transport VJP's scatter for cell (px, py) when its back-trace taps are
@@ -923,15 +938,15 @@ constexpr int THERMAL_LDS = 8 * GNR > 3 * SRN ? 8 * GNR : 3 * SRN;
 // A thermal layer's VJP on tile T, with `lds` (THERMAL_LDS floats) as its
 // LDS.  x: the layer's input rock and dirt.  Writes li's layer plane (fresh)
 // and, for layer 1, adds the rock part to li's rock in place.
-template <int layer>
+template <int NT, int layer>
 __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Planes x, Planes lo, Planes li,
                                                  int nx, int ny, const KParams& k) {
     float* t_r = lds;
     float* t_d = lds + SRN;
     float* t_lh = lds + 2 * SRN;
     float (*s_lD)[GNR] = reinterpret_cast<float (*)[GNR]>(lds);   // sent to the 8 neighbours
-    float o_self[GTIT], o_hl[GTIT], o_lh[GTIT];     // kept per thread
-    float snd[GIT][8];
+    float o_self[GTIT<NT>], o_hl[GTIT<NT>], o_lh[GTIT<NT>];     // kept per thread
+    float snd[GIT<NT>][8];
     constexpr int DX[8] = {-1, 1, 0, 0, -1, 1, -1, 1};
     constexpr int DY[8] = {0, 0, 1, -1, 1, 1, -1, -1};
     const float* R = x.p[HG_P_ROCK];
@@ -940,8 +955,8 @@ __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Pl
     {
         // rock, dirt (out of grid: HG_OOB_HEIGHT) and the layer's adjoint (0)
         // (layer 0 reads no dirt)
-        float a[SIT], b[SIT], c[SIT];
-        stage_walk(T, nx, ny, [&](int it, int, size_t i, bool in) {
+        float a[SIT<NT>], b[SIT<NT>], c[SIT<NT>];
+        stage_walk<NT>(T, nx, ny, [&](int it, int, size_t i, bool in) {
             const float r = R[i], l = LH[i];
             a[it] = in ? r : HG_OOB_HEIGHT;
             if constexpr (layer == 1) {
@@ -950,19 +965,19 @@ __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Pl
             }
             c[it] = in ? l : 0.0f;
         });
-        stage_walk(T, nx, ny, [&](int it, int s, size_t, bool) {
+        stage_walk<NT>(T, nx, ny, [&](int it, int s, size_t, bool) {
             t_r[s] = a[it];
             if constexpr (layer == 1) t_d[s] = b[it];
             t_lh[s] = c[it];
         });
     }
-    tile_gather_late(T, nx, ny,
+    tile_gather_late<NT>(T, nx, ny,
         [&](int, int, size_t) {},
         [&](int it, int e, int px, int py, bool in, bool) {
             float lD[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             float lself = 0.0f, lh_layer = 0.0f;
             const int sc = sidx(e);
-            if (it < GTIT) o_lh[it] = t_lh[sc];
+            if (it < GTIT<NT>) o_lh[it] = t_lh[sc];
             if (in) {
                 const float r = t_r[sc], d = layer == 1 ? t_d[sc] : 0.0f;
                 float Dk[8], lhn[8];
@@ -981,7 +996,7 @@ __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Pl
             }
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk) snd[it][kk] = lD[kk];
-            if (it < GTIT) {                                  // a tile cell keeps its own part
+            if (it < GTIT<NT>) {                                  // a tile cell keeps its own part
                 o_self[it] = lself;
                 o_hl[it] = lh_layer;
             }
@@ -1006,29 +1021,30 @@ __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Pl
         });
 }
 
-template <int layer>
-__global__ __launch_bounds__(GNT) void k_adj_thermal(Planes x, Planes lo, Planes li, int nx, int ny, KParams k) {
+template <int NT, int layer>
+__global__ __launch_bounds__(NT) void k_adj_thermal(Planes x, Planes lo, Planes li, int nx, int ny, KParams k) {
     __shared__ float lds[THERMAL_LDS];
-    adj_thermal_tile<layer>(block_tile(), lds, x, lo, li, nx, ny, k);
+    adj_thermal_tile<NT, layer>(block_tile(), lds, x, lo, li, nx, ny, k);
 }
 
 // ---- thermal layer 0 and the transport's far taps in one launch ----------
 // Run after the transport's near gather (the two passes' adjoints touch
 // disjoint planes, so their order does not matter): workgroups [0, tiles)
 // take the layer-0 VJP's tiles in row-major order (as k_adj_thermal<0>'s
-// grid does), the rest scatter the far taps of 256 cells each (as
+// grid does), the rest scatter the far taps of NT cells each (as
 // k_adj_transport_far), filling the thermal tiles' tail instead of a launch
 // of their own.  x0: layer 0's inputs; xt, lot, lit: the transport's.
-__global__ __launch_bounds__(GNT) void k_adj_thermal0_far(Planes x0, Planes lo0, Planes li0, Planes xt, Planes lot,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_thermal0_far(Planes x0, Planes lo0, Planes li0, Planes xt, Planes lot,
                                                           Planes lit, int nx, int ny, KParams k) {
     __shared__ float lds[THERMAL_LDS];
     const int ntx = (nx + GTX - 1) / GTX, nty = (ny + GTY - 1) / GTY;
     const int w = int(blockIdx.x);
     if (w < ntx * nty) {
-        adj_thermal_tile<0>(tile_at(w, ntx * nty, ntx), lds, x0, lo0, li0, nx, ny, k);
+        adj_thermal_tile<NT, 0>(tile_at(w, ntx * nty, ntx), lds, x0, lo0, li0, nx, ny, k);
         return;
     }
-    const size_t cell = size_t(w - ntx * nty) * GNT + threadIdx.x;
+    const size_t cell = size_t(w - ntx * nty) * NT + threadIdx.x;
     if (cell >= size_t(nx) * size_t(ny)) return;
     transport_far_cell(xt, lot, lit, int(cell % size_t(nx)), int(cell / size_t(nx)), nx, ny, k);
 }
@@ -1038,7 +1054,8 @@ __global__ __launch_bounds__(GNT) void k_adj_thermal0_far(Planes x0, Planes lo0,
 // receives 0.2 m dL/dy(q) from each interior neighbour q that is an extremum.
 // The extremum flags of the tile + 1-cell ring are evaluated once into LDS.
 // Writes li's rock and dirt (fresh).
-__global__ __launch_bounds__(GNT) void k_adj_smooth(Planes x, Planes lo, Planes li, int nx, int ny, KParams k) {
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_smooth(Planes x, Planes lo, Planes li, int nx, int ny, KParams k) {
     const TileId T = block_tile();
     // rock, dirt and their adjoints on the tile + 2-cell region; cells off the
     // grid hold the clamped cell's values, which only feed extremum flags of
@@ -1047,18 +1064,18 @@ __global__ __launch_bounds__(GNT) void k_adj_smooth(Planes x, Planes lo, Planes 
     // per tile/ring cell: bit 0 rock, bit 1 surface flag of an interior extremum
     __shared__ unsigned char s_f[GNR];
     {
-        float a[SIT], b[SIT], c[SIT], d[SIT];
-        stage_walk(T, nx, ny, [&](int it, int, size_t i, bool) {
+        float a[SIT<NT>], b[SIT<NT>], c[SIT<NT>], d[SIT<NT>];
+        stage_walk<NT>(T, nx, ny, [&](int it, int, size_t i, bool) {
             a[it] = x.p[HG_P_ROCK][i]; b[it] = x.p[HG_P_DIRT][i];
             c[it] = lo.p[HG_P_ROCK][i]; d[it] = lo.p[HG_P_DIRT][i];
         });
-        stage_walk(T, nx, ny, [&](int it, int s, size_t, bool) {
+        stage_walk<NT>(T, nx, ny, [&](int it, int s, size_t, bool) {
             t_r[s] = a[it]; t_d[s] = b[it]; t_lr[s] = c[it]; t_ld[s] = d[it];
         });
     }
     const float m = k.smooth_m;
-    float o_lr[GTIT], o_ld[GTIT];
-    tile_gather(T, nx, ny,
+    float o_lr[GTIT<NT>], o_ld[GTIT<NT>];
+    tile_gather<NT>(T, nx, ny,
         [&](int, int, size_t) {},
         [&](int it, int e, int px, int py, bool, bool) {
             const int sc = sidx(e);
@@ -1070,7 +1087,7 @@ __global__ __launch_bounds__(GNT) void k_adj_smooth(Planes x, Planes lo, Planes 
                 f = (er ? 1u : 0u) | (eg ? 2u : 0u);
             }
             s_f[e] = (unsigned char)f;
-            if (it < GTIT) {                                  // a tile cell keeps its own share
+            if (it < GTIT<NT>) {                                  // a tile cell keeps its own share
                 const float lr = t_lr[sc], ld = t_ld[sc];
                 o_lr[it] = (f & 1u) ? lr * (1.0f - 0.8f * m) : lr;
                 o_ld[it] = (f & 2u) ? ld * (1.0f - 0.8f * m) : ld;
@@ -1110,11 +1127,12 @@ constexpr int ST1_LDS = 2 * ST1_N4 + 2 * ST1_N3 + (ST1_N3 + 3) / 4 > 8 * GNR
                             ? 2 * ST1_N4 + 2 * ST1_N3 + (ST1_N3 + 3) / 4
                             : 8 * GNR;
 
+template <int NT>
 __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float* u, Planes x, Planes lo,
                                                          Planes li, const float* d3, int nx, int ny,
                                                          const KParams& k) {
-    constexpr int W4 = GTX + 8, N4 = ST1_N4, IT4 = (N4 + GNT - 1) / GNT;
-    constexpr int W3 = GTX + 6, N3 = ST1_N3, IT3 = (N3 + GNT - 1) / GNT;
+    constexpr int W4 = GTX + 8, N4 = ST1_N4, IT4 = per_thread(N4, NT);
+    constexpr int W3 = GTX + 6, N3 = ST1_N3, IT3 = per_thread(N3, NT);
     // One LDS array (21.1 KB), in turn:
     //  * rock after layer 0 (t_r5) and dirt after layer 1 (t_d6) on tile + 4,
     //    HG_OOB_HEIGHT off the grid (the flags of cells off or on the edge of
@@ -1135,34 +1153,34 @@ __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float*
     float* t_md = t_d6;
     float* t_d = t_lr;
     float (*s_lD)[GNR] = reinterpret_cast<float (*)[GNR]>(u);
-    float o_mr[GTIT], o_lh[GTIT], o_self[GTIT], o_hl[GTIT];
-    float snd[GIT][8];
+    float o_mr[GTIT<NT>], o_lh[GTIT<NT>], o_self[GTIT<NT>], o_hl[GTIT<NT>];
+    float snd[GIT<NT>][8];
     constexpr int DX[8] = {-1, 1, 0, 0, -1, 1, -1, 1};
     constexpr int DY[8] = {0, 0, 1, -1, 1, 1, -1, -1};
     const float m = k.smooth_m;
-    float e[SIT];                                // dirt after erosion, tile + 2, until its place is free
+    float e[SIT<NT>];                                // dirt after erosion, tile + 2, until its place is free
     {
         float a[IT4], b[IT4], c[IT3], d[IT3];
-        region_walk<4>(T, nx, ny, [&](int it, int, size_t i, bool in, int, int) {
+        region_walk<NT, 4>(T, nx, ny, [&](int it, int, size_t i, bool in, int, int) {
             const float r = x.p[HG_P_ROCK][i], dd = x.p[HG_P_DIRT][i];
             a[it] = in ? r : HG_OOB_HEIGHT;
             b[it] = in ? dd : HG_OOB_HEIGHT;
         });
-        region_walk<3>(T, nx, ny, [&](int it, int, size_t i, bool in, int, int) {
+        region_walk<NT, 3>(T, nx, ny, [&](int it, int, size_t i, bool in, int, int) {
             const float lr = lo.p[HG_P_ROCK][i], ld = lo.p[HG_P_DIRT][i];
             c[it] = in ? lr : 0.0f;
             d[it] = in ? ld : 0.0f;
         });
-        region_walk<2>(T, nx, ny, [&](int it, int, size_t i, bool in, int, int) {
+        region_walk<NT, 2>(T, nx, ny, [&](int it, int, size_t i, bool in, int, int) {
             const float v = d3[i];
             e[it] = in ? v : HG_OOB_HEIGHT;
         });
-        region_walk<4>(T, nx, ny, [&](int it, int s, size_t, bool, int, int) { t_r5[s] = a[it]; t_d6[s] = b[it]; });
-        region_walk<3>(T, nx, ny, [&](int it, int s, size_t, bool, int, int) { t_lr[s] = c[it]; t_ld[s] = d[it]; });
+        region_walk<NT, 4>(T, nx, ny, [&](int it, int s, size_t, bool, int, int) { t_r5[s] = a[it]; t_d6[s] = b[it]; });
+        region_walk<NT, 3>(T, nx, ny, [&](int it, int s, size_t, bool, int, int) { t_lr[s] = c[it]; t_ld[s] = d[it]; });
     }
     __syncthreads();
     // extremum flags on tile + 3, as k_adj_smooth evaluates them
-    region_walk<3>(T, nx, ny, [&](int, int s, size_t, bool, int gx, int gy) {
+    region_walk<NT, 3>(T, nx, ny, [&](int, int s, size_t, bool, int gx, int gy) {
         const int sy = s / W3, sx = s - sy * W3;
         const int c = (sy + 1) * W4 + sx + 1;
         unsigned f = 0;
@@ -1201,28 +1219,28 @@ __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float*
         return ad;
     };
     // the dirt adjoint on tile + 2 (layer 1's input adjoint)
-    region_walk<2>(T, nx, ny, [&](int, int s, size_t, bool in, int, int) {
+    region_walk<NT, 2>(T, nx, ny, [&](int, int s, size_t, bool in, int, int) {
         const int sy = s / SRW, sx = s - sy * SRW;
         t_md[s] = in ? smooth_d((sy + 1) * W3 + sx + 1) : 0.0f;
     });
     // the rock adjoint of each tile cell, kept by the thread that writes it
 #pragma unroll
-    for (int it = 0; it < GTIT; ++it) {
+    for (int it = 0; it < GTIT<NT>; ++it) {
         int ex, ey;
-        ring_cell(it, ex, ey);
+        ring_cell<NT>(it, ex, ey);
         o_mr[it] = smooth_r((ey + 2) * W3 + ex + 2);
     }
     __syncthreads();                             // the adjoints after smoothing are no longer read
-    region_walk<2>(T, nx, ny, [&](int it, int s, size_t, bool, int, int) { t_d[s] = e[it]; });
+    region_walk<NT, 2>(T, nx, ny, [&](int it, int s, size_t, bool, int, int) { t_d[s] = e[it]; });
     // layer 1, as k_adj_thermal<1> with t_lh = t_md (tile_gather_late's first
     // barrier completes t_d)
-    tile_gather_late(T, nx, ny,
+    tile_gather_late<NT>(T, nx, ny,
         [&](int, int, size_t) {},
         [&](int it, int e, int px, int py, bool in, bool) {
             float lD[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             float lself = 0.0f, lh_layer = 0.0f;
             const int sc = sidx(e);
-            if (it < GTIT) o_lh[it] = t_md[sc];
+            if (it < GTIT<NT>) o_lh[it] = t_md[sc];
             if (in) {
                 const int sy = sc / SRW, sx = sc - sy * SRW;
                 const int c4 = (sy + 2) * W4 + sx + 2;
@@ -1241,7 +1259,7 @@ __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float*
             }
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk) snd[it][kk] = lD[kk];
-            if (it < GTIT) {
+            if (it < GTIT<NT>) {
                 o_self[it] = lself;
                 o_hl[it] = lh_layer;
             }
@@ -1261,10 +1279,11 @@ __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float*
         });
 }
 
-__global__ __launch_bounds__(GNT) void k_adj_smooth_thermal1(Planes x, Planes lo, Planes li, const float* d3,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_smooth_thermal1(Planes x, Planes lo, Planes li, const float* d3,
                                                              int nx, int ny, KParams k) {
     __shared__ float u[ST1_LDS];
-    adj_smooth_thermal1_tile(block_tile(), u, x, lo, li, d3, nx, ny, k);
+    adj_smooth_thermal1_tile<NT>(block_tile(), u, x, lo, li, d3, nx, ny, k);
 }
 
 // ---- smoothing + thermal layer 1 and the transport's near gather ----------
@@ -1274,7 +1293,8 @@ __global__ __launch_bounds__(GNT) void k_adj_smooth_thermal1(Planes x, Planes lo
 // the transport's tiles (each on the XCD its own kernel would give it, with
 // the tile's coefficient slot), starting as the first ones finish.  xs, los,
 // lis: the smoothing + layer-1 planes; xt, lot, lit: the transport's.
-__global__ __launch_bounds__(GNT) void k_adj_smooth_thermal1_transport(Planes xs, Planes los, Planes lis,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_adj_smooth_thermal1_transport(Planes xs, Planes los, Planes lis,
                                                                        const float* d3, Planes xt, Planes lot,
                                                                        Planes lit, int nx, int ny, KParams k,
                                                                        double* gpart) {
@@ -1283,11 +1303,17 @@ __global__ __launch_bounds__(GNT) void k_adj_smooth_thermal1_transport(Planes xs
     const int ntx = (nx + GTX - 1) / GTX, nty = (ny + GTY - 1) / GTY, nt = ntx * nty;
     const int w = int(blockIdx.x);
     if (w < nt) {
-        adj_smooth_thermal1_tile(tile_at(w, nt, ntx), u, xs, los, lis, d3, nx, ny, k);
+        adj_smooth_thermal1_tile<NT>(tile_at(w, nt, ntx), u, xs, los, lis, d3, nx, ny, k);
     } else {
-        adj_transport_tile(tile_at(w - nt, nt, ntx), u, xt, lot, lit, nx, ny, k, gpart);
+        adj_transport_tile<NT>(tile_at(w - nt, nt, ntx), u, xt, lot, lit, nx, ny, k, gpart);
     }
 }
+
+// 512 threads per tile below 768^2 cells: a rollout of 32 steps at 256^2 takes
+// 0.99 ms instead of 1.15, at 512^2 1.80 instead of 1.92, at 600^2 2.14 instead
+// of 2.22; the two are equal at 768^2, and at 1024^2, where the tiles of 256
+// threads fill the chip and idle less at their barriers, 4.68 against 4.48.
+inline bool wide_gather(size_t cells) { return cells < size_t(768) * 768; }
 
 // Copies the 9 state planes of n floats (n = side^2, side % 8 == 0) in one launch.
 struct StateCopy {
@@ -1592,6 +1618,14 @@ extern "C" int hg_adjoint_rollout(hg_ctx* c, uint32_t nsteps, uint32_t k_ckpt, u
 
     const dim3 blk(BX, BY), grd((n + BX - 1) / BX, (n + BY - 1) / BY);
     const dim3 gtile((n + GTX - 1) / GTX, (n + GTY - 1) / GTY);
+    const bool wide = wide_gather(size_t(n) * size_t(n));
+    const unsigned nt = wide ? 512 : 256;
+    auto gather = [&](auto k512, auto k256, dim3 grid, auto... args) {
+        if (wide)
+            k512<<<grid, 512, 0, c->stream>>>(args...);
+        else
+            k256<<<grid, 256, 0, c->stream>>>(args...);
+    };
     // The taped recompute of a segment runs on a second stream (default
     // priority) while the main stream reverses the segment after it: at 1024^2
     // neither kernel sequence fills the chip alone.  Segment i (counting from
@@ -1706,55 +1740,57 @@ extern "C" int hg_adjoint_rollout(hg_ctx* c, uint32_t nsteps, uint32_t k_ckpt, u
                 const Planes li = planes_of(fresh);
                 switch (pass) {
                     case HG_PASS_FLUX:
-                        k_adj_flux<<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp);
+                        gather(k_adj_flux<512>, k_adj_flux<256>, gtile, X, lo, li, n, n, c->kp);
                         break;
                     case HG_PASS_EROSION:
-                        k_adj_erosion<<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp, w.gpart);
+                        gather(k_adj_erosion<512>, k_adj_erosion<256>, gtile, X, lo, li, n, n, c->kp, w.gpart);
                         break;
                     case UNIT_EROSION_FLUX:
-                        k_adj_erosion_flux<<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp, w.gpart);
+                        gather(k_adj_erosion_flux<512>, k_adj_erosion_flux<256>, gtile, X, lo, li, n, n, c->kp,
+                               w.gpart);
                         break;
                     case HG_PASS_TRANSPORT:
-                        k_adj_transport<<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp, w.gpart);
+                        gather(k_adj_transport<512>, k_adj_transport<256>, gtile, X, lo, li, n, n, c->kp, w.gpart);
                         HG_HIP(c, hipGetLastError());
                         k_adj_transport_far<<<grd, blk, 0, c->stream>>>(X, lo, li, n, n, c->kp);
                         break;
                     case UNIT_ST1_TRANSPORT: {
                         const Planes Xs = x_of(UNIT_SMOOTH_THERMAL1), Xt = x_of(HG_PASS_TRANSPORT);
-                        k_adj_smooth_thermal1_transport<<<2 * gtile.x * gtile.y, GNT, 0, c->stream>>>(
-                            Xs, lo, li, tp[T_D3], Xt, lo, li, n, n, c->kp, w.gpart);
+                        gather(k_adj_smooth_thermal1_transport<512>, k_adj_smooth_thermal1_transport<256>,
+                               2 * gtile.x * gtile.y, Xs, lo, li, tp[T_D3], Xt, lo, li, n, n, c->kp, w.gpart);
                         far_lo = lo;
                         far_li = li;
                         break;
                     }
                     case UNIT_THERMAL0_FAR: {
                         const Planes Xt = x_of(HG_PASS_TRANSPORT), X0 = x_of(HG_PASS_THERMAL_TRANSPORT_0);
-                        const unsigned nfar = unsigned((size_t(n) * size_t(n) + GNT - 1) / GNT);
-                        k_adj_thermal0_far<<<gtile.x * gtile.y + nfar, GNT, 0, c->stream>>>(X0, lo, li, Xt, far_lo,
-                                                                                            far_li, n, n, c->kp);
+                        const unsigned nfar = unsigned((size_t(n) * size_t(n) + nt - 1) / nt);
+                        gather(k_adj_thermal0_far<512>, k_adj_thermal0_far<256>, gtile.x * gtile.y + nfar, X0, lo, li,
+                               Xt, far_lo, far_li, n, n, c->kp);
                         break;
                     }
                     case UNIT_TRANSPORT_THERMAL0: {
                         const Planes Xt = x_of(HG_PASS_TRANSPORT), X0 = x_of(HG_PASS_THERMAL_TRANSPORT_0);
-                        k_adj_transport<<<gtile, GNT, 0, c->stream>>>(Xt, lo, li, n, n, c->kp, w.gpart);
+                        gather(k_adj_transport<512>, k_adj_transport<256>, gtile, Xt, lo, li, n, n, c->kp, w.gpart);
                         HG_HIP(c, hipGetLastError());
-                        const unsigned nfar = unsigned((size_t(n) * size_t(n) + GNT - 1) / GNT);
-                        k_adj_thermal0_far<<<gtile.x * gtile.y + nfar, GNT, 0, c->stream>>>(X0, lo, li, Xt, lo, li,
-                                                                                            n, n, c->kp);
+                        const unsigned nfar = unsigned((size_t(n) * size_t(n) + nt - 1) / nt);
+                        gather(k_adj_thermal0_far<512>, k_adj_thermal0_far<256>, gtile.x * gtile.y + nfar, X0, lo, li,
+                               Xt, lo, li, n, n, c->kp);
                         break;
                     }
                     case HG_PASS_THERMAL_TRANSPORT_0:
                     case HG_PASS_THERMAL_TRANSPORT_1:
                         if (pass == HG_PASS_THERMAL_TRANSPORT_0)
-                            k_adj_thermal<0><<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp);
+                            gather(k_adj_thermal<512, 0>, k_adj_thermal<256, 0>, gtile, X, lo, li, n, n, c->kp);
                         else
-                            k_adj_thermal<1><<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp);
+                            gather(k_adj_thermal<512, 1>, k_adj_thermal<256, 1>, gtile, X, lo, li, n, n, c->kp);
                         break;
                     case HG_PASS_SMOOTH:
-                        k_adj_smooth<<<gtile, GNT, 0, c->stream>>>(X, lo, li, n, n, c->kp);
+                        gather(k_adj_smooth<512>, k_adj_smooth<256>, gtile, X, lo, li, n, n, c->kp);
                         break;
                     case UNIT_SMOOTH_THERMAL1:
-                        k_adj_smooth_thermal1<<<gtile, GNT, 0, c->stream>>>(X, lo, li, tp[T_D3], n, n, c->kp);
+                        gather(k_adj_smooth_thermal1<512>, k_adj_smooth_thermal1<256>, gtile, X, lo, li, tp[T_D3], n, n,
+                               c->kp);
                         break;
                     default: break;
                 }
