@@ -85,35 +85,33 @@ __device__ __forceinline__ TileId block_tile() {
     return tile_at(int(blockIdx.y * gridDim.x + blockIdx.x), int(gridDim.x * gridDim.y), int(gridDim.x));
 }
 
-// Block reduction of up to 4 doubles, added by thread 0 to the block's own 4
+// Block reduction of up to 4 doubles, added by threads 0-3 to the block's own 4
 // slots of `gpart` (one slot set per workgroup of the launch, so no atomics:
 // same-address atomics from every workgroup serialise in one L2 channel).
-// Each wave sums its lanes by a fixed butterfly, then thread 0 adds the wave
-// sums in wave order, so the result does not depend on scheduling.  The host
+// Each wave sums its lanes by a fixed butterfly, then a thread per sum adds the
+// waves' in wave order, so the result does not depend on scheduling.  The host
 // sums the slots in workgroup order at the end of the rollout.
 template <int NT>
 __device__ void reduce_coef(double* gpart, int slot, double a, double b, double c, double d) {
     static_assert(NT % 64 == 0, "whole waves");
     constexpr int NW = NT / 64;
     __shared__ double sh[NW][4];
+    const int t = threadIdx.x;
+    double* q = gpart + 4 * size_t(slot) + (t & 3);
+    const double had = t < 4 ? *q : 0.0;         // under way while the waves are summed
     double v[4] = {a, b, c, d};
 #pragma unroll
     for (int m = 32; m > 0; m >>= 1)
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] += __shfl_xor(v[j], m, 64);
-    const int t = threadIdx.y * blockDim.x + threadIdx.x;
     if ((t & 63) == 0)
 #pragma unroll
         for (int j = 0; j < 4; ++j) sh[t >> 6][j] = v[j];
     __syncthreads();
-    if (t == 0) {
-        double* q = gpart + 4 * size_t(slot);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            double s = sh[0][j];
-            for (int w = 1; w < NW; ++w) s += sh[w][j];
-            if (s != 0.0) q[j] += s;
-        }
+    if (t < 4) {
+        double s = sh[0][t];
+        for (int w = 1; w < NW; ++w) s += sh[w][t];
+        if (s != 0.0) *q = had + s;
     }
 }
 
@@ -432,13 +430,14 @@ __device__ __forceinline__ ErosionVjp erosion_vjp(float r_in, float d_in, float 
     double cKc = 0, cKs = 0, cKd = 0;
     // conversion s1 += s0 kc, s0 -= s0 kc
     const float kc = k.Kconv * k.dt;
+    const float as1 = k.dt * k.Ks[1], ad1 = k.dt * k.Kd[1], as0 = k.dt * k.Ks[0], ad0 = k.dt * k.Kd[0];
     const float ls0c = ls0 * (1.0f - kc) + ls1 * kc, ls1c = ls1;
     // rock layer: (r, s0, c0) -> (r', s0c)
     float lc0 = 0.0f, lcap0 = 0.0f, lcap = 0.0f;
     float ls0_in = ls0c;
     float lr_in = lr;
     if (tp.case0 == 0 || tp.case0 == 2) {
-        const float a = k.dt * (tp.case0 == 0 ? k.Ks[0] : k.Kd[0]);
+        const float a = tp.case0 == 0 ? as0 : ad0;
         ls0_in = lr * a + ls0c * (1.0f - a);
         lc0 = (ls0c - lr) * a;
         if (tp.case0 == 0) cKs += double(k.dt) * double(tp.c0 - s0_in) * double(ls0c - lr);
@@ -456,7 +455,7 @@ __device__ __forceinline__ ErosionVjp erosion_vjp(float r_in, float d_in, float 
     float ls1_in = ls1c;
     float ld_in = ld;
     if (tp.case1 == 0 || tp.case1 == 2) {
-        const float a = k.dt * (tp.case1 == 0 ? k.Ks[1] : k.Kd[1]);
+        const float a = tp.case1 == 0 ? as1 : ad1;
         ls1_in = ld * a + ls1c * (1.0f - a);
         lc1 = (ls1c - ld) * a;
         if (tp.case1 == 0) cKs += double(k.dt) * double(tp.c1 - s1_in) * double(ls1c - ld);

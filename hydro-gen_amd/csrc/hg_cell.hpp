@@ -252,11 +252,14 @@ __device__ __forceinline__ void erosion_cell_t(float& r, float& d, float& s0, fl
     const float cap0 = k.Kc * fmaxf(0.02f, sin_a) * ero;
     tp.cap0 = cap0;
     // layer loop, dirt (1) then rock (0), :58-83.  Dissolving and depositing take
-    // the same a (c - s) off the layer and onto the sediment, each with its own a.
+    // the same a (c - s) off the layer and onto the sediment, each with its own a
+    // (both computed before the choice: chosen by address, they are loaded in
+    // every lane, behind all of the kernel's loads in flight).
+    const float as1 = k.dt * k.Ks[1], ad1 = k.dt * k.Kd[1], as0 = k.dt * k.Ks[0], ad0 = k.dt * k.Kd[0];
     const float c1 = fmaxf(0.0f, cap0);
     const bool take1 = c1 > s1;
     const float old = d;
-    const float delta1 = (take1 ? k.dt * k.Ks[1] : k.dt * k.Kd[1]) * (c1 - s1);
+    const float delta1 = (take1 ? as1 : ad1) * (c1 - s1);
     d -= delta1;
     s1 += delta1;
     const bool out1 = take1 && d < 0.0f;             // the layer was used up
@@ -267,7 +270,7 @@ __device__ __forceinline__ void erosion_cell_t(float& r, float& d, float& s0, fl
     tp.case1 = out1 ? 1 : (take1 ? 0 : 2);
     const float c0 = fmaxf(0.0f, cap0 - (out1 ? old : 0.0f));
     const bool take0 = c0 > s0;
-    const float delta0 = (take0 ? k.dt * k.Ks[0] : k.dt * k.Kd[0]) * (c0 - s0);
+    const float delta0 = (take0 ? as0 : ad0) * (c0 - s0);
     float rn = r - delta0, sn = s0 + delta0;
     const bool out0 = take0 && rn < 0.0f;
     sn = out0 ? sn + rn : sn;
