@@ -65,3 +65,24 @@ def test_march_in_a_batch(flags):
             states.append([b.read_state(i) for i in range(len(sides))])
     for x, y in zip(*states):
         assert np.array_equal(x, y)
+
+
+def test_march_per_terrain_launches_of_a_batch():
+    """A batch's terrains launched one by one, eagerly and from a graph, take row
+    segments of their own."""
+    sides, flags, states = [8, 120, 256, 1032], hg.STEP_DEFAULT, []
+    for per_terrain in (0, hg.STEP_PER_TERRAIN):
+        with hg.Batch(sides) as b:
+            b.set_rain(hg.RAIN_UNIFORM, amount=0.02, seed=5)
+            b.set_erosion(hg.erosion_settings())
+            for i, n in enumerate(sides):
+                b.init_fbm(i, hg.fbm_params(seed=i + 1, base_freq=1.0 / 24, hi=24.0))
+            b.set_tiles(-1, MARCH)
+            b.step(2, flags | per_terrain)
+            b.capture(2, flags | per_terrain)
+            for _ in range(3):
+                b.run()
+            b.sync()
+            states.append([b.read_state(i) for i in range(len(sides))])
+    for x, y in zip(*states):
+        assert np.array_equal(x, y)
