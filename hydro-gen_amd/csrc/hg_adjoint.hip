@@ -709,7 +709,7 @@ __global__ __launch_bounds__(NT) void k_adj_erosion_flux(Planes x, Planes lo, Pl
 // atomics afterwards (k_adj_transport_far).
 struct Taps {
     int ix, iy, ix1, iy1;
-    float w00, w10, w01, w11;
+    float fx, fy;
     bool near;
 };
 __device__ __forceinline__ Taps taps_of(int qx, int qy, float vx, float vy, int nx, int ny, float dt) {
@@ -717,29 +717,30 @@ __device__ __forceinline__ Taps taps_of(int qx, int qy, float vx, float vy, int 
     float bx, by;
     back_trace(qx, qy, vx, vy, dt, nx, ny, bx, by);
     t.ix = int(bx); t.iy = int(by);
-    const float fx = bx - float(t.ix), fy = by - float(t.iy);
+    t.fx = bx - float(t.ix); t.fy = by - float(t.iy);
     t.ix1 = min(t.ix + 1, nx - 1); t.iy1 = min(t.iy + 1, ny - 1);
-    t.w00 = (1.0f - fx) * (1.0f - fy); t.w10 = fx * (1.0f - fy); t.w01 = (1.0f - fx) * fy; t.w11 = fx * fy;
     t.near = t.ix >= qx - 1 && t.ix1 <= qx + 1 && t.iy >= qy - 1 && t.iy1 <= qy + 1;
     return t;
 }
 
 // LDS of one transport tile, in floats.
-constexpr int TRANSPORT_LDS = 6 * GNR + (GNR + 3) / 4;
+constexpr int TRANSPORT_LDS = 8 * GNR;
 
 // The transport VJP's near gather on tile T, with `lds` (TRANSPORT_LDS
 // floats) as its LDS.
 template <int NT>
 __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, Planes x, Planes lo, Planes li,
                                                    int nx, int ny, const KParams& k, double* gpart) {
-    // per tile/ring cell q: its 4 bilinear weights, its taps as offsets from
-    // q (bits 0-1: ix - qx + 1, 2-3: ix1 - qx + 1, 4-5: iy - qy + 1, 6-7:
-    // iy1 - qy + 1; 0 when q is off the grid or its taps are not near), and the
-    // sediment adjoints it spreads over them
-    float (*s_w)[GNR] = reinterpret_cast<float (*)[GNR]>(lds);
-    float* s_l0 = lds + 4 * GNR;
-    float* s_l1 = lds + 5 * GNR;
-    unsigned char* s_tap = reinterpret_cast<unsigned char*>(lds + 6 * GNR);
+    // per tile/ring cell q: the weight its back-trace gives the columns qx - 1,
+    // qx and qx + 1, and the rows (0 where it has no tap), and the sediment
+    // adjoints it spreads over them (0 off the grid, and where the taps are not
+    // near); a tap's bilinear weight is its column's times its row's.  Gathering
+    // by 4 weights and a byte of tap offsets took 340 VALU instructions a cell
+    // for the tests, this takes 45 for the nine neighbours.
+    float (*s_wx)[GNR] = reinterpret_cast<float (*)[GNR]>(lds);
+    float (*s_wy)[GNR] = reinterpret_cast<float (*)[GNR]>(lds + 3 * GNR);
+    float* s_l0 = lds + 6 * GNR;
+    float* s_l1 = lds + 7 * GNR;
     const float* VX = x.p[HG_P_VEL_U];
     const float* VY = x.p[HG_P_VEL_V];
     double gKe = 0;
@@ -747,7 +748,7 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
     // a tile cell's own water and its adjoint, and the sediment at its own
     // back-trace taps (both layers: s00, s10, s01, s11), loaded before the
     // gather phase needs them
-    float plb[GTIT<NT>], pb[GTIT<NT>], ps[GTIT<NT>][8];
+    float plb[GTIT<NT>], pb[GTIT<NT>], ps[GTIT<NT>][8], pfx[GTIT<NT>], pfy[GTIT<NT>];
     tile_gather<NT>(T, nx, ny,
         [&](int it, int, size_t i) {
             pvx[it] = VX[i]; pvy[it] = VY[i];
@@ -758,14 +759,25 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
             }
         },
         [&](int it, int e, int qx, int qy, bool in, bool) {
-            unsigned code = 0;
-            float w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            float wx[3] = {0.0f, 0.0f, 0.0f}, wy[3] = {0.0f, 0.0f, 0.0f}, l0 = 0.0f, l1 = 0.0f;
             if (in) {
                 const Taps t = taps_of(qx, qy, pvx[it], pvy[it], nx, ny, k.dt);
                 if (t.near) {
-                    code = unsigned(t.ix - qx + 1) | (unsigned(t.ix1 - qx + 1) << 2) | (unsigned(t.iy - qy + 1) << 4) |
-                           (unsigned(t.iy1 - qy + 1) << 6);
-                    w[0] = t.w00; w[1] = t.w10; w[2] = t.w01; w[3] = t.w11;
+                    // a column clamped onto the one before it (ix1 = ix = nx - 1) has fx = 0
+                    const int mx = t.ix - qx, my = t.iy - qy;
+                    const float gx = 1.0f - t.fx, gy = 1.0f - t.fy;
+                    wx[0] = mx < 0 ? gx : 0.0f;
+                    wx[1] = mx < 0 ? t.fx : mx == 0 ? gx : 0.0f;
+                    wx[2] = mx < 0 ? 0.0f : mx == 0 ? t.fx : gx;
+                    wy[0] = my < 0 ? gy : 0.0f;
+                    wy[1] = my < 0 ? t.fy : my == 0 ? gy : 0.0f;
+                    wy[2] = my < 0 ? 0.0f : my == 0 ? t.fy : gy;
+                    l0 = pl0[it];
+                    l1 = pl1[it];
+                }
+                if (it < GTIT<NT>) {
+                    pfx[it] = t.fx;
+                    pfy[it] = t.fy;
                 }
                 if (it < GTIT<NT>) {
                     const size_t j00 = at(t.ix, t.iy, nx), j10 = at(t.ix1, t.iy, nx), j01 = at(t.ix, t.iy1, nx),
@@ -779,38 +791,23 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
                 }
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s_w[j][e] = w[j];
-            s_tap[e] = (unsigned char)code;
-            s_l0[e] = in ? pl0[it] : 0.0f;
-            s_l1[e] = in ? pl1[it] : 0.0f;
+            for (int j = 0; j < 3; ++j) {
+                s_wx[j][e] = wx[j];
+                s_wy[j][e] = wy[j];
+            }
+            s_l0[e] = l0;
+            s_l1[e] = l1;
         },
         [&](int it, int e, int px, int py) {
             const size_t i = at(px, py, nx);
-            // sediment: gather from the near cells whose taps include p.  A
-            // neighbour q = p + (dx, dy) has p as a tap column when
-            // ix - qx = -dx (or ix1 - qx = -dx), and likewise for rows.  A
-            // near cell's code is never 0: that needs ix1 = ix = qx - 1, and
-            // ix1 = ix only at ix = nx - 1, i.e. qx = nx.
+            // sediment: what each neighbour q = p + (dx, dy) gives p's column and row
             float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
             for (int dy = -1; dy <= 1; ++dy)
 #pragma unroll
                 for (int dx = -1; dx <= 1; ++dx) {
                     const int eq = e + dx + dy * GRW;
-                    const unsigned code = s_tap[eq];
-                    if (code == 0) continue;
-                    const int cx = 1 - dx, cy = 1 - dy;     // p - q + 1
-                    const bool x0 = int(code & 3u) == cx, x1 = int((code >> 2) & 3u) == cx;
-                    const bool y0 = int((code >> 4) & 3u) == cy, y1 = int((code >> 6) & 3u) == cy;
-                    float w = 0.0f;
-                    if (y0) {
-                        if (x0) w += s_w[0][eq];
-                        if (x1) w += s_w[1][eq];
-                    }
-                    if (y1) {
-                        if (x0) w += s_w[2][eq];
-                        if (x1) w += s_w[3][eq];
-                    }
+                    const float w = s_wx[1 - dx][eq] * s_wy[1 - dy][eq];
                     a0 += s_l0[eq] * w;
                     a1 += s_l1[eq] * w;
                 }
@@ -820,10 +817,7 @@ __device__ __forceinline__ void adj_transport_tile(const TileId& T, float* lds, 
             const float vx = pvx[it], vy = pvy[it];
             const float bxr = float(px) - vx * k.dt;
             const float byr = float(py) - vy * k.dt;
-            const Taps t = taps_of(px, py, vx, vy, nx, ny, k.dt);
-            float bx, by;
-            back_trace(px, py, vx, vy, k.dt, nx, ny, bx, by);
-            const float fx = bx - float(t.ix), fy = by - float(t.iy);
+            const float fx = pfx[it], fy = pfy[it];
             const float l0 = pl0[it], l1 = pl1[it];
             float lbx = 0.0f, lby = 0.0f;
 #pragma unroll
@@ -861,16 +855,18 @@ __device__ __forceinline__ void transport_far_cell(const Planes& x, const Planes
     const Taps t = taps_of(px, py, x.p[HG_P_VEL_U][i], x.p[HG_P_VEL_V][i], nx, ny, k.dt);
     if (t.near) return;
     const float l0 = lo.p[HG_P_SED_ROCK][i], l1 = lo.p[HG_P_SED_DIRT][i];
+    const float w00 = (1.0f - t.fx) * (1.0f - t.fy), w10 = t.fx * (1.0f - t.fy), w01 = (1.0f - t.fx) * t.fy,
+                w11 = t.fx * t.fy;
     const size_t j00 = at(t.ix, t.iy, nx), j10 = at(t.ix1, t.iy, nx), j01 = at(t.ix, t.iy1, nx),
                  j11 = at(t.ix1, t.iy1, nx);
-    aadd(li.p[HG_P_SED_ROCK] + j00, l0 * t.w00);
-    aadd(li.p[HG_P_SED_ROCK] + j10, l0 * t.w10);
-    aadd(li.p[HG_P_SED_ROCK] + j01, l0 * t.w01);
-    aadd(li.p[HG_P_SED_ROCK] + j11, l0 * t.w11);
-    aadd(li.p[HG_P_SED_DIRT] + j00, l1 * t.w00);
-    aadd(li.p[HG_P_SED_DIRT] + j10, l1 * t.w10);
-    aadd(li.p[HG_P_SED_DIRT] + j01, l1 * t.w01);
-    aadd(li.p[HG_P_SED_DIRT] + j11, l1 * t.w11);
+    aadd(li.p[HG_P_SED_ROCK] + j00, l0 * w00);
+    aadd(li.p[HG_P_SED_ROCK] + j10, l0 * w10);
+    aadd(li.p[HG_P_SED_ROCK] + j01, l0 * w01);
+    aadd(li.p[HG_P_SED_ROCK] + j11, l0 * w11);
+    aadd(li.p[HG_P_SED_DIRT] + j00, l1 * w00);
+    aadd(li.p[HG_P_SED_DIRT] + j10, l1 * w10);
+    aadd(li.p[HG_P_SED_DIRT] + j01, l1 * w01);
+    aadd(li.p[HG_P_SED_DIRT] + j11, l1 * w11);
 }
 
 __global__ __launch_bounds__(256) void k_adj_transport_far(Planes x, Planes lo, Planes li, int nx, int ny,
@@ -888,44 +884,51 @@ __global__ __launch_bounds__(256) void k_adj_transport_far(Planes x, Planes lo, 
 // sum to p (both rock and dirt for layer 1, whose D_k spans both layers).
 //
 // thermal_vjp: one in-grid cell p.  Dk: p's height differences to its 8
-// neighbours (thermal_g's order), h_layer: p's height of the layer, lh and
-// lhn: the layer's adjoint at p and at its neighbours, ok: whether each
-// neighbour is on the grid.  Gives lD (what p sends to each neighbour, 0 off
-// the grid), lself (p's own part) and lh_layer (through H = min(h_layer, .)).
+// neighbours (thermal_g's order; very negative off the grid), h_layer: p's
+// height of the layer, lh and lhn: the layer's adjoint at p and at its
+// neighbours.  Gives lD (what p sends to each neighbour; nobody gathers what
+// goes off the grid), lself (p's own part) and lh_layer (through H =
+// min(h_layer, .)).
 template <int layer>
 __device__ __forceinline__ void thermal_vjp(const float Dk[8], float h_layer, float lh, const float lhn[8],
-                                            const bool ok[8], const KParams& k, float lD[8], float& lself,
-                                            float& lh_layer) {
+                                            const KParams& k, float lD[8], float& lself, float& lh_layer) {
     ThermalTape tp;
     const float g = thermal_g_t(Dk, h_layer, layer, k, tp);
     if (tp.bk > 0.0f) {
         float lg = 0.0f;
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) {
-            const bool m = talus_marked(Dk[kk], kk, layer, k);
             const float lout = lhn[kk] - lh;          // dL/dT_k
-            lD[kk] = m ? lout * g : 0.0f;
-            if (m) lg += lout * Dk[kk];
+            lD[kk] = lout * g;
+            if (talus_marked(Dk[kk], kk, layer, k)) lg += lout * Dk[kk];
         }
         const float rb = rcp(tp.bk);              // g = S / bk
         const float lS = lg * rb, lbk = -lg * g * rb;
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-            if (talus_marked(Dk[kk], kk, layer, k)) lD[kk] += lbk;
+        for (int kk = 0; kk < 8; ++kk) lD[kk] = talus_marked(Dk[kk], kk, layer, k) ? lD[kk] + lbk : 0.0f;
         const float A = k.dt * k.Kspeed[layer] * 0.5f;  // S = A sharp^3 H
         const float sh3 = tp.sharp * (tp.sharp * tp.sharp);
         const float lsh3 = lS * A * tp.H, lH = lS * A * sh3;
+        // what reaches the largest cross (c) and diagonal (d) difference
+        float rc = 0.0f, rd = 0.0f, hc = 0.0f, hd = 0.0f;
         if (tp.sharp_active) {                    // sharp = 1 + atan(rmax) - Kalpha
             const float lrmax = lsh3 * 3.0f * tp.sharp * tp.sharp * rcp(1.0f + tp.rmax * tp.rmax);
-            if (tp.mc >= tp.md * 0.70710678118654752f) lD[tp.kc] += lrmax;
-            else lD[tp.kd] += lrmax * 0.70710678118654752f;
+            const bool cross = tp.mc >= tp.md * 0.70710678118654752f;
+            rc = cross ? lrmax : 0.0f;
+            rd = cross ? 0.0f : lrmax * 0.70710678118654752f;
         }
-        if (tp.h_is_layer) lh_layer = lH;         // H = min(h_l, max(0, mc, md))
-        else if (fmaxf(tp.mc, tp.md) > 0.0f) lD[tp.mc >= tp.md ? tp.kc : tp.kd] += lH;
+        if (tp.h_is_layer) {                      // H = min(h_l, max(0, mc, md))
+            lh_layer = lH;
+        } else if (fmaxf(tp.mc, tp.md) > 0.0f) {
+            const bool cross = tp.mc >= tp.md;
+            hc = cross ? lH : 0.0f;
+            hd = cross ? 0.0f : lH;
+        }
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) {
+            const float with = (lD[kk] + (kk < 4 ? rc : rd)) + (kk < 4 ? hc : hd);
+            lD[kk] = tp.top[kk] ? with : lD[kk];
             lself += lD[kk];
-            if (!ok[kk]) lD[kk] = 0.0f;           // nothing is sent off the grid
         }
     }
 }
@@ -972,7 +975,7 @@ __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Pl
     }
     tile_gather_late<NT>(T, nx, ny,
         [&](int, int, size_t) {},
-        [&](int it, int e, int px, int py, bool in, bool) {
+        [&](int it, int e, int, int, bool in, bool) {
             float lD[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             float lself = 0.0f, lh_layer = 0.0f;
             const int sc = sidx(e);
@@ -980,18 +983,15 @@ __device__ __forceinline__ void adj_thermal_tile(const TileId& T, float* lds, Pl
             if (in) {
                 const float r = t_r[sc], d = layer == 1 ? t_d[sc] : 0.0f;
                 float Dk[8], lhn[8];
-                bool ok[8];
 #pragma unroll
                 for (int kk = 0; kk < 8; ++kk) {
-                    const int xx = px + DX[kk], yy = py + DY[kk];
                     const int o = sc + DX[kk] + DY[kk] * SRW;
-                    ok[kk] = xx >= 0 && yy >= 0 && xx < nx && yy < ny;
                     float v = r - t_r[o];
                     if constexpr (layer == 1) v = v + (d - t_d[o]);
                     Dk[kk] = v;
                     lhn[kk] = t_lh[o];
                 }
-                thermal_vjp<layer>(Dk, layer == 0 ? r : d, t_lh[sc], lhn, ok, k, lD, lself, lh_layer);
+                thermal_vjp<layer>(Dk, layer == 0 ? r : d, t_lh[sc], lhn, k, lD, lself, lh_layer);
             }
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk) snd[it][kk] = lD[kk];
@@ -1235,7 +1235,7 @@ __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float*
     // barrier completes t_d)
     tile_gather_late<NT>(T, nx, ny,
         [&](int, int, size_t) {},
-        [&](int it, int e, int px, int py, bool in, bool) {
+        [&](int it, int e, int, int, bool in, bool) {
             float lD[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             float lself = 0.0f, lh_layer = 0.0f;
             const int sc = sidx(e);
@@ -1245,16 +1245,13 @@ __device__ __forceinline__ void adj_smooth_thermal1_tile(const TileId& T, float*
                 const int c4 = (sy + 2) * W4 + sx + 2;
                 const float r = t_r5[c4], d = t_d[sc];
                 float Dk[8], lhn[8];
-                bool ok[8];
 #pragma unroll
                 for (int kk = 0; kk < 8; ++kk) {
-                    const int xx = px + DX[kk], yy = py + DY[kk];
                     const int o = sc + DX[kk] + DY[kk] * SRW;
-                    ok[kk] = xx >= 0 && yy >= 0 && xx < nx && yy < ny;
                     Dk[kk] = (r - t_r5[c4 + DX[kk] + DY[kk] * W4]) + (d - t_d[o]);
                     lhn[kk] = t_md[o];
                 }
-                thermal_vjp<1>(Dk, d, t_md[sc], lhn, ok, k, lD, lself, lh_layer);
+                thermal_vjp<1>(Dk, d, t_md[sc], lhn, k, lD, lself, lh_layer);
             }
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk) snd[it][kk] = lD[kk];

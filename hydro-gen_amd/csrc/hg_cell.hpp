@@ -316,7 +316,7 @@ __device__ __forceinline__ bool talus_marked(float D, int k, int layer, const KP
 // Intermediates of thermal_g kept for the adjoint.
 struct ThermalTape {
     float bk, mc, md, H, rmax, sharp, S;
-    int kc, kd;            // first index of the largest cross / diagonal D
+    bool top[8];           // the first of the largest cross (0-3) and diagonal (4-7) D
     bool h_is_layer;       // H = h_l (else H = max(0, mc, md))
     bool sharp_active;     // 1 + atan(rmax) - Kalpha > 1
 };
@@ -324,19 +324,24 @@ struct ThermalTape {
 __device__ __forceinline__ float thermal_g_t(const float D[8], float h_layer, int layer,
                                              const KParams& p, ThermalTape& tp) {
     const float ta = p.tan_alpha[layer], td = p.thr_diag[layer];
-    float bk = 0.0f, mc = D[0], md = D[4];
-    int kc = 0, kd = 4;
+    float bk = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) bk += D[k] > ta ? D[k] : 0.0f;
+#pragma unroll
+    for (int k = 4; k < 8; ++k) bk += D[k] > td ? D[k] : 0.0f;
+    const float mc = fmaxf(fmaxf(D[0], D[1]), fmaxf(D[2], D[3]));
+    const float md = fmaxf(fmaxf(D[4], D[5]), fmaxf(D[6], D[7]));
+    // as lane masks, one compare each: an index would cost a compare and two
+    // selects here, and a select per element where it is used
+    bool below_c = true, below_d = true;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        bk += D[k] > ta ? D[k] : 0.0f;
-        if (D[k] > mc) { mc = D[k]; kc = k; }
+        tp.top[k] = below_c && D[k] == mc;
+        below_c = below_c && D[k] != mc;
+        tp.top[4 + k] = below_d && D[4 + k] == md;
+        below_d = below_d && D[4 + k] != md;
     }
-#pragma unroll
-    for (int k = 4; k < 8; ++k) {
-        bk += D[k] > td ? D[k] : 0.0f;
-        if (D[k] > md) { md = D[k]; kd = k; }
-    }
-    tp.bk = bk; tp.mc = mc; tp.md = md; tp.kc = kc; tp.kd = kd;
+    tp.bk = bk; tp.mc = mc; tp.md = md;
     if (!(bk > 0.0f)) return 0.0f;
     // H = min(h_l, max(0, max_k D_k))                                                  :46-58
     const float M = fmaxf(fmaxf(mc, md), 0.0f);
