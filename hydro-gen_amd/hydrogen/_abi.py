@@ -391,8 +391,8 @@ class Terrain:
         self._check(self.lib.hg_set_droplets(self.h, ctypes.byref(d)))
 
     def set_droplet_order(self, mode: int):
-        """hg_set_droplet_order: 0 thread j runs droplet j, 1 droplets sorted
-        by the tile of their start cell."""
+        """hg_set_droplet_order: 0 droplets in the order of their numbers, 1
+        droplets sorted by the tile of their start cell."""
         self._check(self.lib.hg_set_droplet_order(self.h, mode))
 
     def get_droplet_order(self) -> int:
@@ -548,7 +548,8 @@ class Terrain:
 
     def set_sweep(self, variant: int):
         """One-kernel steps (hg_set_sweep): a KERNEL_SWEEP variant, or -1 for
-        the hydro and thermal kernels."""
+        the hydro and thermal kernels (on small maps the default, while
+        get_sweep gives -1, is a one-kernel tile variant)."""
         self._check(self.lib.hg_set_sweep(self.h, variant))
 
     def get_sweep(self) -> int:
@@ -558,7 +559,8 @@ class Terrain:
 
     def set_xcd_order(self, mode: int):
         """Workgroup-to-tile order of the fused kernels (hg_set_xcd_order):
-        0 row-major, 1 contiguous runs per XCD, 2 column strips per XCD."""
+        0 row-major, 1 contiguous runs per XCD, 2 column strips per XCD
+        (contiguous runs where the tile columns do not divide by 8)."""
         self._check(self.lib.hg_set_xcd_order(self.h, int(mode)))
 
     def autotune(self, steps: int = 10, flags: int = STEP_DEFAULT):

@@ -446,7 +446,9 @@ int hg_adjoint_rollout(hg_ctx* ctx, uint32_t nsteps, uint32_t k_ckpt, uint32_t f
  * (tile width x height, halo, threads per workgroup).  The autotuner times
  * each on the context's own grid and keeps the fastest; the choice is cached
  * per (grid size, device architecture) for contexts created later in the
- * process.  These have no counterpart in the reference (its workgroup is a
+ * process.  Until then, and in batches, a variant is chosen by the number of
+ * cells.  The last HG_KERNEL_THERMAL variant is not tiled but marches: each of
+ * a workgroup's 4 waves takes 116 columns (tile_x) down a segment of rows.  These have no counterpart in the reference (its workgroup is a
  * fixed 8x8, glsl/bindings.glsl:9-10). */
 enum { HG_KERNEL_HYDRO = 0, HG_KERNEL_THERMAL = 1, HG_KERNEL_SWEEP = 2 };
 int hg_tile_variant_count(int kernel);
@@ -459,10 +461,12 @@ int hg_set_tiles(hg_ctx* ctx, int hydro_variant, int thermal_variant);
 int hg_get_tiles(const hg_ctx* ctx, int* hydro_variant, int* thermal_variant);
 /* Tile order of the fused kernels' workgroups, which the hardware deals to
  * the 8 XCDs round robin.  0: row-major tile order.  1: each XCD gets a
- * contiguous run of tiles.  2: each XCD gets a column strip of tiles (when
- * the tile columns divide by 8) and walks it row by row, so the halos a tile
- * shares with its horizontal and vertical neighbours are read through one
- * L2 (the default).  Returns HG_ERR_INVALID for other modes. */
+ * contiguous run of tiles.  2: each XCD gets a column strip of tiles and
+ * walks it row by row, so the halos a tile shares with its horizontal and
+ * vertical neighbours are read through one L2 (the default); where the tile
+ * columns do not divide by 8, a contiguous run of tiles, or row-major order
+ * on maps too wide for two rows of tiles to stay in an L2.  Returns
+ * HG_ERR_INVALID for other modes. */
 int hg_set_xcd_order(hg_ctx* ctx, int mode);
 /* One-kernel steps.  With a HG_KERNEL_SWEEP variant, hg_step_grid runs
  * each fused step as one kernel: each wave (variants 0-4) or workgroup (5-9)
