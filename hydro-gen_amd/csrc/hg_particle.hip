@@ -517,16 +517,32 @@ static uint32_t chunk_spread(uint32_t count) {
     return k;
 }
 
-hipError_t launch_droplets(float* pairs_low, float* pairs_high, int n, const DropletParams& p, const Brush& brush,
+hipError_t launch_droplets(float* a, float* b, bool paired, int n, const DropletParams& p, const Brush& brush,
                            uint32_t iteration, const uint32_t* order, double* exported,
                            unsigned long long* steps, hipStream_t s) {
     if (p.count == 0) return hipSuccess;
     const uint32_t blocks = (p.count + kDropletsPerBlock - 1) / kDropletsPerBlock;
-    const HeightMap<true> map{pairs_low, pairs_high, n, n / 2};
-    k_droplets<false, true><<<blocks, kDropThreads, 0, s>>>(map, p, brush, iteration, 1,
-                                                            order ? chunk_spread(p.count) : 1u, order, exported, steps,
-                                                            nullptr);
+    const uint32_t spread = order ? chunk_spread(p.count) : 1u;
+    if (paired)
+        k_droplets<false, true><<<blocks, kDropThreads, 0, s>>>(HeightMap<true>{a, b, n, n / 2}, p, brush, iteration, 1,
+                                                                spread, order, exported, steps, nullptr);
+    else
+        k_droplets<false, false><<<blocks, kDropThreads, 0, s>>>(HeightMap<false>{a, b, n, 0}, p, brush, iteration, 1,
+                                                                 spread, order, exported, steps, nullptr);
     return hipGetLastError();
+}
+
+// Pairing and unpairing move 32 B a cell, 5.6 ps (once the planes are beyond the
+// caches; 24 us at 2048^2, 380 at 8192^2).  Pairs shorten each step of a
+// droplet's life by 1 to 1.5 us of the chain, and save 0.065 ns of atomics for
+// each step of each droplet.  us an iteration, paired / on the planes:
+//            64 x 20    4096 x 64   65536 x 64   262144 x 20
+//   512^2    123/143     390/482    1988/2479     2429/3082
+//  2048^2    119/131     380/447    1422/1699     1820/2234
+//  8192^2    481/124     733/414    1762/1680     2147/2260
+bool droplets_pair(int n, const DropletParams& p, uint32_t iterations) {
+    const double lives = double(p.count > 0 ? p.max_lifetime : 0u) * iterations;
+    return double(n) * n < lives * (262144.0 + 12.0 * p.count);
 }
 
 hipError_t launch_pair_heights(const float* rock, const float* dirt, float* low, float* high, int n, hipStream_t s) {

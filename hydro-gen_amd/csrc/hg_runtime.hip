@@ -578,13 +578,14 @@ int hg_step_particle(hg_ctx* c, uint32_t iterations, uint32_t flags) {
         }
         tiles = c->drop_order + p.count;
     }
-    // The droplets run on (rock, dirt) pairs, kept in the alternate buffers of
-    // the two planes (every pass that reads those writes them first).
+    // Where it pays, the droplets run on (rock, dirt) pairs, kept in the alternate
+    // buffers of the two planes (every pass that reads those writes them first).
+    const bool pairs = hgk::droplets_pair(c->n, p, thermal || smooth ? 1u : iterations);
     bool paired = false;
     for (uint32_t it = 0; it < iterations; ++it) {
         const uint32_t iter = c->particle_iter;
         int rc = HG_OK;
-        if (!paired && p.count > 0) {
+        if (pairs && !paired) {
             rc = timed_launch(c, "pair_heights", [&] {
                 return hgk::launch_pair_heights(c->cur[HG_P_ROCK], c->cur[HG_P_DIRT], c->alt[HG_P_ROCK],
                                                 c->alt[HG_P_DIRT], c->n, c->stream);
@@ -599,7 +600,8 @@ int hg_step_particle(hg_ctx* c, uint32_t iterations, uint32_t flags) {
             if (rc != HG_OK) return rc;
         }
         rc = timed_launch(c, "droplets", [&] {
-            return hgk::launch_droplets(c->alt[HG_P_ROCK], c->alt[HG_P_DIRT], c->n, p, brush, iter,
+            return hgk::launch_droplets(pairs ? c->alt[HG_P_ROCK] : c->cur[HG_P_ROCK],
+                                        pairs ? c->alt[HG_P_DIRT] : c->cur[HG_P_DIRT], pairs, c->n, p, brush, iter,
                                         ordered ? c->drop_order : nullptr, c->dev_exported, c->dev_dsteps,
                                         c->stream);
         });

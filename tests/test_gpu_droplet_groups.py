@@ -72,3 +72,29 @@ def test_noalloc_several_rounds_per_workgroup():
         steps = int(out.read_plane(hg.P_VEL_V).view(np.uint64).ravel()[0])
     assert abs(m1 + ex - m0) <= 1e-6 * m0
     assert count <= steps <= 2 * count and steps > 1.9 * count
+
+
+@pytest.mark.parametrize("n", [1768, 1776])
+def test_single_droplet_on_pairs_and_on_planes(n):
+    """On the larger map pairing the planes does not pay for one droplet of 12
+    steps, so it runs on the planes themselves; both follow the FP32 oracle."""
+    d = dict(count=1, seed=7, max_lifetime=12)
+    with hg.Terrain(n) as t:
+        t.init_fbm(hg.fbm_params(seed=7, base_freq=1.0 / 64, hi=32.0))
+        dirt = (np.random.default_rng(n).random((n, n)) * 0.02).astype(np.float32)
+        t.write_plane(hg.P_DIRT, dirt)
+        r0 = t.read_plane(hg.P_ROCK)
+        t.set_timing(True)
+        t.set_droplets(hg.droplet_settings(**d))
+        t.dispatch_particle(1)
+        r, dd = t.read_plane(hg.P_ROCK), t.read_plane(hg.P_DIRT)
+        ex, steps = t.particle_stats()
+        paired = "pair_heights" in t.kernel_stats()
+    r32, d32 = r0.copy(), dirt.copy()
+    ex32 = O.droplets(r32, d32, O.droplet_settings(**d), 0)
+    change = max(np.abs(r32 - r0).max(), np.abs(d32 - dirt).max())
+    err = max(np.abs(r - r32).max(), np.abs(dd - d32).max())
+    assert paired == (n == 1768)
+    assert steps > 0
+    assert err <= 1e-5 * max(change, 1e-3)
+    assert abs(ex - ex32) <= 1e-5 * max(abs(ex32), 1.0)
