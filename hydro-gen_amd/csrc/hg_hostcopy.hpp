@@ -13,7 +13,8 @@
 //
 // A HostCopy belongs to one context or batch and is used by its one host
 // thread.  The pinned slots (8 MB) and the helper threads are made when first
-// needed, sleep between copies, and end with the object.
+// needed, sleep between copies, and end with the object.  At most kCrews objects
+// of a process have helpers at a time; the others copy by their own thread.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -38,6 +39,7 @@ public:
         cv_.notify_all();
         for (std::thread& t : helper_)
             if (t.joinable()) t.join();
+        if (counted_) crews().fetch_sub(1);
         for (int i = 0; i < kSlots; ++i) {
             if (pin_[i]) (void)hipHostFree(pin_[i]);
             if (ev_[i]) (void)hipEventDestroy(ev_[i]);
@@ -49,7 +51,7 @@ public:
     hipError_t to_host(const void* src, void* dst, size_t bytes, hipStream_t s) {
         if (bytes == 0) return hipSuccess;
         hipError_t e = reserve(bytes);
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) return unpinned(dst, src, bytes, hipMemcpyDeviceToHost, s);
         const char* from = static_cast<const char*>(src);
         const size_t chunks = (bytes + kSlot - 1) / kSlot;
         auto enqueue = [&](size_t c) {
@@ -77,12 +79,10 @@ public:
     // `bytes` from `src` to device `dst`, in order with the work on `s`;
     // returns when the device holds them.
     hipError_t to_device(const void* src, void* dst, size_t bytes, hipStream_t s) {
-        if (bytes < kCrewMin) {                               // the runtime's own path is the shorter one here
-            const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);
-            return e != hipSuccess ? e : hipStreamSynchronize(s);
-        }
-        hipError_t e = reserve(bytes);
-        if (e != hipSuccess) return e;
+        hipError_t e = hipSuccess;
+        // below kCrewMin the runtime's own path is the shorter one
+        if (bytes < kCrewMin || (e = reserve(bytes)) != hipSuccess)
+            return unpinned(dst, src, bytes, hipMemcpyHostToDevice, s);
         const size_t chunks = (bytes + kSlot - 1) / kSlot;
         begin(nullptr, static_cast<const char*>(src), bytes);
         for (size_t c = 0; c < chunks && e == hipSuccess; ++c) {
@@ -105,9 +105,22 @@ private:
     static constexpr size_t kPiecesPerSlot = kSlot / kPiece;
     static constexpr size_t kCrewMin = size_t(1) << 20;       // smaller copies are over before a helper wakes
     static constexpr int kHelpers = 3;
+    static constexpr int kCrews = 32;                         // more copying at once than a host has links or cores for
+
+    static std::atomic<int>& crews() {
+        static std::atomic<int> n{0};
+        return n;
+    }
 
     static size_t chunk_bytes(size_t bytes, size_t c) { return std::min(kSlot, bytes - c * kSlot); }
     static size_t pieces_of(size_t bytes) { return (bytes + kPiece - 1) / kPiece; }
+
+    // The runtime's path for pageable memory; also when no more can be pinned.
+    static hipError_t unpinned(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+        (void)hipGetLastError();
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
+        return e != hipSuccess ? e : hipStreamSynchronize(s);
+    }
 
     hipError_t reserve(size_t bytes) {
         for (size_t i = 0; i < kSlots && i * kSlot < bytes; ++i) {   // each piece stored only once it exists
@@ -139,8 +152,11 @@ private:
         if (bytes < kCrewMin) return;
         if (!crew_tried_) {
             crew_tried_ = true;
+            counted_ = crews().fetch_add(1) < kCrews;
+            if (!counted_) crews().fetch_sub(1);
             try {
-                for (std::thread& t : helper_) t = std::thread([this] { help(); });
+                if (counted_)
+                    for (std::thread& t : helper_) t = std::thread([this] { help(); });
             } catch (...) {                                   // no threads to be had: fewer helpers, or none
             }
         }
@@ -217,7 +233,7 @@ private:
     std::atomic<int> inside_{0};
     // the helpers
     std::thread helper_[kHelpers];
-    bool crew_tried_ = false;
+    bool crew_tried_ = false, counted_ = false;
     std::mutex mu_;
     std::condition_variable cv_;
     bool stop_ = false, active_ = false;

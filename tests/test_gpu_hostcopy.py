@@ -42,3 +42,18 @@ def test_contexts_of_several_threads_copy_at_once():
     for th in threads:
         th.join()
     assert all(ok)
+
+
+def test_more_contexts_than_helper_crews():
+    """Contexts beyond those that have helpers copy by their own thread."""
+    n, a = 520, []
+    terrains = [hg.Terrain(n) for _ in range(36)]
+    try:
+        for i, t in enumerate(terrains):
+            a.append(np.random.default_rng(i).random((n, n), dtype=np.float32))
+            t.write_plane(hg.P_ROCK, a[-1])
+        for t, want in zip(terrains, a):
+            assert np.array_equal(t.read_plane(hg.P_ROCK), want)
+    finally:
+        for t in terrains:
+            t.close()
