@@ -117,7 +117,6 @@ private:
 
     // The runtime's path for pageable memory; also when no more can be pinned.
     static hipError_t unpinned(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
-        (void)hipGetLastError();
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
         return e != hipSuccess ? e : hipStreamSynchronize(s);
     }
@@ -127,7 +126,10 @@ private:
             if (!pin_[i]) {
                 void* p = nullptr;
                 const hipError_t e = hipHostMalloc(&p, kSlot, hipHostMallocDefault);
-                if (e != hipSuccess) return e;
+                if (e != hipSuccess) {
+                    (void)hipGetLastError();                  // the caller's other path is not to find it
+                    return e;
+                }
                 pin_[i] = static_cast<char*>(p);
             }
             if (!ev_[i]) {
