@@ -663,13 +663,15 @@ __global__ __launch_bounds__(NT) void k_step_tile(HydroIO io, ThermIO tio, int n
 // known the transfer is T = P g_p + N g_q: one of the products is the tile
 // form's G * D, the other is a zero.  p adds -T, q adds T, in the same
 // order of directions as thermal_g and thermal_term, so the results are the
-// same bit for bit (for finite heights: beside a cell whose g is not a number,
-// the tile form's unmarked transfer is 0 and this one is not).
+// same bit for bit, as long as the zeros meet no infinity or NaN, in a height or
+// a g.  A wave that has seen one (its sums of products of them are not finite)
+// runs its segment again in the ODD form, which takes thermal_term (a test per
+// row instead, and the products or thermal_term after it: 5 % slower).
 //
 // About 260 VALU instructions per cell, times 1.10 for the columns and 1.12
 // (at 49 rows) for the rows that are not its own, issued at one per 3.5 cycles
 // per SIMD, near the rate of their mix (2.7 with two operands, 4.2 with three
-// or a lane shift).  137 registers: three waves per SIMD; held to 128 for four
+// or a lane shift).  142 registers: three waves per SIMD; held to 128 for four
 // it spills and slows down (150).  4096^2: 165 -> 126 us per launch, a step
 // 430 -> 389 us, with three maps at once 402 -> 354; 2048^2 with three maps at
 // once 104 -> 91 us per step.
@@ -715,6 +717,7 @@ struct MarchLayer {
     float e_N_left;
     float mc[2], md[2];                 // largest difference of row a's cells towards row z
     float gz[2], gz_right;              // outflow scale of row z
+    float finite;                       // so were all heights and g so far, if this is
     float th[2], th_left;               // transfers along row z
     float tv[2], te[2], te_left, tf[2]; // transfers between row z and the row below it
 };
@@ -722,7 +725,7 @@ struct MarchLayer {
 // Takes the next row b; returns in out[] the layer's new heights of row z
 // (a.* are then b, z.* a).  in_a, in_z: whether this lane's cells of those rows
 // are on the grid.
-template <int LAYER>
+template <int LAYER, bool ODD>
 __device__ __forceinline__ void march_advance(MarchLayer<LAYER>& s, const MarchRow<LAYER>& b, bool in_a, bool in_z,
                                               const KParams& k, float (&out)[2]) {
     const float ta = k.tan_alpha[LAYER], td = k.thr_diag[LAYER];
@@ -765,16 +768,32 @@ __device__ __forceinline__ void march_advance(MarchLayer<LAYER>& s, const MarchR
     }
     const float g_right = lane_right(g[0]);
     // transfers along row a and between rows z and a
-    auto send = [](float P, float gp, float N, float gq) { return fmaf(N, gq, P * gp); };
+    s.finite = fmaf(a.r[0], a.r[1], fmaf(g[0], g[1], s.finite));
+    if constexpr (LAYER == 1) s.finite = fmaf(a.d[0], a.d[1], s.finite);
     float th[2], tv[2], te[2], tf[2];
-    th[0] = send(s.h.P[0], g[0], s.h.N[0], g[1]);
-    th[1] = send(s.h.P[1], g[1], s.h.N[1], g_right);
-    tv[0] = send(s.v.P[0], s.gz[0], s.v.N[0], g[0]);
-    tv[1] = send(s.v.P[1], s.gz[1], s.v.N[1], g[1]);
-    te[0] = send(s.e.P[0], s.gz[0], s.e.N[0], g[1]);
-    te[1] = send(s.e.P[1], s.gz[1], s.e.N[1], g_right);
-    tf[0] = send(s.f.P[0], s.gz[1], s.f.N[0], g[0]);
-    tf[1] = send(s.f.P[1], s.gz_right, s.f.N[1], g[1]);
+    if constexpr (!ODD) {
+        auto send = [](float P, float gp, float N, float gq) { return fmaf(N, gq, P * gp); };
+        th[0] = send(s.h.P[0], g[0], s.h.N[0], g[1]);
+        th[1] = send(s.h.P[1], g[1], s.h.N[1], g_right);
+        tv[0] = send(s.v.P[0], s.gz[0], s.v.N[0], g[0]);
+        tv[1] = send(s.v.P[1], s.gz[1], s.v.N[1], g[1]);
+        te[0] = send(s.e.P[0], s.gz[0], s.e.N[0], g[1]);
+        te[1] = send(s.e.P[1], s.gz[1], s.e.N[1], g_right);
+        tf[0] = send(s.f.P[0], s.gz[1], s.f.N[0], g[0]);
+        tf[1] = send(s.f.P[1], s.gz_right, s.f.N[1], g[1]);
+    } else {
+        const MarchRow<LAYER>& z = s.z;
+        const float zr = lane_right(z.r[0]), zd = lane_right(z.d[0]);
+        auto send = [](float D, float thr, float gp, float gq) { return -thermal_term(D, gp, gq, thr); };
+        th[0] = send(s.h.D[0], ta, g[0], g[1]);
+        th[1] = send(s.h.D[1], ta, g[1], g_right);
+        tv[0] = send(diff(z.r[0], z.d[0], a.r[0], a.d[0]), ta, s.gz[0], g[0]);
+        tv[1] = send(diff(z.r[1], z.d[1], a.r[1], a.d[1]), ta, s.gz[1], g[1]);
+        te[0] = send(diff(z.r[0], z.d[0], a.r[1], a.d[1]), td, s.gz[0], g[1]);
+        te[1] = send(diff(z.r[1], z.d[1], a.r_right, a.d_right), td, s.gz[1], g_right);
+        tf[0] = send(diff(z.r[1], z.d[1], a.r[0], a.d[0]), td, s.gz[1], g[0]);
+        tf[1] = send(diff(zr, zd, a.r[1], a.d[1]), td, s.gz_right, g[1]);
+    }
     const float th_left = lane_left(th[1]), te_left = lane_left(te[1]), tf_left = lane_left(tf[1]);
     // new heights of row z: L, R, T, B, LT, RT, LB, RB
 #pragma unroll
@@ -833,9 +852,10 @@ inline int march_rows(int nx, int ny) {
     }
 }
 
-// Rows [ys, ye) of the strip whose first written column is xs.
-template <bool EXTRA, bool NTS>
-__device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny, int xs, int ys, int ye, int do_thermal,
+// Rows [ys, ye) of the strip whose first written column is xs; false if the
+// lane met a height or g that is not finite.
+template <bool EXTRA, bool NTS, bool ODD>
+__device__ __forceinline__ bool march_segment(const ThermIO& io, int nx, int ny, int xs, int ys, int ye, int do_thermal,
                                               int do_smooth, const KParams& k) {
     const int lane = int(threadIdx.x) & 63;
     const int x = xs - MARCH_HX + 2 * lane;                  // the lane's first column; even, like nx
@@ -890,7 +910,7 @@ __device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny,
             push(r.x, r.y, d.x, d.y);
             if (y > ys) emit(y - 1);
         }
-        return;
+        return true;
     }
     MarchLayer<0> l0{};
     MarchLayer<1> l1{};
@@ -907,7 +927,7 @@ __device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny,
         if (upper) nd = load(io.d, y - 1);
         b.r_right = lane_right(b.r[0]);
         float rz[2];
-        march_advance<0>(l0, b, inx && iny(y - 1), inx && iny(y - 2), k, rz);
+        march_advance<0, ODD>(l0, b, inx && iny(y - 1), inx && iny(y - 2), k, rz);
         if (!upper) return;
         const bool in2 = inx && iny(y - 2);
         MarchRow<1> q;
@@ -919,7 +939,7 @@ __device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny,
         q.d_right = lane_right(q.d[0]);
         const float rock[2] = {l1.z.r[0], l1.z.r[1]};        // rock of row y - 4
         float dz[2];
-        march_advance<1>(l1, q, inx && iny(y - 3), inx && iny(y - 4), k, dz);
+        march_advance<1, ODD>(l1, q, inx && iny(y - 3), inx && iny(y - 4), k, dz);
         push(rock[0], rock[1], dz[0], dz[1]);
         if (y - 5 >= ys && y - 5 < ye) emit(y - 5);
     };
@@ -929,6 +949,14 @@ __device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny,
         row(y, true);
         row(y + 1, true);
     }
+    return fabsf(l0.finite) < INFINITY && fabsf(l1.finite) < INFINITY;
+}
+
+template <bool EXTRA, bool NTS>
+__device__ __forceinline__ void thermal_march(const ThermIO& io, int nx, int ny, int xs, int ys, int ye, int do_thermal,
+                                              int do_smooth, const KParams& k) {
+    const bool finite = march_segment<EXTRA, NTS, false>(io, nx, ny, xs, ys, ye, do_thermal, do_smooth, k);
+    if (__any(!finite)) (void)march_segment<EXTRA, NTS, true>(io, nx, ny, xs, ys, ye, do_thermal, do_smooth, k);
 }
 
 template <bool EXTRA, bool NTS>

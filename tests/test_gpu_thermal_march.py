@@ -36,6 +36,33 @@ def test_march_equals_per_pass(n, flags):
     assert np.array_equal(x, y)
 
 
+@pytest.mark.parametrize("n", [120, 352])
+@pytest.mark.parametrize("flags", [hg.STEP_THERMAL | hg.STEP_SMOOTH, hg.STEP_THERMAL])
+def test_march_equals_tiles_beside_infinite_heights(n, flags):
+    """The thermal passes alone (after an iteration of no droplets) on a map with
+    single infinities, pairs and a plateau of them, and cells that are no number:
+    the same cells are infinite or no number as with the tile kernel, and the
+    others are equal."""
+    rng, out = np.random.default_rng(n), []
+    rock = rng.random((n, n), dtype=np.float32) * 24
+    dirt = rng.random((n, n), dtype=np.float32)
+    rock[20, 30] = rock[60, 57] = rock[60, 58] = rock[n - 1, 0] = np.inf
+    rock[80:90, 50:66] = np.inf
+    rock[40, 90], dirt[100, 20], rock[8, 100] = -np.inf, np.inf, np.nan
+    dirt[30:33, 3:6] = -np.inf
+    for v in (0, MARCH):
+        with hg.Terrain(n) as t:
+            t.set_erosion(hg.erosion_settings())
+            t.write_plane(hg.P_ROCK, rock)
+            t.write_plane(hg.P_DIRT, dirt)
+            t.set_droplets(hg.droplet_settings(count=0))
+            t.set_tiles(-1, v)
+            t.dispatch_particle(1, flags)
+            out.append(t.read_state(hg.NUM_STATE_PLANES)[:2])
+    assert not np.isfinite(out[0]).all()
+    assert np.array_equal(out[0], out[1], equal_nan=True)
+
+
 def test_march_records_the_adjoint_tape():
     n, out = 232, []
     g = (np.random.default_rng(1).random((n, n), dtype=np.float32) - 0.5) / (n * n)
