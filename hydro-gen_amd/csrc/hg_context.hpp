@@ -51,7 +51,7 @@ struct hg_ctx {
     int thermal_variant = 0;
     int sweep_variant = -1;          // one-kernel step variant; -1: the hydro and thermal kernels
     // the one-kernel variant of a small map whose steps were neither tuned nor
-    // set (hg_set_sweep); -1: none.  Not while launches are timed, so that
+    // set (hg_set_sweep, hg_set_tiles); -1: none.  Not while launches are timed, so that
     // the two kernels are seen apart.
     int small_map_variant = -1;
     int step_variant() const { return sweep_variant < 0 && !timing ? small_map_variant : sweep_variant; }

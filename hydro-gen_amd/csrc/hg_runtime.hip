@@ -965,6 +965,8 @@ int hg_set_tiles(hg_ctx* c, int hydro_variant, int thermal_variant) {
         return fail(c, HG_ERR_INVALID, "hg_set_tiles: no such variant");
     if (hydro_variant >= 0) c->hydro_variant = hydro_variant;
     if (thermal_variant >= 0) c->thermal_variant = thermal_variant;
+    // tiles of the two kernels are a choice of these over a small map's one
+    if (hydro_variant >= 0 || thermal_variant >= 0) c->small_map_variant = -1;
     return HG_OK;
 }
 

@@ -539,6 +539,7 @@ class Terrain:
 
     # -- tiles / autotuning --
     def set_tiles(self, hydro: int = -1, thermal: int = -1):
+        """Tile variants of the two kernels (hg_set_tiles); -1 keeps one."""
         self._check(self.lib.hg_set_tiles(self.h, hydro, thermal))
 
     def get_tiles(self):

@@ -274,7 +274,9 @@ int hg_get_stream(hg_ctx* ctx, void** stream);
 /* ---- per-kernel timing -------------------------------------------------- */
 
 /* When enabled, every kernel launch is bracketed by HIP events on the
- * context's stream and its duration is accumulated per kernel name.
+ * context's stream and its duration is accumulated per kernel name.  An
+ * untuned small map then steps by the hydro and the thermal kernel instead of
+ * by one (hg_set_sweep); to time that one, select its variant.
  * hg_kernel_stats() synchronises and reports kernel i (0-based, in first-
  * launch order); returns HG_ERR_INVALID past the last one. */
 int hg_set_timing(hg_ctx* ctx, int enable);
@@ -456,7 +458,8 @@ int hg_tile_variant_count(int kernel);
  * width in columns, tile_y = rows of the segment a workgroup sweeps, halo =
  * rows per iteration of the sweep. */
 int hg_tile_variant_info(int kernel, int variant, int* tile_x, int* tile_y, int* halo, int* threads);
-/* -1 keeps the current choice. */
+/* -1 keeps the current choice.  A variant >= 0 of either kernel also ends the
+ * one-kernel steps that an untuned small map takes by default (hg_set_sweep). */
 int hg_set_tiles(hg_ctx* ctx, int hydro_variant, int thermal_variant);
 int hg_get_tiles(const hg_ctx* ctx, int* hydro_variant, int* thermal_variant);
 /* Tile order of the fused kernels' workgroups, which the hardware deals to
@@ -476,8 +479,8 @@ int hg_set_xcd_order(hg_ctx* ctx, int mode);
  * halo of 5 cells, and are for small maps, whose steps are bound by their
  * launches.  -1 (the default, kept by hg_autotune unless a one-kernel variant
  * times faster) runs the hydro kernel and then the thermal kernel; until this
- * call or hg_autotune, a map of up to 648 x 648 cells runs a tile variant
- * instead while launches are not timed.  All give the per-pass result bit for
+ * call, hg_set_tiles or hg_autotune, a map of up to 648 x 648 cells runs a tile
+ * variant instead while launches are not timed.  All give the per-pass result bit for
  * bit; steps with HG_STEP_KEEP_VELOCITY always use the two kernels. */
 int hg_set_sweep(hg_ctx* ctx, int variant);
 int hg_get_sweep(const hg_ctx* ctx, int* variant);
