@@ -120,12 +120,13 @@ hipError_t launch_fused_thermal(int variant, const ThermIO& io, int nx, int ny, 
                                 bool smooth, int xcd, const KParams& k, hipStream_t s);
 
 // the whole step in one kernel (hg_sweep.hip): strips of columns swept row
-// by row; rain / thermal / smoothing as the step's flags say
+// by row; rain / thermal / smoothing as the step's flags say.  xcd_mode: the tile
+// order (tile_order) of the variants that work tile by tile
 int sweep_variant_count();
 int step_tile_first();      // the first of its variants that is a k_step_tile
 bool sweep_variant_info(int v, int* strip_w, int* rows, int* threads, int* seg_rows);
 hipError_t launch_step_sweep(int variant, const HydroIO& io, int n, uint32_t step, uint32_t terrain, bool rain,
-                             bool thermal, bool smooth, const KParams& k, hipStream_t s);
+                             bool thermal, bool smooth, int xcd_mode, const KParams& k, hipStream_t s);
 
 // the whole step on one tile per workgroup, for small maps (hg_fused.hip): io's
 // ro and dout are the tape's rock and dirt after erosion, written with the rest

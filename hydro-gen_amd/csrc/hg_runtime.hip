@@ -199,8 +199,8 @@ int fused_step(hg_ctx* c, bool rain, bool thermal, bool smooth, bool keep_veloci
     if (one_kernel >= 0 && !keep_velocity) {
         // the whole step in one kernel; rock and dirt come out of its last pass
         const int rc = timed_launch(c, "step_sweep", [&] {
-            return hgk::launch_step_sweep(one_kernel, io, c->n, step, 0u, rain, thermal, smooth, c->kp,
-                                          c->stream);
+            return hgk::launch_step_sweep(one_kernel, io, c->n, step, 0u, rain, thermal, smooth,
+                                          c->xcd_order, c->kp, c->stream);
         });
         if (rc != HG_OK) return rc;
         swap_planes(c, {HG_P_ROCK, HG_P_DIRT, HG_P_WATER, HG_P_FLUX_L, HG_P_FLUX_R, HG_P_FLUX_T, HG_P_FLUX_B,

@@ -723,14 +723,15 @@ bool sweep_variant_info(int v, int* strip_w, int* rows, int* threads, int* seg_r
 }
 
 hipError_t launch_step_sweep(int variant, const HydroIO& io, int n, uint32_t step, uint32_t terrain, bool rain,
-                             bool thermal, bool smooth, const KParams& k, hipStream_t s) {
+                             bool thermal, bool smooth, int xcd_mode, const KParams& k, hipStream_t s) {
     if (variant >= step_tile_first()) {
         HydroIO h = io;
         ThermIO t{};
         t.ro = io.ro;
         t.dout = io.dout;
         h.ro = h.dout = nullptr;
-        return launch_step_tile(variant - step_tile_first(), h, t, n, n, step, terrain, rain, thermal, smooth, 2, k, s);
+        return launch_step_tile(variant - step_tile_first(), h, t, n, n, step, terrain, rain, thermal, smooth, xcd_mode,
+                                k, s);
     }
     SweepArgs a;
     a.io = io; a.n = n;

@@ -33,3 +33,20 @@ def test_tiles_that_are_set_are_run_on_a_small_map(so, tiles, one_kernel):
         """)
     want = "True False False" if one_kernel else "False True True"
     assert out.split("\n")[:-1] == [want] * 4
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_tile_order_that_is_set_is_the_small_maps_too(so, mode):
+    """512^2: 16 tile columns, so each order is taken as it is."""
+    out = fakehip.run(so, f"""
+        fake.fake_watch(b"k_step_tile", 9)               # its order
+        with hg.Terrain(512) as t:
+            t.set_xcd_order({mode})
+            fake.fake_clear()
+            t.dispatch_grid(1)
+            print(fake.fake_watched())
+            fake.fake_clear()
+            t.adjoint_rollout(2, 2, np.zeros((512, 512), np.float32))
+            print(fake.fake_watched())
+        """)
+    assert out.split() == [str(mode)] * 2
