@@ -19,6 +19,7 @@
 #include <numeric>
 
 #include "hg_kernels.hpp"
+#include "hg_stencil.hpp"
 
 namespace hgk {
 
@@ -82,7 +83,12 @@ template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float other_layer(float v) { return dpp<0xb1>(v); }   // quad_perm 1, 0, 3, 2
+struct GroupLanes {
+    static __device__ __forceinline__ float other_layer(float v) { return dpp<0xb1>(v); }   // quad_perm 1, 0, 3, 2
+    template <int L>
+    static __device__ __forceinline__ float lane(float v) { return dpp<0x150 + L>(v); }     // row_newbcast:L
+};
+__device__ __forceinline__ float other_layer(float v) { return GroupLanes::other_layer(v); }
 
 // The heights.  Planes: rock in a, dirt in b, row by row.  PAIRED: rows of
 // (rock, dirt) pairs, those below `half` in a and the others in b, so that two
@@ -105,20 +111,12 @@ struct HeightMap {
 
 // Heights (rock + dirt) at the corners (0,0), (1,0), (0,1), (1,1) of cell (x,
 // y): lane g of the group loads layer g & 1 of corner (g >> 1) & 1 of row
-// (g >> 2) & 1, adds the other layer's value from the lane beside it, and every
-// lane takes the four sums, two from its own quad, two from the next.
+// (g >> 2) & 1, and every lane takes the four sums of lanes 0-7's loads.
 template <class Map>
 __device__ __forceinline__ void stencil_heights(const Map& m, int x, int y, int g, float& h00, float& h10, float& h01,
                                                 float& h11) {
-    const bool top = (g & 4) != 0;
-    const float v = ld(m.at(g & 1, x + ((g >> 1) & 1), y + (top ? 1 : 0)));
-    const float h = v + other_layer(v);
-    const float h0 = dpp<0x00>(h), h1 = dpp<0xaa>(h);            // quad_perm broadcasts of lanes 0 and 2
-    const float o0 = dpp<0x124>(h0), o1 = dpp<0x124>(h1);        // row_ror:4
-    h00 = top ? o0 : h0;
-    h10 = top ? o1 : h1;
-    h01 = top ? h0 : o0;
-    h11 = top ? h1 : o1;
+    const float v = ld(m.at(g & 1, x + ((g >> 1) & 1), y + ((g >> 2) & 1)));
+    corner_heights<GroupLanes>(v, h00, h10, h01, h11);
 }
 
 // Bilinear deposit of `amount` into dirt around (px, py): the four dirt lanes
