@@ -135,7 +135,10 @@ private:
             if (!ev_[i]) {
                 hipEvent_t v = nullptr;
                 const hipError_t e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
-                if (e != hipSuccess) return e;
+                if (e != hipSuccess) {
+                    (void)hipGetLastError();
+                    return e;
+                }
                 ev_[i] = v;
             }
         }
