@@ -73,6 +73,7 @@ public:
             if (c + kSlots < chunks) e = enqueue(c + kSlots);
         }
         if (begun) end();
+        if (e != hipSuccess) (void)hipStreamSynchronize(s);   // no copy may write the slots after this
         return e;
     }
 
