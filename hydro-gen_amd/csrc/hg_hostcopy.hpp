@@ -156,8 +156,7 @@ private:
         over_.store(false, std::memory_order_relaxed);
         for (auto& d : done_) d.store(0, std::memory_order_relaxed);
         if (bytes < kCrewMin) return;
-        if (!crew_tried_) {
-            crew_tried_ = true;
+        if (!counted_) {                                      // at each copy: another object may have gone
             counted_ = crews().fetch_add(1) < kCrews;
             if (!counted_) crews().fetch_sub(1);
             try {
@@ -239,7 +238,7 @@ private:
     std::atomic<int> inside_{0};
     // the helpers
     std::thread helper_[kHelpers];
-    bool crew_tried_ = false, counted_ = false;
+    bool counted_ = false;
     std::mutex mu_;
     std::condition_variable cv_;
     bool stop_ = false, active_ = false;

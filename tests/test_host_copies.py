@@ -47,3 +47,28 @@ def test_failed_read_leaves_no_copy_under_way(so, failing, nth):
             print(np.array_equal(t.read_plane(hg.P_DIRT), b), np.array_equal(t.read_plane(hg.P_ROCK), a))
         """)
     assert out.split() == ["failed", "True", "True"]
+
+
+def test_helpers_go_to_who_copies_next(so):
+    """32 objects have helper threads at a time; one that came too late gets its
+    own at its next copy once another has gone."""
+    out = fakehip.run(so, """
+        n = 512
+        a = np.random.default_rng(0).random((n, n), dtype=np.float32)
+        def threads():                                   # ended ones leave the list a moment after they are joined
+            time.sleep(0.2)
+            return len(os.listdir("/proc/self/task"))
+        alone = threads()
+        ts = [hg.Terrain(n) for _ in range(33)]
+        for t in ts:
+            t.write_plane(hg.P_ROCK, a)
+        print(threads() - alone)
+        ts.pop(0).close()
+        print(threads() - alone)
+        ts[-1].write_plane(hg.P_ROCK, a)
+        print(threads() - alone, np.array_equal(ts[-1].read_plane(hg.P_ROCK), a))
+        for t in ts:
+            t.close()
+        print(threads() - alone)
+        """)
+    assert out.split() == ["96", "93", "96", "True", "0"]
