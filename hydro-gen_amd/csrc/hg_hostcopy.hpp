@@ -106,6 +106,9 @@ private:
     static constexpr size_t kPiecesPerSlot = kSlot / kPiece;
     static constexpr size_t kCrewMin = size_t(1) << 20;       // smaller copies are over before a helper wakes
     static constexpr int kHelpers = 3;
+    // a helper without work yields this often (some 0.1 ms, a few slots' time on
+    // the link) and then sleeps: a copy may be queued behind seconds of GPU work
+    static constexpr int kIdleYields = 256;
     static constexpr int kCrews = 32;                         // more copying at once than a host has links or cores for
 
     static std::atomic<int>& crews() {
@@ -177,7 +180,8 @@ private:
     void copy_chunk(size_t c) {
         const size_t first = c * kPiecesPerSlot;
         const size_t last = first + pieces_of(chunk_bytes(bytes_, c));
-        limit_.store(last, std::memory_order_release);
+        limit_.store(last);
+        wake();
         while (copy_piece()) {
         }
         std::atomic<size_t>& d = done_[c % kSlots];
@@ -207,8 +211,18 @@ private:
             std::lock_guard<std::mutex> lk(mu_);
             active_ = false;                                  // no helper joins any more
         }
-        over_.store(true, std::memory_order_release);
+        over_.store(true);
+        wake();
         while (inside_.load(std::memory_order_acquire) != 0) std::this_thread::yield();
+    }
+
+    // Wakes the helpers that went to sleep within a copy.  (What they look at is
+    // stored before parked_ is read here, and they raise parked_ before they look:
+    // one of the two sees the other.)
+    void wake() {
+        if (parked_.load() == 0) return;
+        { std::lock_guard<std::mutex> lk(mu_); }
+        cv_.notify_all();
     }
 
     void help() {
@@ -220,8 +234,20 @@ private:
             seen = job_;
             inside_.fetch_add(1, std::memory_order_relaxed);
             lk.unlock();
-            while (!over_.load(std::memory_order_acquire))
-                if (!copy_piece()) std::this_thread::yield();
+            for (int idle = 0; !over_.load(std::memory_order_acquire);) {
+                if (copy_piece()) {
+                    idle = 0;
+                } else if (++idle < kIdleYields) {
+                    std::this_thread::yield();
+                } else {
+                    idle = 0;
+                    lk.lock();
+                    parked_.fetch_add(1);
+                    cv_.wait(lk, [&] { return over_.load() || next_.load() < limit_.load(); });
+                    parked_.fetch_sub(1);
+                    lk.unlock();
+                }
+            }
             inside_.fetch_sub(1, std::memory_order_release);
             lk.lock();
         }
@@ -235,7 +261,7 @@ private:
     size_t bytes_ = 0;
     std::atomic<size_t> next_{0}, limit_{0}, done_[kSlots] = {};
     std::atomic<bool> over_{true};
-    std::atomic<int> inside_{0};
+    std::atomic<int> inside_{0}, parked_{0};
     // the helpers
     std::thread helper_[kHelpers];
     bool counted_ = false;

@@ -72,3 +72,20 @@ def test_helpers_go_to_who_copies_next(so):
         print(threads() - alone)
         """)
     assert out.split() == ["96", "93", "96", "True", "0"]
+
+
+@pytest.mark.parametrize("call", ["write", "read"])
+def test_helpers_sleep_while_the_gpu_is_busy(so, call):
+    """A copy behind work on the stream waits for it: the helpers' processors are
+    others' meanwhile."""
+    out = fakehip.run(so, f"""
+        n, wait = 2048, 0.1
+        a = np.random.default_rng(0).random((n, n), dtype=np.float32)
+        with hg.Terrain(n) as t:
+            t.write_plane(hg.P_ROCK, a)
+            fake.fake_event_delay(int(wait * 1e6))           # 4 of the 8 slots' writes wait, all reads
+            cpu = time.process_time()
+            t.write_plane(hg.P_DIRT, a) if "{call}" == "write" else t.read_plane(hg.P_ROCK)
+            print(time.process_time() - cpu < 4 * wait * 0.5)
+        """)
+    assert out.split() == ["True"]
