@@ -92,7 +92,8 @@ void fake_clear() { launches.clear(); direct_copies = 0; watch_value = -1; }
 // remembers the int argument `index` of the last launch of a kernel whose name holds `name`
 void fake_watch(const char* name, int index) { watch_name = name; watch_index = index; }
 int fake_watched() { return watch_value; }
-// copies whose host side was memory that hipHostMalloc gave to the caller
+// copies to or from the caller's own pinned or device memory (not of 2 MB, the
+// size of the library's slots)
 long fake_direct_copies() { return direct_copies; }
 int fake_last_error() { return last_error; }
 
@@ -184,7 +185,7 @@ int hipMemcpyAsync(void* dst, const void* src, size_t bytes, int kind, void* s) 
     const void* host = kind == kHostToDevice ? src : kind == kDeviceToHost ? dst : nullptr;
     of(s)->queue.push_back({dst, src, bytes});
     if (host && !find(pinned, host)) of(s)->run(size_t(-1));   // pageable memory: the call waits
-    const size_t* size = host ? find(pinned, host) : nullptr;
+    const size_t* size = !host ? nullptr : find(pinned, host) ? find(pinned, host) : find(device, host);
     if (size && *size != (size_t(2) << 20)) ++direct_copies;   // not one of the library's 2 MB slots
     return kOk;
 }

@@ -89,3 +89,40 @@ def test_helpers_sleep_while_the_gpu_is_busy(so, call):
             print(time.process_time() - cpu < 4 * wait * 0.5)
         """)
     assert out.split() == ["True"]
+
+
+@pytest.mark.parametrize("memory", ["hipHostMalloc", "hipMalloc"])
+def test_memory_the_runtime_knows_is_copied_by_it(so, memory):
+    """A caller's pinned buffer goes over the link without a second copy, and device
+    memory is not touched by the host."""
+    out = fakehip.run(so, f"""
+        n = 1024
+        p, a = ctypes.c_void_p(), np.random.default_rng(0).random((n, n), dtype=np.float32)
+        fake.{memory}(ctypes.byref(p), ctypes.c_size_t(a.nbytes), 0)
+        f = ctypes.cast(p, ctypes.POINTER(ctypes.c_float))
+        lib, size = hg.load(), ctypes.c_size_t(n * n)
+        with hg.Terrain(n) as t, hg.Batch([n]) as b:
+            ctypes.memmove(p, a.ctypes.data, a.nbytes)
+            assert lib.hg_write_plane(t.h, hg.P_ROCK, f, size) == 0
+            assert lib.hg_batch_write_plane(b.h, 0, hg.P_ROCK, f, size) == 0
+            print(fake.fake_direct_copies(), np.array_equal(t.read_plane(hg.P_ROCK), a),
+                  np.array_equal(b.read_plane(0, hg.P_ROCK), a))
+            for read in (lambda: lib.hg_read_plane(t.h, hg.P_ROCK, f, size),
+                         lambda: lib.hg_batch_read_plane(b.h, 0, hg.P_ROCK, f, size)):
+                ctypes.memset(p, 0, a.nbytes)
+                assert read() == 0
+                print(fake.fake_direct_copies(), ctypes.string_at(p, a.nbytes) == a.tobytes())
+        """)
+    assert out.split() == ["2", "True", "True", "3", "True", "4", "True"]
+
+
+def test_unknown_pointer_leaves_no_error_behind(so):
+    out = fakehip.run(so, """
+        a = np.random.default_rng(0).random((1024, 1024), dtype=np.float32)
+        with hg.Terrain(1024) as t:
+            fake.fake_fail(b"hipPointerGetAttributes", 1, 1)
+            t.write_plane(hg.P_ROCK, a)
+            fake.fake_fail(b"hipPointerGetAttributes", 1, 1)
+            print(np.array_equal(t.read_plane(hg.P_ROCK), a), fake.fake_last_error())
+        """)
+    assert out.split() == ["True", "0"]
