@@ -5,11 +5,12 @@
 // from or to it at 28 GB/s, and the runtime's own path for pageable memory ran
 // at 5 to 36 GB/s.  So a copy goes through a ring of pinned slots: while the
 // link fills or drains some slots, this thread and a few helpers copy the
-// pieces of the others.  Measured, us, against one copy of up to 16 MB and then
-// one memcpy (reads) or the runtime's path (writes, a batch's reads): 16 MB to
-// the host 850 -> 440 (a batch's plane 2380 -> 440), 4 MB 233 -> 130; 16 MB to
-// the device 748 -> 460.  Slots of 1 MB (560 us for 16 MB) leave the link idle
-// between copies, of 4 MB (145 us for 4 MB) the helpers; 7 helpers or 8 slots
+// pieces of the others.  Slots are drained by a kernel (launch_copy_out, where the
+// reason is) and filled by the runtime's copies.  Measured, us, against one copy of
+// up to 16 MB and then one memcpy (reads) or the runtime's path (writes, a batch's
+// reads): 64 MB to the host 2600 -> 1520, 16 MB 850 -> 398 (a batch's plane 950),
+// 4 MB 232 -> 122; 64 MB to the device 2300 -> 1670.  Slots of 1 MB leave the link
+// idle between copies, of 4 MB the helpers (160 us for 4 MB); 7 helpers or 8 slots
 // gain nothing over 3 and 4.
 //
 // A HostCopy belongs to one context or batch and is used by its one host
@@ -26,6 +27,8 @@
 #include <cstring>
 #include <mutex>
 #include <thread>
+
+#include "hg_kernels.hpp"
 
 class HostCopy {
 public:
@@ -52,14 +55,13 @@ public:
     hipError_t to_host(const void* src, void* dst, size_t bytes, hipStream_t s) {
         if (bytes == 0) return hipSuccess;
         hipError_t e = hipSuccess;
-        if (known(dst) || (e = reserve(bytes)) != hipSuccess)
+        if (known(dst) || bytes % 16 || (e = reserve(bytes)) != hipSuccess)
             return direct(dst, src, bytes, hipMemcpyDeviceToHost, s);
         const char* from = static_cast<const char*>(src);
         const size_t chunks = (bytes + kSlot - 1) / kSlot;
         auto enqueue = [&](size_t c) {
             const size_t off = c * kSlot;
-            const hipError_t r = hipMemcpyAsync(pin_[c % kSlots], from + off, chunk_bytes(bytes, c),
-                                                hipMemcpyDeviceToHost, s);
+            const hipError_t r = hgk::launch_copy_out(pin_[c % kSlots], from + off, chunk_bytes(bytes, c), s);
             return r != hipSuccess ? r : hipEventRecord(ev_[c % kSlots], s);
         };
         for (size_t c = 0; c < chunks && c < kSlots && e == hipSuccess; ++c) e = enqueue(c);
@@ -143,7 +145,7 @@ private:
         for (size_t i = 0; i < kSlots && i * kSlot < bytes; ++i) {   // each piece stored only once it exists
             if (!pin_[i]) {
                 void* p = nullptr;
-                const hipError_t e = hipHostMalloc(&p, kSlot, hipHostMallocDefault);
+                const hipError_t e = hipHostMalloc(&p, kSlot, hipHostMallocCoherent);
                 if (e != hipSuccess) {
                     (void)hipGetLastError();                  // the caller's other path is not to find it
                     return e;

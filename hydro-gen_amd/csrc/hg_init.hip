@@ -396,6 +396,34 @@ hipError_t launch_deinterleave_rgba(const float* in, float* const planes[4], siz
     return hipGetLastError();
 }
 
+// Device memory to pinned host memory, 16 bytes a lane, for reads.  Bound by the
+// link.  The runtime's copies go by a DMA engine, which at times runs at half its
+// rate and 100 us late (a state that lasts for processes on end, and that only
+// copies to the host show): 2 MB chunks, four under way, 41 GB/s and at such times
+// 11.7, by this kernel 47; 64 KB alone 15.6 us and at such times 130, here 12.5.
+// 32 workgroups: more of them write 50 GB/s to idle memory, but the host is copying
+// the chunk before out of it (16 MB to the caller's memory, us: 16 workgroups 407,
+// 32 396, 64 418, 128 442, 256 502, 512 618; a DMA engine 437).
+__global__ __launch_bounds__(256) void k_copy_out(uint4* __restrict__ dst, const uint4* __restrict__ src,
+                                                  unsigned quads) {
+    for (unsigned i = blockIdx.x * 256u + threadIdx.x; i < quads; i += gridDim.x * 256u) dst[i] = src[i];
+    __threadfence_system();
+}
+
+hipError_t launch_copy_out(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (bytes == 0) return hipSuccess;
+    const size_t quads = bytes / sizeof(uint4);
+    if (bytes % sizeof(uint4) || reinterpret_cast<uintptr_t>(dst) % sizeof(uint4) ||
+        reinterpret_cast<uintptr_t>(src) % sizeof(uint4) || quads > (size_t(1) << 30))
+        return hipErrorInvalidValue;
+    // its own status, like a copy's: an error that the caller's program left
+    // behind is not this copy's
+    unsigned n = unsigned(quads);
+    void* args[] = {&dst, &src, &n};
+    return hipLaunchKernel(reinterpret_cast<const void*>(k_copy_out), dim3(std::min((n + 255) / 256, 32u)), dim3(256),
+                           args, 0, s);
+}
+
 hipError_t launch_fill(float* p, size_t n, float value, hipStream_t s) {
     if (n == 0) return hipSuccess;
     k_fill<<<unsigned((n + 255) / 256), 256, 0, s>>>(p, n, value);

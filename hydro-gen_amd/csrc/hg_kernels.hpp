@@ -230,6 +230,9 @@ hipError_t launch_minmax(const float* v, size_t n, unsigned* mm_dev, hipStream_t
 hipError_t launch_rescale(float* v, size_t n, const unsigned* mm_dev, float lo, float hi,
                           hipStream_t s);
 hipError_t launch_fill(float* p, size_t n, float value, hipStream_t s);
+// `bytes` (a multiple of 16, at most 16 GB) from device memory to pinned host
+// memory, both 16-byte aligned
+hipError_t launch_copy_out(void* dst, const void* src, size_t bytes, hipStream_t s);
 // out (4n floats, 16-byte aligned) = RGBA texels of the 4 planes (null: 0);
 // `total`: the fourth component is (p0 + p1) + p2
 hipError_t launch_interleave_rgba(float* out, const float* const planes[4], size_t n, bool total, hipStream_t s);

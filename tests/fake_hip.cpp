@@ -96,6 +96,7 @@ int fake_watched() { return watch_value; }
 // size of the library's slots)
 long fake_direct_copies() { return direct_copies; }
 int fake_last_error() { return last_error; }
+void fake_set_last_error(int e) { last_error = e; }
 
 // ---- kernels
 void** __hipRegisterFatBinary(const void*) { static void* module; return &module; }
@@ -112,10 +113,14 @@ int __hipPopCallConfiguration(Dim* g, Dim* b, size_t* shared, void** s) {
     *g = config.grid; *b = config.block; *shared = config.shared; *s = config.stream;
     return kOk;
 }
-int hipLaunchKernel(const void* f, Dim, Dim, void** args, size_t, void*) {
+int hipLaunchKernel(const void* f, Dim, Dim, void** args, size_t, void* s) {
     std::lock_guard<std::recursive_mutex> lk(mu);
+    if (const int e = injected("hipLaunchKernel")) return e;
     const std::string& name = kernels[f];
     launches += name + "\n";
+    if (name.find("k_copy_out") != std::string::npos)          // (to, from, 16-byte units): the one that is run
+        of(s)->queue.push_back({*static_cast<void**>(args[0]), *static_cast<const void**>(args[1]),
+                                *static_cast<const unsigned*>(args[2]) * size_t(16)});
     if (!watch_name.empty() && name.find(watch_name) != std::string::npos)
         watch_value = *static_cast<const int*>(args[watch_index]);
     return kOk;

@@ -27,7 +27,7 @@ def test_refused_event_leaves_no_error_behind(so):
     assert out.split() == ["0", "True"]
 
 
-@pytest.mark.parametrize("failing", ["hipEventSynchronize", "hipMemcpyAsync"])
+@pytest.mark.parametrize("failing", ["hipEventSynchronize", "hipLaunchKernel"])
 @pytest.mark.parametrize("nth", [1, 2, 5])
 def test_failed_read_leaves_no_copy_under_way(so, failing, nth):
     """After a read that failed midway, its copies no longer write the slots: what
@@ -126,3 +126,19 @@ def test_unknown_pointer_leaves_no_error_behind(so):
             print(np.array_equal(t.read_plane(hg.P_ROCK), a), fake.fake_last_error())
         """)
     assert out.split() == ["True", "0"]
+
+
+def test_reads_are_not_left_to_a_copy_engine(so):
+    """The slots of a read are filled by the library's kernel: an engine may be in
+    a state in which it takes 100 us more per copy, at half the rate.  An error
+    that the caller's program left behind does not fail it."""
+    out = fakehip.run(so, """
+        a = np.random.default_rng(0).random((1456, 1456), dtype=np.float32)
+        with hg.Terrain(1456) as t:
+            t.write_plane(hg.P_ROCK, a)
+            fake.fake_clear()
+            fake.fake_fail(b"hipMemcpyAsync", 1, 2)
+            fake.fake_set_last_error(1)
+            print(np.array_equal(t.read_plane(hg.P_ROCK), a), len(launched()), fake.fake_last_error())
+        """)
+    assert out.split() == ["True", "5", "1"]
