@@ -85,8 +85,9 @@ public:
     // returns when the device holds them.
     hipError_t to_device(const void* src, void* dst, size_t bytes, hipStream_t s) {
         hipError_t e = hipSuccess;
-        // below kCrewMin the runtime's own path is the shorter one
-        if (bytes < kCrewMin || known(src) || (e = reserve(bytes)) != hipSuccess)
+        const bool first = !wrote_ && !pin_[0];
+        wrote_ = true;
+        if (bytes < kRingWrite || first || known(src) || (e = reserve(bytes)) != hipSuccess)
             return direct(dst, src, bytes, hipMemcpyHostToDevice, s);
         const size_t chunks = (bytes + kSlot - 1) / kSlot;
         begin(nullptr, static_cast<const char*>(src), bytes);
@@ -110,6 +111,16 @@ private:
     static constexpr size_t kPiecesPerSlot = kSlot / kPiece;
     static constexpr size_t kCrewMin = size_t(1) << 20;       // smaller copies are over before a helper wakes
     static constexpr int kHelpers = 3;
+    // Smaller writes, and the first of a new object, take the runtime's own path:
+    // the ring gains nothing on the former, and its slots and helpers cost the
+    // latter more than one write gains.  us by the runtime / by the ring, for a
+    // plane of one of three states of 9 planes written in turn, of a state that is
+    // new, for a single plane of new data, and for the first write of a new object:
+    //    1 MB    66/53      56/57      53/61      57/123
+    //    2 MB   111/101    109/107     91/110     94/191
+    //    4 MB   176/140    187/157    135/153    139/234
+    //   16 MB   590/455    643/475    483/505    506/647
+    static constexpr size_t kRingWrite = size_t(4) << 20;
     // a helper without work yields this often (some 0.1 ms, a few slots' time on
     // the link) and then sleeps: a copy may be queued behind seconds of GPU work
     static constexpr int kIdleYields = 256;
@@ -269,6 +280,7 @@ private:
         }
     }
 
+    bool wrote_ = false;
     char* pin_[kSlots] = {};
     hipEvent_t ev_[kSlots] = {};
     // the copy in progress

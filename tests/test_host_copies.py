@@ -33,7 +33,7 @@ def test_failed_read_leaves_no_copy_under_way(so, failing, nth):
     """After a read that failed midway, its copies no longer write the slots: what
     is written next arrives whole."""
     out = fakehip.run(so, f"""
-        n = 2048
+        n = 2904                                         # written through the slots too
         a, b = (np.random.default_rng(i).random((n, n), dtype=np.float32) for i in range(2))
         with hg.Terrain(n) as t:
             t.write_plane(hg.P_ROCK, a)
@@ -62,10 +62,11 @@ def test_helpers_go_to_who_copies_next(so):
         ts = [hg.Terrain(n) for _ in range(33)]
         for t in ts:
             t.write_plane(hg.P_ROCK, a)
+            t.read_plane(hg.P_ROCK)
         print(threads() - alone)
         ts.pop(0).close()
         print(threads() - alone)
-        ts[-1].write_plane(hg.P_ROCK, a)
+        ts[-1].read_plane(hg.P_ROCK)
         print(threads() - alone, np.array_equal(ts[-1].read_plane(hg.P_ROCK), a))
         for t in ts:
             t.close()
@@ -79,14 +80,14 @@ def test_helpers_sleep_while_the_gpu_is_busy(so, call):
     """A copy behind work on the stream waits for it: the helpers' processors are
     others' meanwhile."""
     out = fakehip.run(so, f"""
-        n, wait = 2048, 0.1
+        n, wait = 2904, 0.05
         a = np.random.default_rng(0).random((n, n), dtype=np.float32)
         with hg.Terrain(n) as t:
             t.write_plane(hg.P_ROCK, a)
-            fake.fake_event_delay(int(wait * 1e6))           # 4 of the 8 slots' writes wait, all reads
+            fake.fake_event_delay(int(wait * 1e6))           # 13 of the 17 slots' writes wait, all reads
             cpu = time.process_time()
             t.write_plane(hg.P_DIRT, a) if "{call}" == "write" else t.read_plane(hg.P_ROCK)
-            print(time.process_time() - cpu < 4 * wait * 0.5)
+            print(time.process_time() - cpu < 13 * wait * 0.5)
         """)
     assert out.split() == ["True"]
 
@@ -142,3 +143,19 @@ def test_reads_are_not_left_to_a_copy_engine(so):
             print(np.array_equal(t.read_plane(hg.P_ROCK), a), len(launched()), fake.fake_last_error())
         """)
     assert out.split() == ["True", "5", "1"]
+
+
+@pytest.mark.parametrize("write", ["t.write_plane(hg.P_ROCK, a)", "t.write(hg.CH_HEIGHT, q)",
+                                   "b.write_plane(0, hg.P_ROCK, a)"])
+def test_first_write_of_a_new_object_needs_no_ring(so, write):
+    """It would pay for pinned slots and threads, and gain less than they cost."""
+    out = fakehip.run(so, f"""
+        n = 1024
+        a, q = (np.random.default_rng(i).random(s, dtype=np.float32) for i, s in enumerate([(n, n), (n, n, 4)]))
+        threads = len(os.listdir("/proc/self/task"))
+        with hg.Terrain(n) as t, hg.Batch([n]) as b:
+            for _ in range(2):
+                {write}
+                print(len(os.listdir("/proc/self/task")) - threads)
+        """)
+    assert out.split() == ["0", "3"]
