@@ -82,13 +82,15 @@ public:
     }
 
     // `bytes` from `src` to device `dst`, in order with the work on `s`;
-    // returns when the device holds them.
-    hipError_t to_device(const void* src, void* dst, size_t bytes, hipStream_t s) {
+    // returns when the device holds them or, without `wait`, when they are on their
+    // way: the caller then waits for the stream before it gives src back or copies
+    // again.
+    hipError_t to_device(const void* src, void* dst, size_t bytes, hipStream_t s, bool wait = true) {
         hipError_t e = hipSuccess;
         const bool first = !wrote_ && !pin_[0];
         wrote_ = true;
         if (bytes < kRingWrite || first || known(src) || (e = reserve(bytes)) != hipSuccess)
-            return direct(dst, src, bytes, hipMemcpyHostToDevice, s);
+            return direct(dst, src, bytes, hipMemcpyHostToDevice, s, wait);
         const size_t chunks = (bytes + kSlot - 1) / kSlot;
         begin(nullptr, static_cast<const char*>(src), bytes);
         for (size_t c = 0; c < chunks && e == hipSuccess; ++c) {
@@ -100,6 +102,7 @@ public:
             if (e == hipSuccess) e = hipEventRecord(ev_[c % kSlots], s);
         }
         end();
+        if (!wait) return e;
         const hipError_t w = hipStreamSynchronize(s);         // the slots are free again, whatever happened
         return e != hipSuccess ? e : w;
     }
@@ -147,9 +150,10 @@ private:
     }
 
     // The runtime's own path; also when no more can be pinned.
-    static hipError_t direct(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+    static hipError_t direct(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s,
+                             bool wait = true) {
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, s);
-        return e != hipSuccess ? e : hipStreamSynchronize(s);
+        return e != hipSuccess || !wait ? e : hipStreamSynchronize(s);
     }
 
     hipError_t reserve(size_t bytes) {

@@ -891,13 +891,14 @@ int hg_write(hg_ctx* c, int channel, const float* rgba, size_t n_floats) {
         HG_HIP(c, hipMalloc(&p, 4 * pn * sizeof(float)));
         c->rgba_dev = static_cast<float*>(p);
     }
-    const int rc = write_floats(c, rgba, c->rgba_dev, 4 * pn);
-    if (rc != HG_OK) return rc;
     float* dst[4];
     for (int k = 0; k < 4; ++k) dst[k] = planes[k] < 0 ? nullptr : c->cur[planes[k]];
-    HG_HIP(c, hgk::launch_deinterleave_rgba(c->rgba_dev, dst, pn, c->stream));
-    HG_HIP(c, hipStreamSynchronize(c->stream));
-    return HG_OK;
+    // one wait for both, whatever happened: the caller's memory is in use until then
+    hipError_t e = c->copy.to_device(rgba, c->rgba_dev, 4 * pn * sizeof(float), c->stream, false);
+    if (e == hipSuccess) e = hgk::launch_deinterleave_rgba(c->rgba_dev, dst, pn, c->stream);
+    const hipError_t w = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = w;
+    return e == hipSuccess ? HG_OK : hgctx::hip_fail(c, e, "hg_write: texels to the device");
 }
 
 int hg_plane_device_ptr(hg_ctx* c, int plane, void** ptr) {

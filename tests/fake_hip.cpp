@@ -44,7 +44,7 @@ std::map<const void*, std::string> kernels;
 std::map<std::string, std::pair<int, int>> failing;          // function -> calls until it fails, its code
 std::string launches, watch_name;
 int watch_index = 0, watch_value = -1, last_error = kOk;
-long direct_copies = 0;
+long direct_copies = 0, syncs = 0;
 unsigned event_delay_us = 0;
 
 const size_t* find(const std::map<char*, size_t>& m, const void* p) {
@@ -88,13 +88,15 @@ extern "C" {
 void fake_fail(const char* fn, int nth, int code) { failing[fn] = {nth, code}; }
 void fake_event_delay(unsigned us) { event_delay_us = us; }
 const char* fake_launches() { return launches.c_str(); }
-void fake_clear() { launches.clear(); direct_copies = 0; watch_value = -1; }
+void fake_clear() { launches.clear(); direct_copies = syncs = 0; watch_value = -1; }
 // remembers the int argument `index` of the last launch of a kernel whose name holds `name`
 void fake_watch(const char* name, int index) { watch_name = name; watch_index = index; }
 int fake_watched() { return watch_value; }
 // copies to or from the caller's own pinned or device memory (not of 2 MB, the
 // size of the library's slots)
 long fake_direct_copies() { return direct_copies; }
+// waits for a stream
+long fake_syncs() { return syncs; }
 int fake_last_error() { return last_error; }
 void fake_set_last_error(int e) { last_error = e; }
 
@@ -153,6 +155,7 @@ int hipStreamCreateWithFlags(void** s, unsigned) { *s = new Stream; return kOk; 
 int hipStreamDestroy(void* s) { of(s)->run(size_t(-1)); delete of(s); return kOk; }
 int hipStreamSynchronize(void* s) {
     std::lock_guard<std::recursive_mutex> lk(mu);
+    ++syncs;
     if (const int e = injected("hipStreamSynchronize")) return e;
     of(s)->run(size_t(-1));
     return kOk;

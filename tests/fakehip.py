@@ -14,7 +14,7 @@ PREAMBLE = """
 import ctypes, os, sys, time
 fake = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
 fake.fake_launches.restype = ctypes.c_char_p
-fake.fake_direct_copies.restype = ctypes.c_long
+fake.fake_direct_copies.restype = fake.fake_syncs.restype = ctypes.c_long
 sys.path.insert(0, {pkg!r})
 import numpy as np
 import hydrogen as hg

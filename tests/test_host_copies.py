@@ -159,3 +159,26 @@ def test_first_write_of_a_new_object_needs_no_ring(so, write):
                 print(len(os.listdir("/proc/self/task")) - threads)
         """)
     assert out.split() == ["0", "3"]
+
+
+@pytest.mark.parametrize("n", [8, 512, 1024])
+def test_channel_write_waits_once(so, n):
+    """For the copy and the kernel that splits it, also where the kernel fails: the
+    caller's memory must not be in use when the call returns."""
+    out = fakehip.run(so, f"""
+        q = np.random.default_rng(0).random(({n}, {n}, 4), dtype=np.float32)
+        with hg.Terrain({n}) as t:
+            for _ in range(2):
+                t.write(hg.CH_HEIGHT, q)
+                fake.fake_clear()
+            t.write(hg.CH_HEIGHT, q)
+            print(fake.fake_syncs(), launched())
+            fake.fake_fail(b"hipLaunchKernel", 1, 2)
+            fake.fake_set_last_error(2)                      # what the launch leaves
+            try:
+                t.write(hg.CH_HEIGHT, q)
+            except hg.HGError:
+                print(fake.fake_syncs())
+        """).split("\n")
+    assert out[0].startswith("1 [") and "k_deinterleave_rgba" in out[0]
+    assert out[1] == "1"
