@@ -174,9 +174,9 @@ Brush make_brush(int r);
 // order: null, or the droplet id each thread slot runs (a permutation of
 // [0, count), from launch_droplet_order).  The heights are the planes of rock (a)
 // and dirt (b) or, paired, rows of (rock, dirt) pairs, n * n floats in a (rows
-// below n / 2) and in b.  droplets_pair: whether `iterations` of p are worth
-// pairing the planes for.
-bool droplets_pair(int n, const DropletParams& p, uint32_t iterations);
+// below n / 2) and in b.  droplets_pair: whether `iterations` of p with a brush of
+// `radius` are worth pairing the planes for.
+bool droplets_pair(int n, const DropletParams& p, int radius, uint32_t iterations);
 hipError_t launch_pair_heights(const float* rock, const float* dirt, float* low, float* high, int n, hipStream_t s);
 hipError_t launch_unpair_heights(const float* low, const float* high, float* rock, float* dirt, int n, hipStream_t s);
 hipError_t launch_droplets(float* a, float* b, bool paired, int n, const DropletParams& p, const Brush& brush,

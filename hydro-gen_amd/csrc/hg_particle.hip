@@ -179,7 +179,12 @@ constexpr uint32_t kChunk = 64 / kGroup;         // droplets of a wave
 // atomically to *exported_out and *steps_out.  PARTIALS = true: they are
 // written to partials[blockIdx.x], for k_droplet_totals to sum in a fixed
 // order.
-template <bool PARTIALS, bool PAIRED>
+// ROWS: kRows, or 1 for the brush of radius 1, which is one cell: no loop over
+// rows, and what it gave is passed on by a lane instead of through LDS.  us an
+// iteration of 30 steps at 2048^2 on the planes, a thread per droplet / ROWS = 1:
+// 1 droplet 55/52, 64 109/89, 65536 387/358, 2^20 6160/5345 (with kRows the last
+// two take 421 and 6600).
+template <bool PARTIALS, bool PAIRED, int ROWS>
 __global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map, DropletParams p, Brush brush, uint32_t iteration,
                                                            uint32_t rounds, uint32_t spread,
                                                            const uint32_t* __restrict__ order,
@@ -188,7 +193,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map
     __shared__ double s_exp[kDropletsPerBlock];
     __shared__ unsigned s_steps[kDropletsPerBlock];
     __shared__ float s_w[kSlots];        // the brush's weights, its rows padded to whole chunks of kRowCells
-    __shared__ __align__(16) float s_got[kDropletsPerBlock][kGotPitch];   // what a group's brush cells gave
+    __shared__ __align__(16) float s_got[ROWS > 1 ? kDropletsPerBlock : 1][kGotPitch];   // what a group's brush cells gave
     const int g = int(threadIdx.x) & (kGroup - 1), group = int(threadIdx.x) / kGroup;
     const int n = map.n;
     const int reach = brush.r - 1, width = 2 * reach + 1;         // cells closer than r: rows and columns -reach .. reach
@@ -280,16 +285,16 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map
                     }
                 }
                 const float scale = interior ? amount : amount / wsum;
-                for (int base = 0; base < chunks_of_rows; base += kRows) {
+                for (int base = 0; base < (ROWS > 1 ? chunks_of_rows : 1); base += ROWS) {
                     // lane g: layer g & 1 of cell g >> 1 of each row chunk.  The
                     // dirt goes first, the rock gives the rest, both sent
                     // together as if all the dirt seen will be got.
-                    float *at[kRows], want[kRows], seen[kRows], est[kRows], dirt[kRows], old[kRows];
+                    float *at[ROWS], want[ROWS], seen[ROWS], est[ROWS], dirt[ROWS], old[ROWS];
 #pragma unroll
-                    for (int i = 0; i < kRows; ++i) {
+                    for (int i = 0; i < ROWS; ++i) {
                         at[i] = map.a;
                         want[i] = seen[i] = 0.0f;
-                        if (base + i < chunks_of_rows) {
+                        if (ROWS == 1 || base + i < chunks_of_rows) {
                             const int row = (base + i) >> twice, column = ((base + i) & twice) * kRowCells;
                             const int x = cx - reach + column + (g >> 1), y = cy - reach + row;
                             const float w = s_w[(base + i) * kRowCells + (g >> 1)];
@@ -301,18 +306,28 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map
                         }
                     }
 #pragma unroll
-                    for (int i = 0; i < kRows; ++i) {
+                    for (int i = 0; i < ROWS; ++i) {
                         const float beside = other_layer(seen[i]);
                         dirt[i] = estimate((g & 1) ? seen[i] : beside, want[i]);
                         est[i] = (g & 1) ? dirt[i] : estimate(seen[i], want[i] - dirt[i]);
                     }
 #pragma unroll
-                    for (int i = 0; i < kRows; ++i) {
+                    for (int i = 0; i < ROWS; ++i) {
                         // any value where nothing is taken (taken() does not look
                         // at it): a 0 would have to be merged with the atomic's
                         // result, which waits for it before the next is sent
                         old[i] = __builtin_nondeterministic_value(old[i]);
                         if (est[i] > 0.0f) old[i] = fetch_addf(at[i], -est[i]);
+                    }
+                    if constexpr (ROWS == 1) {
+                        float mine = taken(at[0], old[0], est[0]);
+                        const float beside = other_layer(mine);
+                        if (g == 0 && beside < dirt[0]) {    // as below
+                            const float more = estimate(ld(at[0]), dirt[0] - beside);
+                            if (more > 0.0f) mine += taken(at[0], fetch_addf(at[0], -more), more);
+                        }
+                        sed += GroupLanes::lane<0>(beside + mine);
+                        continue;
                     }
                     // sed += dirt + rock, cell by cell in the brush's order
                     // (slots that gave nothing add 0): the group passes its
@@ -320,7 +335,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map
                     // writes a group's row, and a wave's LDS accesses keep their
                     // order.
 #pragma unroll
-                    for (int i = 0; i < kRows; ++i) {
+                    for (int i = 0; i < ROWS; ++i) {
                         const float mine = taken(at[i], old[i], est[i]);
                         const float beside = other_layer(mine);
                         if ((g & 1) == 0) {
@@ -333,7 +348,7 @@ __global__ __launch_bounds__(kDropThreads) void k_droplets(HeightMap<PAIRED> map
                         }
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    const int m = min(kRows, chunks_of_rows - base) * (kRowCells / 4);
+                    const int m = min(ROWS, chunks_of_rows - base) * (kRowCells / 4);
                     for (int q = 0; q < m; ++q) {
                         const float4 v4 = *reinterpret_cast<const float4*>(&s_got[group][4 * q]);
                         sed += v4.x;
@@ -521,12 +536,15 @@ hipError_t launch_droplets(float* a, float* b, bool paired, int n, const Droplet
     if (p.count == 0) return hipSuccess;
     const uint32_t blocks = (p.count + kDropletsPerBlock - 1) / kDropletsPerBlock;
     const uint32_t spread = order ? chunk_spread(p.count) : 1u;
-    if (paired)
-        k_droplets<false, true><<<blocks, kDropThreads, 0, s>>>(HeightMap<true>{a, b, n, n / 2}, p, brush, iteration, 1,
-                                                                spread, order, exported, steps, nullptr);
+    auto launch = [&](auto kernel, auto map) {
+        kernel<<<blocks, kDropThreads, 0, s>>>(map, p, brush, iteration, 1, spread, order, exported, steps, nullptr);
+    };
+    const HeightMap<true> pairs{a, b, n, n / 2};
+    const HeightMap<false> planes{a, b, n, 0};
+    if (brush.r == 1)
+        paired ? launch(k_droplets<false, true, 1>, pairs) : launch(k_droplets<false, false, 1>, planes);
     else
-        k_droplets<false, false><<<blocks, kDropThreads, 0, s>>>(HeightMap<false>{a, b, n, 0}, p, brush, iteration, 1,
-                                                                 spread, order, exported, steps, nullptr);
+        paired ? launch(k_droplets<false, true, kRows>, pairs) : launch(k_droplets<false, false, kRows>, planes);
     return hipGetLastError();
 }
 
@@ -538,8 +556,12 @@ hipError_t launch_droplets(float* a, float* b, bool paired, int n, const Droplet
 //   512^2    123/143     390/482    1988/2479     2429/3082
 //  2048^2    119/131     380/447    1422/1699     1820/2234
 //  8192^2    481/124     733/414    1762/1680     2147/2260
-bool droplets_pair(int n, const DropletParams& p, uint32_t iterations) {
+// A brush of one cell gains nothing on the chain, and by its atomics only where a
+// cell is visited often (30 steps, on the planes / paired: 65536 at 512^2 504/481,
+// 2^20 at 2048^2 5340/5380, 2^20 at 8192^2 5140/5510, 1 at 2048^2 53/72).
+bool droplets_pair(int n, const DropletParams& p, int radius, uint32_t iterations) {
     const double lives = double(p.count > 0 ? p.max_lifetime : 0u) * iterations;
+    if (radius == 1) return 8.0 * n * n <= lives * p.count;
     return double(n) * n < lives * (262144.0 + 12.0 * p.count);
 }
 
@@ -590,8 +612,12 @@ hipError_t launch_droplets_partials(float* rock, float* dirt, int n, const Dropl
                                     uint32_t iteration, DropletPartial* partials, hipStream_t s) {
     if (p.count == 0) return hipSuccess;
     const HeightMap<false> map{rock, dirt, n, 0};
-    k_droplets<true, false><<<droplet_partial_blocks(p.count), kDropThreads, 0, s>>>(
-        map, p, brush, iteration, partial_rounds(p.count), 1u, nullptr, nullptr, nullptr, partials);
+    auto launch = [&](auto kernel) {
+        kernel<<<droplet_partial_blocks(p.count), kDropThreads, 0, s>>>(map, p, brush, iteration,
+                                                                        partial_rounds(p.count), 1u, nullptr, nullptr,
+                                                                        nullptr, partials);
+    };
+    brush.r == 1 ? launch(k_droplets<true, false, 1>) : launch(k_droplets<true, false, kRows>);
     return hipGetLastError();
 }
 

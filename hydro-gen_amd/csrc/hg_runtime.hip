@@ -580,7 +580,7 @@ int hg_step_particle(hg_ctx* c, uint32_t iterations, uint32_t flags) {
     }
     // Where it pays, the droplets run on (rock, dirt) pairs, kept in the alternate
     // buffers of the two planes (every pass that reads those writes them first).
-    const bool pairs = hgk::droplets_pair(c->n, p, thermal || smooth ? 1u : iterations);
+    const bool pairs = hgk::droplets_pair(c->n, p, brush.r, thermal || smooth ? 1u : iterations);
     bool paired = false;
     for (uint32_t it = 0; it < iterations; ++it) {
         const uint32_t iter = c->particle_iter;
