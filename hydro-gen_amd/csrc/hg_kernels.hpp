@@ -184,7 +184,7 @@ hipError_t launch_droplets(float* a, float* b, bool paired, int n, const Droplet
                            unsigned long long* steps, hipStream_t s);
 // Droplet ordering: a counting sort of an iteration's droplets by the tile of
 // their start cell (tiles of droplet_tile_side(n) cells, row-major), so the
-// 64 droplets of a wave start close together and share cache lines.
+// 4 droplets of a wave start close together and share cache lines.
 // tiles: droplet_tile_count(n) words of scratch; order: count words.
 int droplet_tile_side(int n);
 int droplet_tile_count(int n);

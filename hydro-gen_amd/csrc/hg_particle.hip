@@ -597,7 +597,8 @@ hipError_t launch_droplet_order(int n, const DropletParams& p, uint32_t iteratio
 }
 
 // Rounds per workgroup that keep the workgroups of a partials launch within
-// HG_DROPLET_PARTIALS_MAX (1 up to 2^19 droplets, 8 at 2^22).
+// HG_DROPLET_PARTIALS_MAX (1 up to 2^20 droplets, 4 at 2^22).
+static_assert(kDropletsPerBlock * HG_DROPLET_PARTIALS_MAX == 1u << 20, "droplets of one round");
 static uint32_t partial_rounds(uint32_t count) {
     const uint32_t per = uint32_t(kDropletsPerBlock) * HG_DROPLET_PARTIALS_MAX;
     return std::max(1u, (count + per - 1) / per);
