@@ -668,13 +668,14 @@ __global__ __launch_bounds__(NT) void k_step_tile(HydroIO io, ThermIO tio, int n
 // runs its segment again in the ODD form, which takes thermal_term (a test per
 // row instead, and the products or thermal_term after it: 5 % slower).
 //
-// About 260 VALU instructions per cell, times 1.10 for the columns and 1.12
+// About 265 VALU instructions per cell, times 1.10 for the columns and 1.12
 // (at 49 rows) for the rows that are not its own, issued at one per 3.5 cycles
 // per SIMD, near the rate of their mix (2.7 with two operands, 4.2 with three
 // or a lane shift).  142 registers: three waves per SIMD; held to 128 for four
 // it spills and slows down (150).  4096^2: 165 -> 126 us per launch, a step
 // 430 -> 389 us, with three maps at once 402 -> 354; 2048^2 with three maps at
-// once 104 -> 91 us per step.
+// once 104 -> 91 us per step.  (The check for infinities, 6 of the instructions,
+// came later: 4 steps at 4096^2 1375 -> 1378 us.)
 // ---------------------------------------------------------------------------
 constexpr int MARCH_TX = 116;          // columns a wave writes
 constexpr int MARCH_HX = 6;            // halo columns on each side (5 needed, even for the pairs)

@@ -10,8 +10,8 @@
 // up to 16 MB and then one memcpy (reads) or the runtime's path (writes, a batch's
 // reads): 64 MB to the host 2600 -> 1520, 16 MB 850 -> 398 (a batch's plane 950),
 // 4 MB 232 -> 122; 64 MB to the device 2300 -> 1670.  Slots of 1 MB leave the link
-// idle between copies, of 4 MB the helpers (160 us for 4 MB); 7 helpers or 8 slots
-// gain nothing over 3 and 4.
+// idle between copies (16 MB in 431 us), of 4 MB the helpers (4 MB in 148 us); 6
+// helpers or 8 slots gain nothing over 3 and 4.
 //
 // A HostCopy belongs to one context or batch and is used by its one host
 // thread.  The pinned slots (8 MB) and the helper threads are made when first
