@@ -5,8 +5,8 @@
 // from or to it at 28 GB/s, and the runtime's own path for pageable memory ran
 // at 5 to 36 GB/s.  So a copy goes through a ring of pinned slots: while the
 // link fills or drains some slots, this thread and a few helpers copy the
-// pieces of the others.  Slots are drained by a kernel (launch_copy_out, where the
-// reason is) and filled by the runtime's copies.  Measured, us, against one copy of
+// pieces of the others.  A kernel fills the slots of a read (launch_copy_out, where
+// the reason is), the runtime's copies empty those of a write.  Measured, us, against one copy of
 // up to 16 MB and then one memcpy (reads) or the runtime's path (writes, a batch's
 // reads): 64 MB to the host 2600 -> 1520, 16 MB 850 -> 398 (a batch's plane 950),
 // 4 MB 232 -> 122; 64 MB to the device 2300 -> 1670.  Slots of 1 MB leave the link
